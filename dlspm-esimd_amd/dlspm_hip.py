@@ -10,6 +10,7 @@ import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libdlspm_hip.so")
+CALLS_PATH = os.path.join(_HERE, "_dlspm_torch.so")
 GEN_LIB_PATH = os.path.join(_HERE, "libdlspm_gen.so")
 
 OK = 0
@@ -349,6 +350,30 @@ def prepare(row_offsets, col_indices, K, op, width, info=None) -> Prepared:
     return Prepared(mem, (mem.numel() * 4 if mem is not None else 0) | cp.hints, cp)
 
 
+def _raise(status, where):
+    raise DlspmError(status, where)
+
+
+def __getattr__(name):
+    """spmm, sddmm and fused: native functions (host/torch_calls.cpp) that are loaded, and torch with them, where one of
+    them is first used. They handle the usual call by themselves and hand every other one to _spmm, _sddmm and _fused."""
+    if name not in ("spmm", "sddmm", "fused"):
+        raise AttributeError(f"module {__name__!r} has no attribute {name!r}")
+    import importlib.util
+
+    import torch  # noqa: F401  (its libraries must be there before the module that uses them)
+
+    lib()
+    if not os.path.exists(CALLS_PATH):
+        raise FileNotFoundError(f"{CALLS_PATH} is missing: build it with `make -C {_HERE} calls`")
+    spec = importlib.util.spec_from_file_location("_dlspm_torch", CALLS_PATH)
+    calls = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(calls)
+    calls.register_fallbacks(_spmm, _sddmm, _fused, Prepared, _raise)
+    globals().update(spmm=calls.spmm, sddmm=calls.sddmm, fused=calls.fused)
+    return globals()[name]
+
+
 def _csr_sizes(row_offsets, col_indices):
     if row_offsets.numel() < 1:
         raise ValueError("row_offsets must hold M + 1 >= 1 entries")
@@ -378,7 +403,7 @@ def _workspace_args(workspace, plan, M, banded=False):
     return pointer, size | hint
 
 
-def spmm(row_offsets, col_indices, values, B, K=None, out=None, workspace=None, plan=None, banded=False):
+def _spmm(row_offsets, col_indices, values, B, K=None, out=None, workspace=None, plan=None, banded=False):
     """C = A_csr @ B on the current stream (spmm_csr_f32). row_offsets/col_indices int32, values/B float32, all on
     the GPU. `workspace`: optional GPU tensor of at least workspace_bytes(OP_SPMM, ...) bytes, or ROWS_EVEN.
     `plan`: optional row plan of this matrix (row_plan()), passed as the workspace with DLSPM_HINT_ROW_PLAN.
@@ -428,7 +453,7 @@ def spmm_static(row_offsets, col_indices, values, B, K=None, out=None):
     return out
 
 
-def sddmm(row_offsets, col_indices, lhs, rhs, out=None, workspace=None, plan=None, banded=False):
+def _sddmm(row_offsets, col_indices, lhs, rhs, out=None, workspace=None, plan=None, banded=False):
     """out[j] = <lhs[i], rhs[col[j]]> for each CSR slot j of row i, on the current stream (sddmm_csr_f32).
     `workspace`: None, ROWS_EVEN, or a GPU tensor of workspace_bytes(OP_SDDMM, ...) bytes (the slice boundaries of the
     column-sliced schedule; 0 bytes where that schedule does not apply). `plan`: a row plan of the mask instead."""
@@ -451,7 +476,7 @@ def sddmm(row_offsets, col_indices, lhs, rhs, out=None, workspace=None, plan=Non
     return out
 
 
-def fused(row_offsets, col_indices, Q, Kmat, V, scale=1.0, out=None, workspace=None, plan=None, banded=False):
+def _fused(row_offsets, col_indices, Q, Kmat, V, scale=1.0, out=None, workspace=None, plan=None, banded=False):
     """O = (S .* (Q Kmat^T) * scale) V on the current stream (fused_sddmm_spmm_f32); the scores are never stored.
     `workspace`: optional GPU tensor of at least workspace_bytes(OP_FUSED, ...) bytes, or ROWS_EVEN.
     `plan`: optional row plan of the mask (row_plan()), passed as the workspace with DLSPM_HINT_ROW_PLAN."""
