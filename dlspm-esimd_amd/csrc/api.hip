@@ -431,7 +431,7 @@ int dlspm_set_tuning(const dlspm_tuning* t)
         t->tile_major < -1 || t->tile_major > 3 || t->tile_width < 0 || t->plan_order < 0 || t->plan_order > 2 ||
         t->xcd_contiguous < 0 || t->xcd_contiguous > 1 || t->stream_results < -1 || t->stream_results > 1 ||
         (t->cut_piece_pct != 0 && (t->cut_piece_pct < 10 || t->cut_piece_pct > 1000)) ||
-        (t->cut_longest_pct != 0 && (t->cut_longest_pct < 10 || t->cut_longest_pct > 1000)) || t->rules_off < 0 || t->rules_off > 2047 ||
+        (t->cut_longest_pct != 0 && (t->cut_longest_pct < 10 || t->cut_longest_pct > 1000)) || t->rules_off < 0 || t->rules_off > 4095 ||
         (t->compute_units != 0 && (t->compute_units < 8 || t->compute_units > 1024 || t->compute_units % 8 != 0)))
         return DLSPM_E_INVALID_ARG;
     t_tuning.split_w = t->split_w;
@@ -487,10 +487,15 @@ int spmm_csr_f32(int M, int K, int N, int nnz, const int* row_offsets, const int
     const SpmmArgs args{M, K, N, nnz, row_offsets, col_indices, values, B, C, ws.banded ? 1 : 0};
     hipStream_t st = static_cast<hipStream_t>(stream);
     hipError_t e;
+    const ResidentPlan resident = ws.banded ? ResidentPlan{0, 0, 0} : spmm_resident_choose(dev, M, K, N, nnz, ws.rows_even, ws.mem && (ws.row_plan || ws.cut_plan));
     if (ws.cut_plan && ws.mem) {
         // the memory holds the cut plan of this matrix and room for the partial rows of its pieces
         const CutPlan cp = cut_plan_layout(M, N, dev.cus);
         if (cp.bytes == 0 || ws.bytes < cp.bytes) return DLSPM_E_WORKSPACE;
+        if (resident.rr > 0) {
+            e = spmm_resident_launch(args, resident, st);
+            return e == hipSuccess ? DLSPM_OK : fail_hip(e);
+        }
         SpmmShape shape = spmm_choose(dev, M, K, N, nnz, vec4, false, true);
         e = spmm_plan_applies(dev, shape, M, N, nnz) ? spmm_pieces_launch(args, shape, cp, ws.mem, st)
                                                 : spmm_launch(args, spmm_choose(dev, M, K, N, nnz, vec4, false, true, false, true), st);
@@ -498,6 +503,10 @@ int spmm_csr_f32(int M, int K, int N, int nnz, const int* row_offsets, const int
     }
     if (ws.row_plan && ws.mem) {
         // the memory holds the row plan of this matrix; sizes a planned launch is not built for run as with NULL
+        if (resident.rr > 0) {
+            e = spmm_resident_launch(args, resident, st);
+            return e == hipSuccess ? DLSPM_OK : fail_hip(e);
+        }
         SpmmShape shape = spmm_choose(dev, M, K, N, nnz, vec4, false, true);
         e = spmm_plan_applies(dev, shape, M, N, nnz) ? spmm_planned_launch(args, shape, static_cast<const int*>(ws.mem), st)
                                                 : spmm_launch(args, spmm_choose(dev, M, K, N, nnz, vec4, false, true, false, true), st);
@@ -511,14 +520,16 @@ int spmm_csr_f32(int M, int K, int N, int nnz, const int* row_offsets, const int
         const SlicePlan sliced = spmm_slice_plan(dev, M, K, N, nnz, shape);
         const FlatPlan plan = sliced.slices > 0 ? FlatPlan{0, 0, 0} : flat_plan(dev, M, nnz, N, shape.G);
         if (ws.bytes < (sliced.slices > 0 ? sliced.bytes : plan.bytes)) return DLSPM_E_WORKSPACE;
-        if (sliced.slices > 0)
+        if (resident.rr > 0)
+            e = spmm_resident_launch(args, resident, st);
+        else if (sliced.slices > 0)
             e = spmm_sliced_launch(args, shape, sliced, ws.mem, st);
         else if (plan.chunk > 0)
             e = spmm_flat_launch(args, shape, plan, static_cast<float*>(ws.mem), st);
         else
             e = spmm_launch(args, shape, st);
     } else {
-        e = spmm_launch(args, shape, st);
+        e = resident.rr > 0 ? spmm_resident_launch(args, resident, st) : spmm_launch(args, shape, st);
     }
     return e == hipSuccess ? DLSPM_OK : fail_hip(e);
 }

@@ -101,7 +101,7 @@ struct Tuning {
 // (the values of DLSPM_RULE_* in the header)
 constexpr int kRuleEightWavesFewRows = 1, kRuleSixteenWavesTallLongRows = 2, kRuleMoreWavesFewLongRows = 4, kRuleGroupRows = 8,
               kRuleRowAlignedSplit = 16, kRulePlanUngroups = 32, kRuleExactWidthKernels = 64, kRuleCutRowsByColumns = 128,
-              kRuleFinerColumnTiles = 256, kRuleRowPiecesFewRows = 512, kRuleMaskByRange = 1024;
+              kRuleFinerColumnTiles = 256, kRuleRowPiecesFewRows = 512, kRuleMaskByRange = 1024, kRuleResidentSlices = 2048;
 
 const Tuning& tuning();
 inline bool rule_on(int rule) { return (tuning().rules_off & rule) == 0; }
@@ -216,6 +216,12 @@ hipError_t spmm_flat_launch(const SpmmArgs& x, const SpmmShape& s, const FlatPla
                             hipStream_t stream);
 hipError_t spmm_sliced_launch(const SpmmArgs& x, const SpmmShape& s, const SlicePlan& plan, void* workspace,
                               hipStream_t stream);
+
+// Resident schedule of SpMM (resident.hip): workgroups of sixteen waves own 64 x rr rows and 64 columns and go through slices of
+// `slice` rows of B that lie in LDS, with `chunks` x 64 (column, value) pairs of every row loaded ahead. rr == 0: not used.
+struct ResidentPlan { int rr, chunks, slice; };
+ResidentPlan spmm_resident_choose(const DeviceInfo& dev, int M, int K, int N, int nnz, bool rows_even, bool planned);
+hipError_t spmm_resident_launch(const SpmmArgs& x, const ResidentPlan& plan, hipStream_t stream);
 
 SddmmShape sddmm_choose(const DeviceInfo& dev, int M, int D, int nnz, bool vec4, int rows = kRowsUnknown);
 void sddmm_few_rows_pieces(const DeviceInfo& dev, SddmmShape& s, int M, int nnz);  // a call without plan or memory: sets s.pieces_lg (and W = 4)

@@ -42,6 +42,9 @@
  *         row at most one and a half times nnz / M). Tall matrices of long rows then run one whole row per wave, which
  *         is the faster split for even rows and the slower one for uneven rows. A hint about speed only: a wrong one
  *         costs time, never correctness (a row's products are added in a different, equally fixed order).
+ *       Matrices dense enough that each row of B serves many rows of a workgroup (from a density of about 0.05 on under the
+ *         even-rows hint, about 0.15 otherwise) are multiplied from slices of B in LDS where that is estimated to be faster;
+ *         memory or a plan that comes with such a call is not used. (Not under DLSPM_HINT_BANDED.)
  *       DLSPM_HINT_ROW_PLAN: `workspace` holds the row plan of this matrix (dlspm_row_plan_build, below; at least
  *         dlspm_row_plan_bytes(M) bytes, else DLSPM_E_WORKSPACE) and the launch hands the rows out in the plan's order.
  *         The plan is only read.
@@ -405,6 +408,7 @@ typedef struct dlspm_tuning {
                                                    /* (not 32, 64, 96, 128, 192, 256, 384, 512): rhs read as a buffer of 1 GiB    */
                                                    /* whose range check zeroes the lanes past D, where rhs fits (else: by selects); */
                                                    /* the fused op's first stage likewise at D = 260 ... 380                      */
+#define DLSPM_RULE_RESIDENT_SLICES           2048  /* SpMM on dense enough matrices: slices of B in LDS, whatever memory the call has  */
 void dlspm_tuning_default(dlspm_tuning* t);   /* fills *t with "follow the rules" */
 int dlspm_set_tuning(const dlspm_tuning* t);  /* DLSPM_OK or DLSPM_E_INVALID_ARG (a field out of range) */
 int dlspm_get_tuning(dlspm_tuning* t);        /* what the calling thread's launches currently use */
