@@ -9,6 +9,7 @@
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <ATen/hip/EmptyTensor.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -109,7 +110,8 @@ struct Call {
             Py_INCREF(given);
             result = given;
         } else {
-            at::Tensor t = at::empty(sizes, like.options().requires_grad(false));
+            // (at::empty without the dispatcher: every element is written by the call)
+            at::Tensor t = at::detail::empty_cuda(sizes, at::kFloat, like.device(), std::nullopt);
             out = static_cast<float*>(address(t));
             result = THPVariable_Wrap(std::move(t));
         }
