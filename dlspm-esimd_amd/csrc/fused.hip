@@ -54,6 +54,176 @@ __device__ __forceinline__ void fused_segment(Vec<VEC>* acc, int p, int q, int D
     if constexpr (kWave / G > 1) slots_sum<VEC, G, V2>(acc, lane);
 }
 
+constexpr int kDenseSpan = 304;  // (p of fused_dense_group: 20 KB, eight workgroups per compute unit)
+// the row-block shapes that fused_dense_group is built for: 33 ... 128 columns, four-wave workgroups
+template <int VEC, int DS, int V2, int W, int R>
+constexpr bool kDenseGroups = VEC == 4 && DS >= 2 && DS <= 4 && V2 == 1 && W == 4 && R <= 16;
+
+// Sixteen consecutive rows whose columns form one run (sliding-window masks without other columns): the leading workgroup of the
+// group computes them on the matrix cores, the others leave. What bounds the row-by-row path is the vector-memory path of
+// the compute unit, through which every row gathers its own rows of Kmat and V; here each of them is read once for all sixteen
+// and the time is that of the workgroups' chains of loads (three operand sets in turn, before -> after: 16384 rows, 128
+// columns per row, D = 128: 69 -> 38 us, D = 64: 37 -> 24 us; 8000 rows of 250, D = 80: 57 -> 33 us).
+//   1  p[r][x] <- 1 where row r has column c0 + x (LDS; plain stores: LDS float atomics took 9 us of the first figure)
+//   2  16 x 16 tiles of Q Kmat^T by v_mfma_f32_16x16x4_f32, one wave per tile; p[r][x] <- scale x score where marked
+//   3  O = p V by the same instruction, D / 4 columns of O per wave
+// The k index of both products is permuted so that a lane's four k are consecutive floats in memory (one dwordx4); in step 3 the
+// columns of O are dealt to the lanes in pairs for the same reason.
+// Taken where the span of the columns, which the first and last column of each row say if they ascend, has at most kDenseSpan
+// columns and a quarter of its 16 x span positions and more are nonzeros. Columns outside it (rows that do not ascend),
+// columns that come twice (fewer marks than nonzeros) and results that are not finite (a weight of zero times an infinity of
+// V is not what the row-by-row path computes) send the rows through the row-by-row path, wave by wave.
+// Returns true if the rows are done or another workgroup's.
+template <int G1, int DS, int MASKED, int G, int V2>
+__device__ __forceinline__ bool fused_dense_group(int row0, bool leads, int offsets, int M, int D, float scale, int stream_rule,
+                                                  const int* __restrict__ col_indices,
+                                                  const float* __restrict__ Q, const float* __restrict__ Kmat,
+                                                  const float* __restrict__ Vmat, float* __restrict__ O)
+{
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    constexpr int kRows = 16, kStride = kDenseSpan + 4, NQ = 2 * DS, NT = DS <= 2 ? 1 : 2;
+    __shared__ __attribute__((aligned(16))) float s_p[kRows * kStride];
+    __shared__ int s_left, s_marks;
+    if (row0 + kRows > M) return false;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = lane & 15, kq = lane >> 4;
+    const int from = lane_get(offsets, l), to = lane_get(offsets, l + 1);
+    int edge = 0x7fffffff;  // lanes 0 ... 15: the rows' first columns, lanes 16 ... 31: minus their last ones
+    if (lane < 32 && to > from) {
+        const int c = col_indices[lane & 16 ? to - 1 : from];
+        edge = lane & 16 ? -c : c;
+    }
+    edge = min(edge, __builtin_amdgcn_update_dpp(0, edge, kDppQuadSwap1, 0xF, 0xF, true));
+    edge = min(edge, __builtin_amdgcn_update_dpp(0, edge, kDppQuadSwap2, 0xF, 0xF, true));
+    edge = min(edge, __builtin_amdgcn_update_dpp(0, edge, kDppRowHalfMirror, 0xF, 0xF, true));
+    edge = min(edge, __builtin_amdgcn_update_dpp(0, edge, kDppRowMirror, 0xF, 0xF, true));
+    const int c0 = __builtin_amdgcn_readlane(edge, 0), span = -__builtin_amdgcn_readlane(edge, 16) - c0 + 1;
+    const int T = __builtin_amdgcn_readlane(offsets, 16) - __builtin_amdgcn_readlane(offsets, 0);
+    if (T <= 0 || span <= 0 || span > kDenseSpan || T < 4 * span) return false;
+    if (!leads) return true;
+    const int tiles = (span + 15) >> 4;
+
+    // four consecutive floats of a row, the q-th sixteen of them dealt to the four k of the lanes (zero past D)
+    auto quad = [&](const float* a, int row, int q) -> f4 {
+        const int d = 16 * q + 4 * kq;
+        const bool in = !MASKED || d < D;
+        const Vec<4> x = Vec<4>::gload(a + (size_t)row * D + (in ? d : 0));
+        return in ? f4{x.v.x, x.v.y, x.v.z, x.v.w} : f4{0.f, 0.f, 0.f, 0.f};
+    };
+    f4 qf[NQ], kf[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) qf[q] = quad(Q, row0 + l, q);
+    auto load_k = [&](int t) {
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) kf[q] = quad(Kmat, c0 + min(16 * t + l, span - 1), q);
+    };
+    if (w < tiles) load_k(w);
+    {
+        float* const mine = s_p + (threadIdx.x >> 4) * kStride;
+        for (int x = l * 4; x < tiles * 16; x += 64) *reinterpret_cast<f4*>(mine + x) = f4{0.f, 0.f, 0.f, 0.f};
+    }
+    if (threadIdx.x == 0) s_left = s_marks = 0;
+    __syncthreads();
+    {
+        int at[4], end[4], longest = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            at[j] = __builtin_amdgcn_readlane(offsets, 4 * w + j);
+            end[j] = __builtin_amdgcn_readlane(offsets, 4 * w + j + 1);
+            longest = max(longest, end[j] - at[j]);
+        }
+        for (int base = lane; base - lane < longest; base += kWave) {
+            int c[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) c[j] = col_indices[max(min(at[j] + base, end[j] - 1), 0)];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                if (at[j] + base >= end[j]) continue;
+                const int x = c[j] - c0;
+                if ((unsigned)x < (unsigned)span) s_p[(4 * w + j) * kStride + x] = 1.f;
+                else s_left = 1;
+            }
+        }
+    }
+    __syncthreads();
+    bool left = s_left != 0;
+    if (!left) {
+        int marks = 0;
+        for (int t = w; t < tiles; t += 4) {
+            f4 score = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int q = 0; q < NQ; ++q)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) score = __builtin_amdgcn_mfma_f32_16x16x4f32(qf[q][j], kf[q][j], score, 0, 0, 0);
+            if (t + 4 < tiles) load_k(t + 4);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {  // row 4 kq + i, column 16 t + l
+                float* const p = s_p + (4 * kq + i) * kStride + 16 * t + l;
+                const bool marked = *p > 0.f;
+                marks += marked ? 1 : 0;
+                *p = marked ? score[i] * scale : 0.f;
+            }
+        }
+        marks += __builtin_amdgcn_update_dpp(0, marks, kDppQuadSwap1, 0xF, 0xF, true);
+        marks += __builtin_amdgcn_update_dpp(0, marks, kDppQuadSwap2, 0xF, 0xF, true);
+        marks += __builtin_amdgcn_update_dpp(0, marks, kDppRowHalfMirror, 0xF, 0xF, true);
+        marks += __builtin_amdgcn_update_dpp(0, marks, kDppRowMirror, 0xF, 0xF, true);
+        if (l == 0) __hip_atomic_fetch_add(&s_marks, marks, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        __syncthreads();
+        const int d = min(w * 16 * NT + NT * l, D - NT);  // (lanes past D repeat the last columns and store nothing)
+        f4 acc[NT];
+#pragma unroll
+        for (int n = 0; n < NT; ++n) acc[n] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 2
+        for (int t = 0; t < tiles; ++t) {
+            const f4 p = *reinterpret_cast<const f4*>(s_p + l * kStride + 16 * t + 4 * kq);
+            float v[4][NT];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const float* row = Vmat + (size_t)(c0 + min(16 * t + 4 * kq + j, span - 1)) * D + d;
+                if constexpr (NT == 2) {
+                    typedef float f2 __attribute__((ext_vector_type(2), aligned(4)));
+                    const f2 x = *reinterpret_cast<const f2*>(row);
+                    v[j][0] = x.x;
+                    v[j][1] = x.y;
+                } else v[j][0] = *row;
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int n = 0; n < NT; ++n) acc[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[j], v[j][n], acc[n], 0, 0, 0);
+        }
+        bool finite = true;
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) finite = finite && fabsf(acc[n][i]) < __builtin_inff();
+        if (!finite) s_left = 1;
+        __syncthreads();
+        left = s_left != 0 || s_marks != T;
+        if (!left) {
+            const bool streaming = stream_rule != 1 && (stream_rule == 2 || (long long)M * D >= 1024 * 1024);
+            if (w * 16 * NT + NT * l < D) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    float* const o = O + (size_t)(row0 + 4 * kq + i) * D + d;
+#pragma unroll
+                    for (int n = 0; n < NT; ++n) Vec<1>{acc[n][i]}.gstore(o + n, streaming);
+                }
+            }
+            return true;
+        }
+    }
+    // row by row: four rows per wave
+    const int g = lane % G, col = g * 4, colv[1] = {col < D ? min(col, D - 4) : 0};
+    for (int j = 0; j < 4; ++j) {
+        const int r = 4 * w + j, p = __builtin_amdgcn_readlane(offsets, r), q = __builtin_amdgcn_readlane(offsets, r + 1);
+        Vec<4> acc[1] = {Vec<4>::zero()};
+        if (q > p) fused_segment<4, G1, DS, MASKED, G, 1>(acc, p, q, D, scale, col_indices, Q + (size_t)(row0 + r) * D, Kmat, Vmat, colv, lane);
+        if (lane / G == 0 && col < D) acc[0].gstore(O + (size_t)(row0 + r) * D + colv[0]);
+    }
+    return true;
+}
+
 // The work of workgroup `bid` (RowBlock in common.hpp explains SLICED and PLANNED: with PLANNED workgroup i works on row
 // row_ids[i] of Q, O and the mask). Column tiles (D > 1024) tile-major, as in spmm_block; no division in the usual
 // case of one tile.
@@ -68,10 +238,29 @@ __device__ __forceinline__ void fused_block(int bid, int M, int D, int col_tiles
 {
     const int row_blocks = (M - 1) / R + 1;  // (planned launches have one column tile)
     const int ct = col_tiles == 1 ? 0 : bid / row_blocks;
-    const int rb = bid - ct * row_blocks;
+    int rb = bid - ct * row_blocks;
+    if constexpr (kDenseGroups<VEC, DS, V2, W, R> && !SLICED && !PLANNED) {
+        // Runs of 32 row blocks per XCD (workgroup 8 k + x runs on XCD x): the rows of Kmat and V that neighbouring groups
+        // share are then fetched into one L2. Which of a group's n workgroups leads changes with the group, so that the
+        // leaders lie on all compute units: an XCD's workgroups k go to its four shader engines, and there to the eight
+        // compute units, in turn (4096 rows, 64 columns per row, D = 64: 6.3 us; all leaders on a quarter of them: 9.8 us).
+        if (flags & kFlagDenseGroups) {
+            if (rb < (row_blocks & ~255)) rb = (rb & ~255) + ((rb & 7) << 5) + ((rb >> 3) & 31);
+            constexpr int n = 16 / R;
+            const int group = rb / n, leader = n > 1 ? ((((rb >> 8) << 5) + (rb & 31)) / n / 8) % n : 0;
+            const int offsets = row_offsets[min(group * 16 + min((int)(threadIdx.x & 63), 16), M)], first = rb % n * R;
+            // (a first row that spans more than fused_dense_group takes settles it for all workgroups of the group, by two columns
+            // of the row that the row-by-row path reads next; the leader does not wait for them)
+            const int from = __builtin_amdgcn_readlane(offsets, first), to = __builtin_amdgcn_readlane(offsets, first + 1);
+            if ((rb % n == leader || to <= from || col_indices[to - 1] - col_indices[from] < kDenseSpan) &&
+                fused_dense_group<G1, DS, MASKED, G, V2>(group * 16, rb % n == leader, offsets, M, D, scale, (flags >> 1) & 3, col_indices,
+                                                        Q, Kmat, Vmat, O))
+                return;
+        }
+    }
     RowBlock<W, R, SLICED, PLANNED> blk;
     blk.load(rb, M, nnz, row_offsets, row_ends, row_ids, [&]() { fetch_args_now(col_indices, Q, Kmat, Vmat, O); },
-             col_tiles == 1 ? flags : flags & ~1, row_slots, slots);
+             col_tiles == 1 && !(flags & kFlagDenseGroups) ? flags : flags & ~1, row_slots, slots);
     dense_rows_block<VEC, G, V2>(
         blk, ct, D, O,
         [&](Vec<VEC>* acc, int r, int p, int q, const int* colv) {
@@ -156,6 +345,21 @@ template <int DS> static bool stage1_masked_by_range(int K, int D)
 }
 template <int DS> constexpr int stage1_masked_kind(bool by_range) { return by_range && DS == 12 ? kMaskedByRange : kMaskedBySelect; }
 
+// Whether the row-block launch looks for groups of rows whose columns form one run (fused_dense_group; the kernels built for it
+// are those of 33 ... 128 columns). The look costs every workgroup one more dependent load: nothing measurable on calls of about
+// 45 us and more by the row-by-row path (16384 rows of 128 random columns, D = 128: 201.5 us with and without; 8192 x 2048,
+// 205 per row, D = 84: 55.6 and 55.8 us), but 2-5 % on smaller ones that have no such groups (8192 rows, window of 64 and 24
+// random columns, D = 64: 18.1 -> 19.2 us). Nor on masks whose mean row is longer than a group's span or takes more than a
+// twelfth of the columns, which are seldom windows (1 % of 680 us at 30 % density, 0.8 % of 45 us at 10 %).
+constexpr double kDenseGroupsMinFloats = 1.2e8;  // nnz x D
+static int fused_flags(const FusedArgs& x)
+{
+    const long long nnz = x.nnz;
+    const bool groups = x.D % 4 == 0 && (double)nnz * x.D >= kDenseGroupsMinFloats && nnz >= 16ll * x.M &&
+                        nnz <= (long long)kDenseSpan * x.M && 12 * nnz <= (long long)x.M * x.K && rule_on(kRuleDenseGroups);
+    return launch_flags(x.xcd_contiguous) | (groups ? kFlagDenseGroups : 0);
+}
+
 template <int VEC, int G1, int DS, int G, int V2, int W, int R>
 static hipError_t launch_one(const FusedArgs& x, hipStream_t stream)
 {
@@ -167,7 +371,7 @@ static hipError_t launch_one(const FusedArgs& x, hipStream_t stream)
     if constexpr (DS > 0) {
         if (x.D == G1 * VEC * DS && rule_on(kRuleExactWidthKernels)) {
             hipLaunchKernelGGL((fused_kernel<VEC, G1, DS, false, G, V2, W, R>), dim3((unsigned)blocks), dim3(W * 64),
-                               0, stream, x.M, x.D, col_tiles, launch_flags(x.xcd_contiguous), x.scale, x.row_offsets, x.col_indices,
+                               0, stream, x.M, x.D, col_tiles, fused_flags(x), x.scale, x.row_offsets, x.col_indices,
                                x.Q, x.Kmat, x.V, x.O);
             return hipGetLastError();
         }
@@ -175,13 +379,13 @@ static hipError_t launch_one(const FusedArgs& x, hipStream_t stream)
     if constexpr (VEC == 4 && G1 == 8 && DS == 12) {
         if (stage1_masked_by_range<DS>(x.K, x.D)) {
             hipLaunchKernelGGL((fused_kernel<VEC, G1, DS, kMaskedByRange, G, V2, W, R>), dim3((unsigned)blocks), dim3(W * 64), 0, stream,
-                               x.M, x.D, col_tiles, launch_flags(x.xcd_contiguous), x.scale, x.row_offsets, x.col_indices, x.Q, x.Kmat,
+                               x.M, x.D, col_tiles, fused_flags(x), x.scale, x.row_offsets, x.col_indices, x.Q, x.Kmat,
                                x.V, x.O);
             return hipGetLastError();
         }
     }
     hipLaunchKernelGGL((fused_kernel<VEC, G1, DS, kMaskedBySelect, G, V2, W, R>), dim3((unsigned)blocks), dim3(W * 64), 0, stream,
-                       x.M, x.D, col_tiles, launch_flags(x.xcd_contiguous), x.scale, x.row_offsets, x.col_indices, x.Q, x.Kmat, x.V,
+                       x.M, x.D, col_tiles, fused_flags(x), x.scale, x.row_offsets, x.col_indices, x.Q, x.Kmat, x.V,
                        x.O);
     return hipGetLastError();
 }

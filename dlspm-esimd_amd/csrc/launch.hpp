@@ -101,7 +101,8 @@ struct Tuning {
 // (the values of DLSPM_RULE_* in the header)
 constexpr int kRuleEightWavesFewRows = 1, kRuleSixteenWavesTallLongRows = 2, kRuleMoreWavesFewLongRows = 4, kRuleGroupRows = 8,
               kRuleRowAlignedSplit = 16, kRulePlanUngroups = 32, kRuleExactWidthKernels = 64, kRuleCutRowsByColumns = 128,
-              kRuleFinerColumnTiles = 256, kRuleRowPiecesFewRows = 512, kRuleMaskByRange = 1024, kRuleResidentSlices = 2048;
+              kRuleFinerColumnTiles = 256, kRuleRowPiecesFewRows = 512, kRuleMaskByRange = 1024, kRuleResidentSlices = 2048,
+              kRuleDenseGroups = 4096;
 
 const Tuning& tuning();
 inline bool rule_on(int rule) { return (tuning().rules_off & rule) == 0; }
@@ -112,7 +113,7 @@ inline bool rule_on(int rule) { return (tuning().rules_off & rule) == 0; }
 // bit 3 = never take the row-aligned split (DLSPM_RULE_ROW_ALIGNED_SPLIT switched off); bit 4 (SDDMM, one row per
 // workgroup) = the waves of a row take whole passes of 64 nonzeros in turn (sddmm_row_interleaved).
 constexpr int kFlagXcdContiguous = 1, kFlagStreamShift = 1, kFlagStreamNever = 1, kFlagStreamAlways = 2, kFlagNoAlignedSplit = 8,
-              kFlagFullPasses = 16, kFlagPiecesShift = 8, kFlagPiecesMask = 7, kFlagTileOrderShift = 12;  // (bits 8-10: log2 of the workgroups that share a row, SDDMM; bits 12-13: SpmmShape::tile_major of a planned SpMM launch)
+              kFlagFullPasses = 16, kFlagPiecesShift = 8, kFlagPiecesMask = 7, kFlagTileOrderShift = 12, kFlagDenseGroups = 1 << 14;  // (bits 8-10: log2 of the workgroups that share a row, SDDMM; bits 12-13: SpmmShape::tile_major of a planned SpMM launch; bit 14: fused_dense_group)
 inline int launch_flags(int xcd_contiguous_hint)
 {
     const Tuning& t = tuning();
