@@ -240,6 +240,8 @@ int dlspm_advise(int op, int N_or_D, const dlspm_matrix_info* info, dlspm_call_p
     if (M <= 0 || K <= 0 || nnz <= 0 || N_or_D <= 0) return DLSPM_OK;
     const DeviceInfo& dev = device_info();
     const bool even = (double)longest <= 1.5 * ((double)nnz / M);
+    // (dense tiles look at neither hints nor memory)
+    if (op == DLSPM_OP_SDDMM && sddmm_tiles_choose(dev, M, K, N_or_D, nnz).ranges > 0) return DLSPM_OK;
     // 1. a band: row blocks dealt to the XCDs in contiguous runs, no memory (with the even-rows hint where that holds too)
     if (looks_banded(dev, op, N_or_D, *info)) {
         plan->hints = DLSPM_HINT_BANDED | (even ? DLSPM_HINT_ROWS_EVEN : 0);

@@ -413,6 +413,7 @@ template <typename Shape> struct Call {
     int schedule = DLSPM_SCHEDULE_ROW_BLOCKS;
     Shape shape{};
     ResidentPlan resident{0, 0, 0};
+    TilePlan tiles{0};  // SDDMM: ranges > 0: dense tiles on the matrix cores in place of the schedule
     CutPlan cut{};
     SlicePlan sliced{0, 1, 0, 0};
     FlatPlan flat{0, 0, 0};
@@ -463,6 +464,8 @@ static SpmmCall spmm_decide(const DeviceInfo& dev, int M, int K, int N, int nnz,
 static SddmmCall sddmm_decide(const DeviceInfo& dev, int M, int K, int D, int nnz, const WorkspaceArg& ws)
 {
     SddmmCall c;
+    // (by the sizes alone, so that the bits do not depend on what comes with the call)
+    c.tiles = sddmm_tiles_choose(dev, M, K, D, nnz);
     const bool vec4 = D >= 4;
     if (ws.cut_plan && ws.mem) {
         c.cut = cut_plan_layout(M, 0, dev.cus);
@@ -851,7 +854,8 @@ int sddmm_csr_f32(int M, int K, int D, int nnz, const int* row_offsets, const in
     if (c.status != DLSPM_OK) return c.status;
     const SddmmArgs args{M, K, D, nnz, row_offsets, col_indices, lhs, rhs, out_values, ws.banded ? 1 : 0, dev.l2_bytes, dev.cus};
     hipError_t e;
-    switch (c.schedule) {
+    if (c.tiles.ranges > 0) e = sddmm_tiles_launch(args, c.tiles, st);
+    else switch (c.schedule) {
         case DLSPM_SCHEDULE_CUT_PLAN: e = sddmm_pieces_launch(args, c.shape, c.cut, ws.mem, st); break;
         case DLSPM_SCHEDULE_ROW_PLAN: e = sddmm_planned_launch(args, c.shape, static_cast<const int*>(ws.mem), st); break;
         case DLSPM_SCHEDULE_SLICED: e = sddmm_sliced_launch(args, c.shape, c.sliced, ws.mem, st); break;
@@ -1036,6 +1040,10 @@ int dlspm_describe_schedule(int op, int M, int K, int N_or_D, int nnz, size_t wo
         status = c.status;
         schedule[0] = c.schedule;
         schedule[1] = c.schedule == DLSPM_SCHEDULE_SLICED ? c.sliced.R : c.shape.R;
+        if (c.tiles.ranges > 0 && status == DLSPM_OK) {
+            sddmm_tile_shape(&schedule[1], &schedule[2]);
+            return status;
+        }
     } else if (op == DLSPM_OP_FUSED) {
         const FusedCall c = fused_decide(dev, M, K, N_or_D, nnz, ws);
         status = c.status;

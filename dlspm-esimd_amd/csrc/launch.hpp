@@ -229,6 +229,11 @@ hipError_t spmm_resident_launch(const SpmmArgs& x, const ResidentPlan& plan, hip
 SddmmShape sddmm_choose(const DeviceInfo& dev, int M, int D, int nnz, bool vec4, int rows = kRowsUnknown);
 void sddmm_few_rows_pieces(const DeviceInfo& dev, SddmmShape& s, int M, int nnz);  // a call without plan or memory: sets s.pieces_lg (and W = 4)
 hipError_t sddmm_launch(const SddmmArgs& x, const SddmmShape& s, hipStream_t stream);
+// Dense tiles on the matrix cores (sddmm_tiles.hip): the columns in `ranges` runs, each with its workgroups. ranges == 0: not used.
+struct TilePlan { int ranges; };
+TilePlan sddmm_tiles_choose(const DeviceInfo& dev, int M, int K, int D, int nnz);
+void sddmm_tile_shape(int* rows, int* columns);
+hipError_t sddmm_tiles_launch(const SddmmArgs& x, const TilePlan& plan, hipStream_t stream);
 hipError_t sddmm_flat_launch(const SddmmArgs& x, const SddmmShape& s, int chunk, hipStream_t stream);
 hipError_t sddmm_sliced_launch(const SddmmArgs& x, const SddmmShape& s, const SlicePlan& plan, void* workspace,
                                hipStream_t stream);

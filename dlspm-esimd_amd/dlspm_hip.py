@@ -546,11 +546,14 @@ SCHEDULES = ("row_blocks", "flat", "sliced", "row_plan", "cut_plan", "resident",
 
 def describe_schedule(op: int, M: int, K: int, N: int, nnz: int, plan=None, workspace_bytes: int = 0) -> dict:
     """The schedule that a call runs (dlspm_describe_schedule): {'schedule' (one of SCHEDULES), 'rows' per workgroup, 'slice_rows',
-    'chunks'}. plan: what prepare() returned; or workspace_bytes: the size, with hint bits, that the call passes."""
+    'chunks'}; SDDMM on dense tiles also {'tile_columns'}, with 'rows' those of a tile and 'schedule' the one without tiles. plan: what
+    prepare() returned; or workspace_bytes: the size, with hint bits, that the call passes."""
     out = (ctypes.c_int * 4)()
     st = lib().dlspm_describe_schedule(op, M, K, N, nnz, plan.size_and_hints if plan is not None else workspace_bytes, out)
     if st != OK:
         raise DlspmError(st, "dlspm_describe_schedule")
+    if op == OP_SDDMM and out[2] > 0:
+        return {"schedule": SCHEDULES[out[0]], "rows": out[1], "slice_rows": 0, "chunks": 0, "tile_columns": out[2]}
     return {"schedule": SCHEDULES[out[0]], "rows": out[1], "slice_rows": out[2], "chunks": out[3]}
 
 

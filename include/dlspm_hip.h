@@ -354,7 +354,9 @@ int dlspm_describe_launch_rows(int op, int M, int K, int N_or_D, int nnz, int pa
  * The schedule that a call would run, for these sizes and the `workspace_bytes` that is passed with it (size and hint bits; a
  * size other than 0 stands for memory of that size). The compute entry points decide by the same function. schedule[4]
  * receives: [0] DLSPM_SCHEDULE_*, [1] rows per workgroup (0: flat schedule), and, where [0] is DLSPM_SCHEDULE_RESIDENT, [2] rows
- * of B per slice and [3] chunks of 64 nonzeros of a row that are loaded ahead (else 0). The shapes that
+ * of B per slice and [3] chunks of 64 nonzeros of a row that are loaded ahead (else 0). SDDMM on dense tiles (masks dense enough:
+ * the matrix cores compute whole tiles and the sampled results are picked from them): [1] rows and [2] columns of a tile, [0] the
+ * schedule that the call would run without DLSPM_RULE_DENSE_GROUPS. The shapes that
  * dlspm_describe_launch_rows gives are those of DLSPM_SCHEDULE_ROW_BLOCKS and _FLAT (and, as far as the fields go, of
  * _DENSE_GROUPS for the rows that are not in groups). Host-only. DLSPM_OK, DLSPM_E_WORKSPACE where the call would be
  * refused for its size, or DLSPM_E_INVALID_ARG.
