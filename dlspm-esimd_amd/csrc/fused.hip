@@ -61,12 +61,13 @@ constexpr bool dense_groups_built(int vec, int DS, int V2, int W, int R) { retur
 // Sixteen consecutive rows whose columns form one run (sliding-window masks without other columns): the leading workgroup of the
 // group computes them on the matrix cores, the others leave. What bounds the row-by-row path is the vector-memory path of
 // the compute unit, through which every row gathers its own rows of Kmat and V; here each of them is read once for all sixteen
-// and the time is that of the workgroups' chains of loads (three operand sets in turn, before -> after: 16384 rows, 128
-// columns per row, D = 128: 69 -> 38.6 us, D = 64: 37 -> 21.4 us).
+// and the time is that of the workgroups' chains of loads and, with four workgroups per compute unit, of the fp32 matrix cores (9
+// us; three operand sets in turn, row by row -> here: 16384 rows, 128 columns per row, D = 128: 69 -> 29.1 us, D = 64: 37 -> 17.0 us;
+// 38.6 and 21.4 while a row's columns were loaded 64 at a time, V two tiles ahead and a group led by one of its own workgroups).
 //   1  p[r][x] <- 1 where row r has column c0 + x (LDS; plain stores: LDS float atomics took 9 us of the first figure)
 //   2  16 x 16 tiles of Q Kmat^T by v_mfma_f32_16x16x4_f32, one wave per tile; p[r][x] <- scale x score where marked
 //   3  O = p V by the same instruction, D / 4 columns of O per wave
-// A score is summed in eight chains of D / 8 products as the row-by-row path does, a row of O in four chains per kSumTiles tiles
+// A score is summed in eight chains of D / 8 products as the row-by-row path does, a row of O in four chains per kAhead tiles
 // whose sums are added: an error against 64 bits of 1.1e-7 ... 1.3e-7 (the row-by-row path: 1.3e-7 ... 2.4e-7 on the same calls; one
 // chain for each: 2.4e-7 ... 3.2e-7, at 0.97 ... 1.10 of the time).
 // The k index of both products is permuted so that a lane's four k are consecutive floats in memory (one dwordx4); in step 3 the
@@ -75,25 +76,41 @@ constexpr bool dense_groups_built(int vec, int DS, int V2, int W, int R) { retur
 // columns and a quarter of its 16 x span positions and more are nonzeros. Columns outside it (rows that do not ascend),
 // columns that come twice (fewer marks than nonzeros) and results that are not finite (a weight of zero times an infinity of
 // V is not what the row-by-row path computes) send the rows through the row-by-row path, wave by wave.
-// Returns true if the rows are done or another workgroup's.
-template <int G1, int DS, int MASKED, int G, int V2>
-__device__ __forceinline__ bool fused_dense_group(int row0, bool leads, int offsets, int M, int D, float scale, int stream_rule,
+// Returns true if they are such rows, and done where LEADS.
+template <bool LEADS, int G1, int DS, int MASKED, int G, int V2>
+__device__ __forceinline__ bool fused_dense_group(int row0, int offsets, int M, int D, float scale, int stream_rule,
                                                   const int* __restrict__ col_indices,
                                                   const float* __restrict__ Q, const float* __restrict__ Kmat,
                                                   const float* __restrict__ Vmat, float* __restrict__ O)
 {
     typedef float f4 __attribute__((ext_vector_type(4)));
-    constexpr int kRows = 16, kStride = kDenseSpan + 4, NQ = 2 * DS, NT = DS <= 2 ? 1 : 2, kSumTiles = 4;
+    constexpr int kRows = 16, kStride = kDenseSpan + 4, NQ = 2 * DS, NT = DS <= 2 ? 1 : 2;
     __shared__ __attribute__((aligned(16))) float s_p[kRows * kStride];
     __shared__ int s_left, s_marks;
     if (row0 + kRows > M) return false;
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = lane & 15, kq = lane >> 4;
+    // the columns of the wave's four rows, all of them at once (a row of a group has kDenseSpan at most)
+    constexpr int kChunks = (kDenseSpan + kWave - 1) / kWave, kEarly = 3;
+    int at[4], end[4], longest = 0, c[kChunks][4];
+    auto load_columns = [&](int q) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) c[q][j] = col_indices[max(min(at[j] + q * kWave + lane, end[j] - 1), 0)];
+    };
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        at[j] = __builtin_amdgcn_readlane(offsets, 4 * w + j);
+        end[j] = __builtin_amdgcn_readlane(offsets, 4 * w + j + 1);
+        longest = max(longest, end[j] - at[j]);
+    }
     const int from = lane_get(offsets, l), to = lane_get(offsets, l + 1);
     int edge = 0x7fffffff;  // lanes 0 ... 15: the rows' first columns, lanes 16 ... 31: minus their last ones
     if (lane < 32 && to > from) {
-        const int c = col_indices[lane & 16 ? to - 1 : from];
-        edge = lane & 16 ? -c : c;
+        const int at_edge = col_indices[lane & 16 ? to - 1 : from];
+        edge = lane & 16 ? -at_edge : at_edge;
     }
+    if constexpr (LEADS)
+#pragma unroll
+        for (int q = 0; q < kEarly; ++q) load_columns(q);
     edge = min(edge, __builtin_amdgcn_update_dpp(0, edge, kDppQuadSwap1, 0xF, 0xF, true));
     edge = min(edge, __builtin_amdgcn_update_dpp(0, edge, kDppQuadSwap2, 0xF, 0xF, true));
     edge = min(edge, __builtin_amdgcn_update_dpp(0, edge, kDppRowHalfMirror, 0xF, 0xF, true));
@@ -101,7 +118,7 @@ __device__ __forceinline__ bool fused_dense_group(int row0, bool leads, int offs
     const int c0 = __builtin_amdgcn_readlane(edge, 0), span = -__builtin_amdgcn_readlane(edge, 16) - c0 + 1;
     const int T = __builtin_amdgcn_readlane(offsets, 16) - __builtin_amdgcn_readlane(offsets, 0);
     if (T <= 0 || span <= 0 || span > kDenseSpan || T < 4 * span) return false;
-    if (!leads) return true;
+    if constexpr (!LEADS) return true;
     const int tiles = (span + 15) >> 4;
 
     // four consecutive floats of a row, the q-th sixteen of them dealt to the four k of the lanes (zero past D)
@@ -126,25 +143,19 @@ __device__ __forceinline__ bool fused_dense_group(int row0, bool leads, int offs
     if (threadIdx.x == 0) s_left = s_marks = 0;
     __syncthreads();
     {
-        int at[4], end[4], longest = 0;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            at[j] = __builtin_amdgcn_readlane(offsets, 4 * w + j);
-            end[j] = __builtin_amdgcn_readlane(offsets, 4 * w + j + 1);
-            longest = max(longest, end[j] - at[j]);
-        }
-        for (int base = lane; base - lane < longest; base += kWave) {
-            int c[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) c[j] = col_indices[max(min(at[j] + base, end[j] - 1), 0)];
+        for (int q = 0; q < kChunks; ++q) {
+            if (q * kWave >= longest) break;
+            if (q >= kEarly) load_columns(q);
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                if (at[j] + base >= end[j]) continue;
-                const int x = c[j] - c0;
+                if (at[j] + q * kWave + lane >= end[j]) continue;
+                const int x = c[q][j] - c0;
                 if ((unsigned)x < (unsigned)span) s_p[(4 * w + j) * kStride + x] = 1.f;
                 else s_left = 1;
             }
         }
+        if (longest > kChunks * kWave) s_left = 1;  // (columns that come more than once)
     }
     __syncthreads();
     bool left = s_left != 0;
@@ -187,28 +198,36 @@ __device__ __forceinline__ bool fused_dense_group(int row0, bool leads, int offs
             for (int n = 0; n < NT; ++n) acc[n] += (part[0][n] + part[1][n]) + (part[2][n] + part[3][n]);
         };
         clear();
-#pragma unroll 2
-        for (int t = 0; t < tiles; ++t) {
-            const f4 p = *reinterpret_cast<const f4*>(s_p + l * kStride + 16 * t + 4 * kq);
-            float v[4][NT];
+        constexpr int kAhead = 4;  // tiles of V on their way, and of a chain
+        float v[kAhead][4][NT];
+        auto load_v = [&](int t, int to) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const float* row = Vmat + (size_t)(c0 + min(16 * t + 4 * kq + j, span - 1)) * D + d;
                 if constexpr (NT == 2) {
                     typedef float f2 __attribute__((ext_vector_type(2), aligned(4)));
                     const f2 x = *reinterpret_cast<const f2*>(row);
-                    v[j][0] = x.x;
-                    v[j][1] = x.y;
-                } else v[j][0] = *row;
+                    v[to][j][0] = x.x;
+                    v[to][j][1] = x.y;
+                } else v[to][j][0] = *row;
             }
+        };
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
+        for (int t = 0; t < kAhead; ++t) load_v(t, t);
+        for (int t0 = 0; t0 < tiles; t0 += kAhead) {
 #pragma unroll
-                for (int n = 0; n < NT; ++n) part[j][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[j], v[j][n], part[j][n], 0, 0, 0);
-            if (t % kSumTiles == kSumTiles - 1) {
-                fold();
-                clear();
+            for (int i = 0; i < kAhead; ++i) {
+                const int t = t0 + i;
+                if (t >= tiles) break;
+                const f4 p = *reinterpret_cast<const f4*>(s_p + l * kStride + 16 * t + 4 * kq);
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                    for (int n = 0; n < NT; ++n) part[j][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[j], v[i][j][n], part[j][n], 0, 0, 0);
+                load_v(t + kAhead, i);
             }
+            fold();
+            clear();
         }
         fold();
         bool finite = true;
@@ -259,20 +278,29 @@ __device__ __forceinline__ void fused_block(int bid, int M, int D, int col_tiles
     const int ct = col_tiles == 1 ? 0 : bid / row_blocks;
     int rb = bid - ct * row_blocks;
     if constexpr (GROUPS) {
-        // Runs of 32 row blocks per XCD (workgroup 8 k + x runs on XCD x): the rows of Kmat and V that neighbouring groups
-        // share are then fetched into one L2. Which of a group's n workgroups leads changes with the group, so that the
-        // leaders lie on all compute units: an XCD's workgroups k go to its four shader engines, and there to the eight
-        // compute units, in turn (4096 rows, 64 columns per row, D = 64: 6.3 us; all leaders on a quarter of them: 9.8 us).
-        if (rb < (row_blocks & ~255)) rb = (rb & ~255) + ((rb & 7) << 5) + ((rb >> 3) & 31);
+        // The first workgroups of the launch lead a group each, and are on all compute units at once; whose row blocks those
+        // groups hold is another matter, so that rows that are not dense are gone through in their order. (Led by one of their
+        // own workgroups, some compute units got more groups than others and the last leaders started when the first had long
+        // ended: 16384 rows, 128 columns per row, D = 128: after 22 of 38 us.)
+        // Runs of 32 row blocks and of eight groups per XCD (workgroup 8 k + x runs on XCD x): the rows of Kmat and V that
+        // neighbours share are then fetched into one L2.
         constexpr int n = 16 / R;
-        const int group = rb / n, leader = n > 1 ? ((((rb >> 8) << 5) + (rb & 31)) / n / 8) % n : 0;
-        const int offsets = row_offsets[min(group * 16 + min((int)(threadIdx.x & 63), 16), M)], first = rb % n * R;
-        // (a first row that spans more than fused_dense_group takes settles it for all workgroups of the group, by two columns
-        // of the row that the row-by-row path reads next; the leader does not wait for them)
-        const int from = __builtin_amdgcn_readlane(offsets, first), to = __builtin_amdgcn_readlane(offsets, first + 1);
-        if ((rb % n == leader || to <= from || col_indices[to - 1] - col_indices[from] < kDenseSpan) &&
-            fused_dense_group<G1, DS, MASKED, G, V2>(group * 16, rb % n == leader, offsets, M, D, scale, (flags >> 1) & 3, col_indices,
-                                                    Q, Kmat, Vmat, O))
+        const int groups = M / 16, lane = threadIdx.x & 63;
+        int led = groups, own = rb;
+        if (rb < groups) led = rb < (groups & ~63) ? (rb & ~63) + ((rb & 7) << 3) + ((rb >> 3) & 7) : rb;
+        if (rb < (row_blocks & ~255)) own = (rb & ~255) + ((rb & 7) << 5) + ((rb >> 3) & 31);
+        rb = own;
+        const int of_led = row_offsets[min(led * 16 + min(lane, 16), M)], of_own = row_offsets[min(rb / n * 16 + min(lane, 16), M)];
+        // (a first row that spans more than fused_dense_group takes settles it, by two columns of the row; no workgroup waits for
+        // another)
+        auto may_be = [&](int offsets, int first) {
+            const int from = __builtin_amdgcn_readlane(offsets, first), to = __builtin_amdgcn_readlane(offsets, first + 1);
+            return to <= from || col_indices[to - 1] - col_indices[from] < kDenseSpan;
+        };
+        const bool led_may = led < groups && may_be(of_led, 0), own_may = may_be(of_own, rb % n * R);
+        if (led_may)
+            (void)fused_dense_group<true, G1, DS, MASKED, G, V2>(led * 16, of_led, M, D, scale, (flags >> 1) & 3, col_indices, Q, Kmat, Vmat, O);
+        if (own_may && fused_dense_group<false, G1, DS, MASKED, G, V2>(rb / n * 16, of_own, M, D, scale, (flags >> 1) & 3, col_indices, Q, Kmat, Vmat, O))
             return;
     }
     RowBlock<W, R, SLICED, PLANNED> blk;
@@ -305,7 +333,7 @@ __global__ __launch_bounds__(W * 64) void fused_kernel(int M, int D, int col_til
 // The same with groups of sixteen rows on the matrix cores where their columns form one run (fused_dense_group): a kernel of its
 // own, because what that needs -- 20 KB of LDS and more registers -- takes a wave per SIMD from calls that have no such groups.
 // Four waves per SIMD at least: left to itself the compiler keeps the chains in accumulation registers and ends at two or three
-// (16384 rows, 128 columns per row, D = 128: 40.5 us, D = 64: 26.7 us; with four 38.6 and 21.4 us).
+// (16384 rows, 128 columns per row, D = 128: 40.5 us, D = 64: 26.7 us; with four 38.6 and 21.4 us, as the kernel was then).
 template <int VEC, int G1, int DS, int MASKED, int G, int V2, int W, int R>
 __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(4))) void fused_groups_kernel(int M, int D, int flags, float scale, const int* __restrict__ row_offsets,
                                                               const int* __restrict__ col_indices, const float* __restrict__ Q,

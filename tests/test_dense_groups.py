@@ -152,3 +152,29 @@ def test_values_that_are_not_finite_or_tiny(where):
         assert np.abs(other).max() > 0 and np.linalg.norm(got - other) <= 1e-3 * np.linalg.norm(other)
     elif fine.any():
         assert np.linalg.norm(got[fine].astype(np.float64) - other[fine]) <= 1e-5 * np.linalg.norm(other[fine].astype(np.float64))
+
+
+@pytest.mark.parametrize("M,D", [(20000, 64), (16395, 112)])
+def test_groups_led_by_workgroups_of_other_rows(M, D):
+    """Runs of window rows between rows with scattered columns, rows longer than a group's columns (all of them twice) and rows without
+    any: who leads a group is not who owns its row blocks, and what a group is must come out the same for both."""
+    K, band = M, 200
+    ro, ci, rng = window(M, K, band, M)
+    rows = np.split(ci, ro[1:-1])
+    kind = rng.integers(0, 5, M // 48 + 1)
+    for r in range(M):
+        if kind[r // 48] == 1:
+            rows[r] = np.sort(rng.choice(K, rows[r].size, replace=False)).astype(np.int32)
+        elif kind[r // 48] == 2 and r % 16 == 5:
+            rows[r] = np.repeat(rows[r], 2)
+        elif kind[r // 48] == 3 and r % 7 == 0:
+            rows[r] = rows[r][:0]
+    ro = np.concatenate(([0], np.cumsum([r.size for r in rows]))).astype(np.int32)
+    ci = np.concatenate(rows)
+    Q, Km, V = (rng.normal(size=(n, D)).astype(np.float32) for n in (M, K, K))
+    got, other = run(ro, ci, Q, Km, V, 0.125)
+    assert oracle.rel_frobenius(got, oracle.fused(ro, ci, Q, Km, V, 0.125)) <= 1e-5  # (as in test_windows)
+    differ = (got != other).any(axis=1)[:M // 16 * 16].reshape(-1, 16)
+    whole = np.array([[kind[(g * 16 + i) // 48] for i in range(16)] for g in range(M // 16)])
+    assert differ[(whole == 0).all(axis=1)].any(axis=1).all()  # on the matrix cores
+    assert not differ[(whole == 1).all(axis=1)].any()          # row by row
