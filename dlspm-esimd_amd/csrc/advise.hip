@@ -268,7 +268,13 @@ int dlspm_advise(int op, int N_or_D, const dlspm_matrix_info* info, dlspm_call_p
         if (op != DLSPM_OP_SPMM && (double)longest * M >= 20.0 * (double)nnz) plan->hints |= DLSPM_HINT_ROWS_SKEWED;
         return DLSPM_OK;
     }
-    // 3. schedule memory (column slices, flat schedule), the even-rows hint, or nothing
+    // 3. even rows on dense tiles: memory for the parts of B
+    if (op == DLSPM_OP_SPMM && even && spmm_tiles_choose(dev, M, K, N_or_D, nnz, spmm_resident_choose(dev, M, K, N_or_D, nnz, true, false).us)) {
+        plan->bytes = spmm_tiles_bytes(K, N_or_D);
+        plan->hints = DLSPM_HINT_ROWS_EVEN;
+        return DLSPM_OK;
+    }
+    // 4. schedule memory (column slices, flat schedule), the even-rows hint, or nothing
     const int passing = dlspm_workspace_advice(op, M, K, N_or_D, nnz, longest);
     if (passing == DLSPM_PASS_WORKSPACE && op == DLSPM_OP_SPMM && spmm_resident_choose(dev, M, K, N_or_D, nnz, false, false).rr > 0) return DLSPM_OK;
     if (passing == DLSPM_PASS_WORKSPACE) plan->bytes = dlspm_workspace_bytes(op, M, K, N_or_D, nnz);

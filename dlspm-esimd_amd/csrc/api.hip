@@ -412,7 +412,7 @@ template <typename Shape> struct Call {
     int status = DLSPM_OK;  // DLSPM_E_WORKSPACE: the memory is too small for what the call was to run
     int schedule = DLSPM_SCHEDULE_ROW_BLOCKS;
     Shape shape{};
-    ResidentPlan resident{0, 0, 0};
+    ResidentPlan resident{0, 0, 0, 0.0};
     TilePlan tiles{0};  // SDDMM: ranges > 0: dense tiles on the matrix cores in place of the schedule
     CutPlan cut{};
     SlicePlan sliced{0, 1, 0, 0};
@@ -458,6 +458,9 @@ static SpmmCall spmm_decide(const DeviceInfo& dev, int M, int K, int N, int nnz,
         else if (c.flat.chunk > 0) c.schedule = DLSPM_SCHEDULE_FLAT;
     }
     if (c.resident.rr > 0) c.schedule = DLSPM_SCHEDULE_RESIDENT;
+    // (memory that comes with the even-rows hint has this one use)
+    if (ws.rows_even && !ws.banded && ws.mem && ws.bytes >= spmm_tiles_bytes(K, N) && spmm_tiles_choose(dev, M, K, N, nnz, c.resident.us))
+        c.schedule = DLSPM_SCHEDULE_DENSE_TILES;
     return c;
 }
 
@@ -622,6 +625,7 @@ int spmm_csr_f32(int M, int K, int N, int nnz, const int* row_offsets, const int
     hipError_t e;
     switch (c.schedule) {
         case DLSPM_SCHEDULE_RESIDENT: e = spmm_resident_launch(args, c.resident, st); break;
+        case DLSPM_SCHEDULE_DENSE_TILES: e = spmm_tiles_launch(args, ws.mem, st); break;
         case DLSPM_SCHEDULE_CUT_PLAN: e = spmm_pieces_launch(args, c.shape, c.cut, ws.mem, st); break;
         case DLSPM_SCHEDULE_ROW_PLAN: e = spmm_planned_launch(args, c.shape, static_cast<const int*>(ws.mem), st); break;
         case DLSPM_SCHEDULE_SLICED: e = spmm_sliced_launch(args, c.shape, c.sliced, ws.mem, st); break;
@@ -1035,6 +1039,7 @@ int dlspm_describe_schedule(int op, int M, int K, int N_or_D, int nnz, size_t wo
             schedule[2] = c.resident.slice;
             schedule[3] = c.resident.chunks;
         }
+        if (c.schedule == DLSPM_SCHEDULE_DENSE_TILES) spmm_tile_shape(&schedule[1], &schedule[2]);
     } else if (op == DLSPM_OP_SDDMM) {
         const SddmmCall c = sddmm_decide(dev, M, K, N_or_D, nnz, ws);
         status = c.status;

@@ -20,16 +20,17 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 struct Parts { bf16x8 hi, mid, lo; };
 
 // the eight floats x[0 ... 7] of a lane. Two at a time: the conversion makes two, and what it rounds them to are the halves of its
-// result (seven instructions a float with the look for values too small)
-__device__ __forceinline__ Parts split_parts(const float* x)
+// result (seven instructions a float with the look for values too small). The least of 2 |x| - 1 as an integer (x == 0: the largest)
+// goes to `least`.
+constexpr unsigned kTooSmall = (18u << 24) - 1;  // `least` below this: a nonzero value below 2^-109
+__device__ __forceinline__ Parts split_parts(const float* x, unsigned& least)
 {
     typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
     typedef float f32x2 __attribute__((ext_vector_type(2)));
     typedef unsigned u4 __attribute__((ext_vector_type(4)));
-    constexpr unsigned kTiny = (18u << 24) - 1;  // 2 |x| as an integer, minus one: x == 0 becomes the largest
     auto round2 = [](float a, float b) { return __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{a, b}, bf16x2)); };
     u4 hi, mid, lo;
-    unsigned least = ~0u;
+    least = ~0u;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const float a = x[2 * i], b = x[2 * i + 1];
@@ -39,8 +40,18 @@ __device__ __forceinline__ Parts split_parts(const float* x)
         lo[i] = round2(ra - __uint_as_float(mid[i] << 16), rb - __uint_as_float(mid[i] & 0xffff0000u));
         least = min(min(least, (__float_as_uint(a) << 1) - 1u), (__float_as_uint(b) << 1) - 1u);
     }
-    hi[0] = least < kTiny ? 0x7fc07fc0u : hi[0];
     return Parts{__builtin_bit_cast(bf16x8, hi), __builtin_bit_cast(bf16x8, mid), __builtin_bit_cast(bf16x8, lo)};
+}
+// ... with NaN in the place of a part where a value is too small
+__device__ __forceinline__ Parts split_parts(const float* x)
+{
+    typedef unsigned u4 __attribute__((ext_vector_type(4)));
+    unsigned least;
+    Parts p = split_parts(x, least);
+    u4 hi = __builtin_bit_cast(u4, p.hi);
+    hi[0] = least < kTooSmall ? 0x7fc07fc0u : hi[0];
+    p.hi = __builtin_bit_cast(bf16x8, hi);
+    return p;
 }
 
 // 32 x 32 results, sixteen products each: lane l holds row l % 32 of `a` and of `b`, elements 8 (l / 32) ... + 7; element r of the

@@ -220,11 +220,21 @@ hipError_t spmm_sliced_launch(const SpmmArgs& x, const SpmmShape& s, const Slice
 
 // Resident schedule of SpMM (resident.hip): workgroups of sixteen waves own 64 x rr rows and 64 columns and go through slices of
 // `slice` rows of B that lie in LDS, with `chunks` x 64 (column, value) pairs of every row loaded ahead. rr == 0: not used.
-struct ResidentPlan { int rr, chunks, slice; };
+struct ResidentPlan {
+    int rr, chunks, slice;
+    double us;  // estimated time: of this schedule, or (rr == 0) of the row-block kernels where the estimate was made, else 0
+};
 // uneven: the caller knows (a plan that comes with the call, DLSPM_HINT_ROWS_SKEWED)
 ResidentPlan spmm_resident_choose(const DeviceInfo& dev, int M, int K, int N, int nnz, bool rows_even, bool uneven);
 int resident_rows_per_workgroup(const ResidentPlan& plan);
 hipError_t spmm_resident_launch(const SpmmArgs& x, const ResidentPlan& plan, hipStream_t stream);
+
+// Dense tiles of SpMM (spmm_tiles.hip): A scattered into dense tiles, multiplied on the matrix cores with the parts of B, which lie in
+// spmm_tiles_bytes of the caller's memory. For calls with memory and the even-rows hint
+bool spmm_tiles_choose(const DeviceInfo& dev, int M, int K, int N, int nnz, double other_us);
+size_t spmm_tiles_bytes(int K, int N);
+void spmm_tile_shape(int* rows, int* columns);
+hipError_t spmm_tiles_launch(const SpmmArgs& x, void* memory, hipStream_t stream);
 
 SddmmShape sddmm_choose(const DeviceInfo& dev, int M, int D, int nnz, bool vec4, int rows = kRowsUnknown);
 void sddmm_few_rows_pieces(const DeviceInfo& dev, SddmmShape& s, int M, int nnz);  // a call without plan or memory: sets s.pieces_lg (and W = 4)

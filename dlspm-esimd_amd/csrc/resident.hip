@@ -402,7 +402,7 @@ template <int RR, int QC, int CHAINS> static hipError_t launch_one(const SpmmArg
 ResidentPlan spmm_resident_choose(const DeviceInfo& dev, int M, int K, int N, int nnz, bool rows_even, bool uneven_rows)
 {
     const Tuning& t = tuning();
-    const ResidentPlan none{0, 0, 0};
+    ResidentPlan none{0, 0, 0, 0.0};
     if (!rule_on(kRuleResidentSlices) || N < 4 || M <= 0 || K <= 0 || nnz <= 0 || nnz >= (1 << 29) || !dense_fits_buffer(K, N)) return none;
     // (a schedule that was asked for by name)
     if (t.split_w > 0 || t.flat >= 0 || t.slices >= 0 || t.tile_major >= 0 || t.tile_width > 0 || t.plan_order > 0 || t.xcd_contiguous) return none;
@@ -415,6 +415,7 @@ ResidentPlan spmm_resident_choose(const DeviceInfo& dev, int M, int K, int N, in
     // what a dense row costs the row-block kernels: half of the lanes that its layout leaves idle count
     const double width = N <= 32 ? 32 : N <= 64 ? 64 : N <= 128 ? 0.5 * (N + 128) : N <= 256 ? 0.5 * (N + 256) : N;
     const double row_block_us = 2.0 + (double)nnz * width * 1.55e-7;
+    none.us = row_block_us;
     ResidentPlan best = none;
     double best_us = 0.9 * row_block_us;
     for (int rr = 1; rr <= (chunks == 1 ? 4 : 3); ++rr) {
@@ -426,7 +427,7 @@ ResidentPlan spmm_resident_choose(const DeviceInfo& dev, int M, int K, int N, in
         else if (!rows_even) us *= std::max(1.0, uneven / (M <= 16 * dev.cus ? 1.5 : 1.15));
         if (us < best_us) {
             best_us = us;
-            best = ResidentPlan{rr, chunks, slice};
+            best = ResidentPlan{rr, chunks, slice, us};
         }
     }
     return best;

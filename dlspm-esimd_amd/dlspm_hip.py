@@ -29,6 +29,7 @@ HINT_ROW_PLAN = 1 << 61
 HINT_BANDED = 1 << 60
 HINT_CUT_PLAN = 1 << 59
 HINT_ROWS_SKEWED = 1 << 58
+HINT_MASK = 0xFF << 56
 
 
 class _RowsEven:
@@ -327,7 +328,8 @@ def advise(op, width, info: MatrixInfo) -> CallPlan:
 
 
 class Prepared:
-    """What dlspm_advise said for one matrix, op and width, allocated and built (prepare()): pass as prepared=... ."""
+    """What dlspm_advise said for one matrix, op and width, allocated and built (prepare()): pass as plan=... . A size without
+    memory is that of memory which each call takes from PyTorch's allocator (SpMM on dense tiles: B's parts)."""
 
     def __init__(self, memory, size_and_hints, call_plan):
         self.memory, self.size_and_hints, self.call_plan = memory, size_and_hints, call_plan
@@ -340,6 +342,8 @@ def prepare(row_offsets, col_indices, K, op, width, info=None) -> Prepared:
     info = info if info is not None else analyze(row_offsets, col_indices, K)
     cp = advise(op, width, info)
     M = row_offsets.numel() - 1
+    if op == OP_SPMM and cp.build == BUILD_NOTHING and cp.hints & HINT_ROWS_EVEN:
+        return Prepared(None, cp.bytes | cp.hints, cp)
     mem = torch.empty(((cp.bytes + 3) // 4,), dtype=torch.int32, device=row_offsets.device) if cp.bytes else None
     if cp.build == BUILD_ROW_PLAN:
         st = lib().dlspm_row_plan_build(M, _ptr(row_offsets, torch.int32, "row_offsets", M + 1), ctypes.c_void_p(mem.data_ptr()),
@@ -407,6 +411,25 @@ def _csr_sizes(row_offsets, col_indices):
     return row_offsets.numel() - 1, col_indices.numel()
 
 
+class _Owner(ctypes.c_void_p):
+    """A pointer that keeps the tensor it points to."""
+
+
+def _own_memory(size):
+    """(pointer, size) of memory for one call on the current stream, or (None, 0): with size 0, or where there is no room."""
+    import torch
+
+    if size == 0:
+        return None, 0
+    try:
+        memory = torch.empty((size,), dtype=torch.uint8, device="cuda")
+    except torch.OutOfMemoryError:
+        return None, 0
+    pointer = _Owner(memory.data_ptr())
+    pointer.memory = memory
+    return pointer, size
+
+
 def _workspace_args(workspace, plan, M, banded=False):
     """(pointer, size with hint bits) for the pair (workspace, workspace_bytes) of the three compute entry points.
     banded: the caller knows that every row's columns lie in a narrow window that moves with the row (DLSPM_HINT_BANDED)."""
@@ -416,7 +439,10 @@ def _workspace_args(workspace, plan, M, banded=False):
     if isinstance(plan, Prepared):
         if workspace is not None:
             raise ValueError("pass what prepare() returned or a workspace, not both")
-        return (ctypes.c_void_p(plan.memory.data_ptr()) if plan.memory is not None else None), plan.size_and_hints | hint
+        if plan.memory is not None:
+            return ctypes.c_void_p(plan.memory.data_ptr()), plan.size_and_hints | hint
+        pointer, size = _own_memory(plan.size_and_hints & ~HINT_MASK)
+        return pointer, plan.size_and_hints & HINT_MASK | size | hint
     if isinstance(plan, CutPlan):
         if workspace is not None:
             raise ValueError("pass a row plan or a workspace, not both")
@@ -541,18 +567,18 @@ def describe_launch(op: int, M: int, K: int, N: int, nnz: int, rows_even: bool =
                     (int(x) for x in out)))
 
 
-SCHEDULES = ("row_blocks", "flat", "sliced", "row_plan", "cut_plan", "resident", "dense_groups")
+SCHEDULES = ("row_blocks", "flat", "sliced", "row_plan", "cut_plan", "resident", "dense_groups", "dense_tiles")
 
 
 def describe_schedule(op: int, M: int, K: int, N: int, nnz: int, plan=None, workspace_bytes: int = 0) -> dict:
     """The schedule that a call runs (dlspm_describe_schedule): {'schedule' (one of SCHEDULES), 'rows' per workgroup, 'slice_rows',
-    'chunks'}; SDDMM on dense tiles also {'tile_columns'}, with 'rows' those of a tile and 'schedule' the one without tiles. plan: what
+    'chunks'}; on dense tiles also {'tile_columns'}, with 'rows' those of a tile (SDDMM: 'schedule' is the one without tiles). plan: what
     prepare() returned; or workspace_bytes: the size, with hint bits, that the call passes."""
     out = (ctypes.c_int * 4)()
     st = lib().dlspm_describe_schedule(op, M, K, N, nnz, plan.size_and_hints if plan is not None else workspace_bytes, out)
     if st != OK:
         raise DlspmError(st, "dlspm_describe_schedule")
-    if op == OP_SDDMM and out[2] > 0:
+    if out[2] > 0 and (op == OP_SDDMM or SCHEDULES[out[0]] == "dense_tiles"):
         return {"schedule": SCHEDULES[out[0]], "rows": out[1], "slice_rows": 0, "chunks": 0, "tile_columns": out[2]}
     return {"schedule": SCHEDULES[out[0]], "rows": out[1], "slice_rows": out[2], "chunks": out[3]}
 

@@ -63,6 +63,7 @@ struct Call {
     const int *row_offsets = nullptr, *col_indices = nullptr;
     void* memory = nullptr;
     size_t size_and_hints = 0;
+    at::Tensor scratch;  // memory of this call alone
     PyObject* result = nullptr;  // a new reference
     float* out = nullptr;
 
@@ -97,6 +98,19 @@ struct Call {
         Py_XDECREF(mem);
         Py_XDECREF(size);
         return good;
+    }
+    // What prepare() left to be allocated by each call: from PyTorch's allocator, so that calls on several streams do not share it.
+    // Without it, where there is no room, the call runs as with the hints alone.
+    void own_memory(const at::Tensor& like)
+    {
+        const size_t bytes = size_and_hints & ~DLSPM_HINT_MASK;
+        if (memory || bytes == 0) return;
+        try {
+            scratch = at::detail::empty_cuda({(int64_t)bytes}, at::kByte, like.device(), std::nullopt);
+            memory = scratch.data_ptr();
+        } catch (const c10::OutOfMemoryError&) {
+            size_and_hints &= DLSPM_HINT_MASK;
+        }
     }
     // `given`, or a new tensor on `like`'s device
     bool output(PyObject* given, at::IntArrayRef sizes, const at::Tensor& like)
@@ -171,6 +185,7 @@ PyObject* call_spmm(PyObject*, PyObject* const* args, Py_ssize_t npos, PyObject*
             PyErr_Clear();
             return fallback(DLSPM_OP_SPMM, args, npos, kwnames);
         }
+        c.own_memory(*B);
         const int K = (int)K_given, N = (int)B->size(1);
         const float *v = static_cast<const float*>(address(*values)), *b = static_cast<const float*>(address(*B));
         return c.run("spmm_csr_f32", [&](void* stream) {

@@ -44,7 +44,10 @@
  *         costs time, never correctness (a row's products are added in a different, equally fixed order).
  *       Matrices dense enough that each row of B serves many rows of a workgroup (from a density of about 0.05 on under the
  *         even-rows hint, about 0.15 otherwise) are multiplied from slices of B in LDS where that is estimated to be faster;
- *         memory or a plan that comes with such a call is not used.
+ *         memory or a plan that comes with such a call is not used. Large ones under the even-rows hint are multiplied as dense
+ *         tiles on the matrix cores where that is estimated to be faster still and the call has memory for it, which then
+ *         holds B split into parts: dlspm_advise names the size (6.02 bytes per float of B, its rows rounded up to 128 and
+ *         its columns to 32); less memory, or none, is as good as the hint alone.
  *       DLSPM_HINT_ROW_PLAN: `workspace` holds the row plan of this matrix (dlspm_row_plan_build, below; at least
  *         dlspm_row_plan_bytes(M) bytes, else DLSPM_E_WORKSPACE) and the launch hands the rows out in the plan's order.
  *         The plan is only read.
@@ -354,9 +357,10 @@ int dlspm_describe_launch_rows(int op, int M, int K, int N_or_D, int nnz, int pa
  * The schedule that a call would run, for these sizes and the `workspace_bytes` that is passed with it (size and hint bits; a
  * size other than 0 stands for memory of that size). The compute entry points decide by the same function. schedule[4]
  * receives: [0] DLSPM_SCHEDULE_*, [1] rows per workgroup (0: flat schedule), and, where [0] is DLSPM_SCHEDULE_RESIDENT, [2] rows
- * of B per slice and [3] chunks of 64 nonzeros of a row that are loaded ahead (else 0). SDDMM on dense tiles (masks dense enough:
- * the matrix cores compute whole tiles and the sampled results are picked from them): [1] rows and [2] columns of a tile, [0] the
- * schedule that the call would run without DLSPM_RULE_DENSE_GROUPS. The shapes that
+ * of B per slice and [3] chunks of 64 nonzeros of a row that are loaded ahead (else 0). DLSPM_SCHEDULE_DENSE_TILES: [1] rows and [2]
+ * columns of C per workgroup. SDDMM on dense tiles (masks dense enough: the matrix cores compute whole tiles and the sampled results
+ * are picked from them): [1] rows and [2] columns of a tile, [0] the schedule that the call would run without
+ * DLSPM_RULE_DENSE_GROUPS. The shapes that
  * dlspm_describe_launch_rows gives are those of DLSPM_SCHEDULE_ROW_BLOCKS and _FLAT (and, as far as the fields go, of
  * _DENSE_GROUPS for the rows that are not in groups). Host-only. DLSPM_OK, DLSPM_E_WORKSPACE where the call would be
  * refused for its size, or DLSPM_E_INVALID_ARG.
@@ -368,6 +372,7 @@ int dlspm_describe_launch_rows(int op, int M, int K, int N_or_D, int nnz, int pa
 #define DLSPM_SCHEDULE_CUT_PLAN     4  /* ... of a cut plan                                                                 */
 #define DLSPM_SCHEDULE_RESIDENT     5  /* SpMM: slices of B in LDS                                                          */
 #define DLSPM_SCHEDULE_DENSE_GROUPS 6  /* fused: row blocks, sixteen rows whose columns form one run on the matrix cores    */
+#define DLSPM_SCHEDULE_DENSE_TILES  7  /* SpMM, even rows and memory: dense tiles on the matrix cores                       */
 int dlspm_describe_schedule(int op, int M, int K, int N_or_D, int nnz, size_t workspace_bytes, int* schedule);
 
 /*
@@ -435,7 +440,7 @@ typedef struct dlspm_tuning {
                                                    /* the fused op's first stage likewise at D = 260 ... 380                      */
 #define DLSPM_RULE_RESIDENT_SLICES           2048  /* SpMM on dense enough matrices: slices of B in LDS, whatever memory the call has  */
 #define DLSPM_RULE_DENSE_GROUPS              4096  /* fused op, D = 36 ... 128, large calls: sixteen rows whose columns form one run on the  */
-                                                   /* matrix cores                                                            */
+                                                   /* matrix cores; SDDMM (D = 17 ... 128) and SpMM with memory: dense tiles  */
 void dlspm_tuning_default(dlspm_tuning* t);   /* fills *t with "follow the rules" */
 int dlspm_set_tuning(const dlspm_tuning* t);  /* DLSPM_OK or DLSPM_E_INVALID_ARG (a field out of range) */
 int dlspm_get_tuning(dlspm_tuning* t);        /* what the calling thread's launches currently use */

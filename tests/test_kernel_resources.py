@@ -52,3 +52,9 @@ def test_lds_of_the_dense_groups_is_in_their_kernels_only(kernels):
     assert len(plain) > 100 and max(v["lds"] for v in plain.values()) <= 33000
     four_waves = {k: v for k, v in plain.items() if re.search(r"Li8ELi[234]ELi[01]ELi(16|32)ELi1ELi4ELi\d+EE", k)}
     assert len(four_waves) == 30 and max(v["lds"] for v in four_waves.values()) <= 4096, four_waves
+
+
+def test_dense_tiles_spill_nothing(kernels):
+    used = {k: v for k, v in kernels.items() if re.match(r"_ZN5dlspm\d+(spmm|sddmm)_tiles_kernel", k)}
+    assert len(used) == 17
+    assert all(v["scratch"] == 0 and v["vgpr_spills"] == 0 for v in used.values()), used
