@@ -247,7 +247,16 @@ int dlspm_advise(int op, int N_or_D, const dlspm_matrix_info* info, dlspm_call_p
         plan->hints = DLSPM_HINT_BANDED | (even ? DLSPM_HINT_ROWS_EVEN : 0);
         return DLSPM_OK;
     }
-    // 2. uneven rows: a row plan, with the longest rows cut where that pays; where the call is multiplied from slices of B in LDS all
+    // 2. the fused op on dense masks: memory for the scores between its two steps (never less than what the call would refuse)
+    if (op == DLSPM_OP_FUSED) {
+        const size_t bytes = fused_two_steps_bytes(dev, M, K, N_or_D, nnz, even);
+        if (bytes > 0) {
+            plan->bytes = std::max(bytes, dlspm_workspace_bytes(op, M, K, N_or_D, nnz));
+            plan->hints = even ? DLSPM_HINT_ROWS_EVEN : 0;
+            return DLSPM_OK;
+        }
+    }
+    // 3. uneven rows: a row plan, with the longest rows cut where that pays; where the call is multiplied from slices of B in LDS all
     // the same, the word that the rows are uneven, which those slices count with, and no memory
     const int planned = dlspm_row_plan_advice(op, M, K, N_or_D, nnz, longest);
     if (planned >= 1 && op == DLSPM_OP_SPMM && spmm_resident_choose(dev, M, K, N_or_D, nnz, false, true).rr > 0) {
@@ -268,13 +277,13 @@ int dlspm_advise(int op, int N_or_D, const dlspm_matrix_info* info, dlspm_call_p
         if (op != DLSPM_OP_SPMM && (double)longest * M >= 20.0 * (double)nnz) plan->hints |= DLSPM_HINT_ROWS_SKEWED;
         return DLSPM_OK;
     }
-    // 3. even rows on dense tiles: memory for the parts of B
+    // 4. even rows on dense tiles: memory for the parts of B
     if (op == DLSPM_OP_SPMM && even && spmm_tiles_choose(dev, M, K, N_or_D, nnz, spmm_resident_choose(dev, M, K, N_or_D, nnz, true, false).us)) {
         plan->bytes = spmm_tiles_bytes(K, N_or_D);
         plan->hints = DLSPM_HINT_ROWS_EVEN;
         return DLSPM_OK;
     }
-    // 4. schedule memory (column slices, flat schedule), the even-rows hint, or nothing
+    // 5. schedule memory (column slices, flat schedule), the even-rows hint, or nothing
     const int passing = dlspm_workspace_advice(op, M, K, N_or_D, nnz, longest);
     if (passing == DLSPM_PASS_WORKSPACE && op == DLSPM_OP_SPMM && spmm_resident_choose(dev, M, K, N_or_D, nnz, false, false).rr > 0) return DLSPM_OK;
     if (passing == DLSPM_PASS_WORKSPACE) plan->bytes = dlspm_workspace_bytes(op, M, K, N_or_D, nnz);

@@ -413,14 +413,16 @@ template <typename Shape> struct Call {
     int schedule = DLSPM_SCHEDULE_ROW_BLOCKS;
     Shape shape{};
     ResidentPlan resident{0, 0, 0, 0.0};
-    TilePlan tiles{0};  // SDDMM: ranges > 0: dense tiles on the matrix cores in place of the schedule
+    TilePlan tiles{0, 0.0};  // SDDMM: ranges > 0: dense tiles on the matrix cores in place of the schedule
     CutPlan cut{};
     SlicePlan sliced{0, 1, 0, 0};
     FlatPlan flat{0, 0, 0};
 };
 using SpmmCall = Call<SpmmShape>;
 using SddmmCall = Call<SddmmShape>;
-using FusedCall = Call<FusedShape>;
+struct FusedCall : Call<FusedShape> {
+    SpmmCall second;  // DLSPM_SCHEDULE_TWO_STEPS: the SpMM that follows the SDDMM on `tiles`
+};
 
 static int told_rows(const WorkspaceArg& ws) { return ws.rows_even ? kRowsEven : ws.skewed ? kRowsSkewed : kRowsUnknown; }
 
@@ -462,6 +464,19 @@ static SpmmCall spmm_decide(const DeviceInfo& dev, int M, int K, int N, int nnz,
     if (ws.rows_even && !ws.banded && ws.mem && ws.bytes >= spmm_tiles_bytes(K, N) && spmm_tiles_choose(dev, M, K, N, nnz, c.resident.us))
         c.schedule = DLSPM_SCHEDULE_DENSE_TILES;
     return c;
+}
+
+static hipError_t spmm_run(const SpmmArgs& args, const SpmmCall& c, void* mem, hipStream_t st)
+{
+    switch (c.schedule) {
+        case DLSPM_SCHEDULE_RESIDENT: return spmm_resident_launch(args, c.resident, st);
+        case DLSPM_SCHEDULE_DENSE_TILES: return spmm_tiles_launch(args, mem, st);
+        case DLSPM_SCHEDULE_CUT_PLAN: return spmm_pieces_launch(args, c.shape, c.cut, mem, st);
+        case DLSPM_SCHEDULE_ROW_PLAN: return spmm_planned_launch(args, c.shape, static_cast<const int*>(mem), st);
+        case DLSPM_SCHEDULE_SLICED: return spmm_sliced_launch(args, c.shape, c.sliced, mem, st);
+        case DLSPM_SCHEDULE_FLAT: return spmm_flat_launch(args, c.shape, c.flat, static_cast<float*>(mem), st);
+    }
+    return spmm_launch(args, c.shape, st);
 }
 
 static SddmmCall sddmm_decide(const DeviceInfo& dev, int M, int K, int D, int nnz, const WorkspaceArg& ws)
@@ -513,6 +528,49 @@ static SddmmCall sddmm_decide(const DeviceInfo& dev, int M, int K, int D, int nn
     return c;
 }
 
+// The fused op as SDDMM on dense tiles and then SpMM, the scores in the caller's memory in between: where the masks are dense enough that
+// the scores of whole tiles cost less than the gathered ones, and both steps together take less than 0.95 of the fused kernels' time.
+// Estimates (us): those of the two steps, 2 for the second launch, and 2 + nnz x 0.0100 / 0.0162 / 0.0343 x 1e-3 for the fused kernels at
+// D <= 32 / 64 / 128 (8192 x 8192, D = 128 at 0.1 / 0.2 / 0.3 232 / 442 / 688, D = 32 at 0.3 200; 16384 x 4096, D = 64 at 0.2 218;
+// 24576 x 8192, D = 80 at 0.1 623). A second step of row blocks takes more than its estimate on uneven rows (4000 x 4090, D = 77 at 0.2,
+// lognormal: fused 96, two steps 118) and below D = 64 (8192 x 8192, D = 32 at 0.3 145, estimate 105). Measured, fused -> two steps: 8192 x 8192, D = 128 at 0.1 / 0.2 / 0.3 230 / 437 / 683 -> 206 / 261 / 325, with
+// lognormal rows at 0.3 747 -> 392; 16384 x 8192, D = 128 at 0.3 1357 -> 451; 16384 x 4096, D = 64 at 0.2 217 -> 144; 4096 x 4096, D = 128 at
+// 0.3 165 -> 140; 12288 x 2048, D = 128 at 0.3 235 -> 112; 32768 x 8192, D = 32 at 0.3 890 -> 622.
+static size_t scores_bytes(int nnz) { return ((size_t)nnz * sizeof(float) + 255) / 256 * 256; }
+static WorkspaceArg behind_scores(const WorkspaceArg& ws, int nnz)
+{
+    WorkspaceArg rest{};
+    rest.rows_even = ws.rows_even;
+    rest.skewed = !ws.rows_even;  // (nobody said that they are even: memory is passed for uneven rows above all)
+    if (ws.rows_even && ws.bytes > scores_bytes(nnz)) {
+        rest.mem = static_cast<char*>(ws.mem) + scores_bytes(nnz);
+        rest.bytes = ws.bytes - scores_bytes(nnz);
+    }
+    return rest;
+}
+static bool fused_two_steps(const DeviceInfo& dev, int M, int K, int D, int nnz, const WorkspaceArg& ws, FusedCall& c)
+{
+    if (!ws.mem || ws.bytes < scores_bytes(nnz)) return false;
+    c.tiles = sddmm_tiles_choose(dev, M, K, D, nnz);
+    if (c.tiles.ranges == 0) return false;
+    c.second = spmm_decide(dev, M, K, D, nnz, behind_scores(ws, nnz));
+    const double second_us = c.second.schedule == DLSPM_SCHEDULE_DENSE_TILES ? spmm_tiles_us(dev, M, K, D, nnz) : c.second.resident.us;
+    if (c.second.schedule == DLSPM_SCHEDULE_ROW_BLOCKS && (!ws.rows_even || D < 64)) return false;
+    const double fused_us = 2.0 + (double)nnz * (D <= 32 ? 1.00e-5 : D <= 64 ? 1.62e-5 : 3.43e-5);
+    return c.second.resident.us > 0.0 && c.tiles.us + second_us + 2.0 < 0.95 * fused_us;  // (no estimate: a schedule was asked for by name)
+}
+size_t fused_two_steps_bytes(const DeviceInfo& dev, int M, int K, int D, int nnz, bool rows_even)
+{
+    static char some_memory;  // (never looked at)
+    WorkspaceArg ws{};
+    ws.rows_even = rows_even;
+    ws.mem = &some_memory;
+    ws.bytes = (size_t)1 << 48;
+    FusedCall c;
+    if (!fused_two_steps(dev, M, K, D, nnz, ws, c)) return 0;
+    return scores_bytes(nnz) + (c.second.schedule == DLSPM_SCHEDULE_DENSE_TILES ? spmm_tiles_bytes(K, D) : 0);
+}
+
 static FusedCall fused_decide(const DeviceInfo& dev, int M, int K, int D, int nnz, const WorkspaceArg& ws)
 {
     FusedCall c;
@@ -537,6 +595,10 @@ static FusedCall fused_decide(const DeviceInfo& dev, int M, int K, int D, int nn
             if (c.sliced.slices > 0) c.schedule = DLSPM_SCHEDULE_SLICED;
             else if (c.flat.chunk > 0) c.schedule = DLSPM_SCHEDULE_FLAT;
         }
+    }
+    if (!ws.cut_plan && !ws.row_plan && !ws.banded && c.status == DLSPM_OK && fused_two_steps(dev, M, K, D, nnz, ws, c)) {
+        c.schedule = DLSPM_SCHEDULE_TWO_STEPS;
+        return c;
     }
     if (c.schedule == DLSPM_SCHEDULE_ROW_BLOCKS && fused_looks_for_groups(c.shape, M, K, D, nnz)) c.schedule = DLSPM_SCHEDULE_DENSE_GROUPS;
     return c;
@@ -621,17 +683,7 @@ int spmm_csr_f32(int M, int K, int N, int nnz, const int* row_offsets, const int
     const SpmmCall c = spmm_decide(dev, M, K, N, nnz, ws);
     if (c.status != DLSPM_OK) return c.status;
     const SpmmArgs args{M, K, N, nnz, row_offsets, col_indices, values, B, C, ws.banded ? 1 : 0};
-    hipStream_t st = static_cast<hipStream_t>(stream);
-    hipError_t e;
-    switch (c.schedule) {
-        case DLSPM_SCHEDULE_RESIDENT: e = spmm_resident_launch(args, c.resident, st); break;
-        case DLSPM_SCHEDULE_DENSE_TILES: e = spmm_tiles_launch(args, ws.mem, st); break;
-        case DLSPM_SCHEDULE_CUT_PLAN: e = spmm_pieces_launch(args, c.shape, c.cut, ws.mem, st); break;
-        case DLSPM_SCHEDULE_ROW_PLAN: e = spmm_planned_launch(args, c.shape, static_cast<const int*>(ws.mem), st); break;
-        case DLSPM_SCHEDULE_SLICED: e = spmm_sliced_launch(args, c.shape, c.sliced, ws.mem, st); break;
-        case DLSPM_SCHEDULE_FLAT: e = spmm_flat_launch(args, c.shape, c.flat, static_cast<float*>(ws.mem), st); break;
-        default: e = spmm_launch(args, c.shape, st);
-    }
+    const hipError_t e = spmm_run(args, c, ws.mem, static_cast<hipStream_t>(stream));
     return e == hipSuccess ? DLSPM_OK : fail_hip(e);
 }
 
@@ -858,7 +910,7 @@ int sddmm_csr_f32(int M, int K, int D, int nnz, const int* row_offsets, const in
     if (c.status != DLSPM_OK) return c.status;
     const SddmmArgs args{M, K, D, nnz, row_offsets, col_indices, lhs, rhs, out_values, ws.banded ? 1 : 0, dev.l2_bytes, dev.cus};
     hipError_t e;
-    if (c.tiles.ranges > 0) e = sddmm_tiles_launch(args, c.tiles, st);
+    if (c.tiles.ranges > 0) e = sddmm_tiles_launch(args, 1.0f, c.tiles, st);
     else switch (c.schedule) {
         case DLSPM_SCHEDULE_CUT_PLAN: e = sddmm_pieces_launch(args, c.shape, c.cut, ws.mem, st); break;
         case DLSPM_SCHEDULE_ROW_PLAN: e = sddmm_planned_launch(args, c.shape, static_cast<const int*>(ws.mem), st); break;
@@ -889,6 +941,12 @@ int fused_sddmm_spmm_f32(int M, int K, int D, int nnz, const int* row_offsets, c
     const FusedArgs args{M, K, D, nnz, row_offsets, col_indices, Q, Kmat, V, scale, O, ws.banded ? 1 : 0};
     hipError_t e;
     switch (c.schedule) {
+        case DLSPM_SCHEDULE_TWO_STEPS: {
+            float* const scores = static_cast<float*>(ws.mem);
+            e = sddmm_tiles_launch(SddmmArgs{M, K, D, nnz, row_offsets, col_indices, Q, Kmat, scores, 0, dev.l2_bytes, dev.cus}, scale, c.tiles, st);
+            if (e == hipSuccess) e = spmm_run(SpmmArgs{M, K, D, nnz, row_offsets, col_indices, scores, V, O, 0}, c.second, behind_scores(ws, nnz).mem, st);
+            break;
+        }
         case DLSPM_SCHEDULE_CUT_PLAN: e = fused_pieces_launch(args, c.shape, c.cut, ws.mem, st); break;
         case DLSPM_SCHEDULE_ROW_PLAN: e = fused_planned_launch(args, c.shape, static_cast<const int*>(ws.mem), st); break;
         case DLSPM_SCHEDULE_SLICED: e = fused_sliced_launch(args, c.shape, c.sliced, ws.mem, st); break;
@@ -1054,6 +1112,10 @@ int dlspm_describe_schedule(int op, int M, int K, int N_or_D, int nnz, size_t wo
         status = c.status;
         schedule[0] = c.schedule;
         schedule[1] = c.schedule == DLSPM_SCHEDULE_SLICED ? c.sliced.R : c.shape.R;
+        if (c.schedule == DLSPM_SCHEDULE_TWO_STEPS) {
+            sddmm_tile_shape(&schedule[1], &schedule[2]);
+            schedule[3] = c.second.schedule;
+        }
     } else {
         return DLSPM_E_INVALID_ARG;
     }

@@ -231,6 +231,7 @@ hipError_t spmm_resident_launch(const SpmmArgs& x, const ResidentPlan& plan, hip
 
 // Dense tiles of SpMM (spmm_tiles.hip): A scattered into dense tiles, multiplied on the matrix cores with the parts of B, which lie in
 // spmm_tiles_bytes of the caller's memory. For calls with memory and the even-rows hint
+double spmm_tiles_us(const DeviceInfo& dev, int M, int K, int N, int nnz);  // estimated time
 bool spmm_tiles_choose(const DeviceInfo& dev, int M, int K, int N, int nnz, double other_us);
 size_t spmm_tiles_bytes(int K, int N);
 void spmm_tile_shape(int* rows, int* columns);
@@ -240,16 +241,21 @@ SddmmShape sddmm_choose(const DeviceInfo& dev, int M, int D, int nnz, bool vec4,
 void sddmm_few_rows_pieces(const DeviceInfo& dev, SddmmShape& s, int M, int nnz);  // a call without plan or memory: sets s.pieces_lg (and W = 4)
 hipError_t sddmm_launch(const SddmmArgs& x, const SddmmShape& s, hipStream_t stream);
 // Dense tiles on the matrix cores (sddmm_tiles.hip): the columns in `ranges` runs, each with its workgroups. ranges == 0: not used.
-struct TilePlan { int ranges; };
+struct TilePlan {
+    int ranges;
+    double us;  // estimated time
+};
 TilePlan sddmm_tiles_choose(const DeviceInfo& dev, int M, int K, int D, int nnz);
 void sddmm_tile_shape(int* rows, int* columns);
-hipError_t sddmm_tiles_launch(const SddmmArgs& x, const TilePlan& plan, hipStream_t stream);
+hipError_t sddmm_tiles_launch(const SddmmArgs& x, float scale, const TilePlan& plan, hipStream_t stream);  // (the results times scale)
 hipError_t sddmm_flat_launch(const SddmmArgs& x, const SddmmShape& s, int chunk, hipStream_t stream);
 hipError_t sddmm_sliced_launch(const SddmmArgs& x, const SddmmShape& s, const SlicePlan& plan, void* workspace,
                                hipStream_t stream);
 
 // K > 0: the height of Kmat and V is known and may count (operands beyond one L2 group long rows as under the even-rows hint)
 FusedShape fused_choose(const DeviceInfo& dev, int M, int D, int nnz, bool vec4, int rows = kRowsUnknown, int K = 0);
+// Bytes of the memory with which the fused op runs as SDDMM on dense tiles and SpMM one after the other; 0: it does not.
+size_t fused_two_steps_bytes(const DeviceInfo& dev, int M, int K, int D, int nnz, bool rows_even);
 bool fused_looks_for_groups(const FusedShape& s, int M, int K, int D, int nnz);  // of a launch as row blocks: the groups on the matrix cores come first
 hipError_t fused_launch(const FusedArgs& x, const FusedShape& s, hipStream_t stream);
 hipError_t fused_flat_launch(const FusedArgs& x, const FusedShape& s, const FlatPlan& plan, float* partial,

@@ -35,10 +35,10 @@ static inline SampledOut sampled_out(const SddmmArgs& x)
 }
 
 // out[j] = <lhs_row, rhs[col_indices[j]]> for the nonzeros j in [p, q) of one row (p < q, wave-uniform).
-template <int VEC, int G1, int DS, int MASKED>
+template <int VEC, int G1, int DS, int MASKED, typename Out>
 __device__ __forceinline__ void sddmm_segment(int p, int q, int D, const int* __restrict__ col_indices,
                                               const float* __restrict__ lhs_row, const float* __restrict__ rhs,
-                                              SampledOut out, int lane)
+                                              Out out, int lane)
 {
     using VecT = Vec<VEC>;
     const int g = lane % G1;

@@ -59,11 +59,17 @@ template <int STAGES, int PARTS> struct __attribute__((aligned(16))) TileLds : S
     bf16x8 lhs_parts[PARTS][kWave];
 };
 
+struct ScaledOut {
+    float* __restrict__ at;
+    float scale;
+    __device__ __forceinline__ void store(int j, float v) const { at[j] = v * scale; }
+};
+
 // SEGMENTS: of 32 floats, of a row of lhs and rhs. FULL: D == 32 SEGMENTS
 template <int SEGMENTS, bool FULL, bool STREAM>
 __global__ __launch_bounds__(kTileWaves * 64) __attribute__((amdgpu_waves_per_eu(SEGMENTS == 1 ? 4 : 2, SEGMENTS == 1 ? 4 : 2))) void sddmm_tiles_kernel(
     int M, int K, int D, int nnz, int row_blocks, int range_tiles, const int* __restrict__ row_offsets, const int* __restrict__ col_indices,
-    const float* __restrict__ lhs, const float* __restrict__ rhs, float* __restrict__ out)
+    const float* __restrict__ lhs, const float* __restrict__ rhs, float scale, float* __restrict__ out)
 {
     constexpr int KS = 2 * SEGMENTS;  // steps of sixteen floats
     constexpr bool kTwoPerUnit = SEGMENTS == 1;  // workgroups per compute unit: rhs goes through the wave's own columns of the tile
@@ -269,6 +275,7 @@ __global__ __launch_bounds__(kTileWaves * 64) __attribute__((amdgpu_waves_per_eu
         };
         auto read = [&](int i, int q) { v[i][q] = mine[i * kTileCols + ((int)min((unsigned)(c[i][q] - k0), (unsigned)kTileCols - 1) ^ turned(i))]; };
         auto store = [&](int i, int q) {
+            v[i][q] *= scale;
             all_finite = fmaf(v[i][q], 0.f, all_finite);
             if (lane + q * kWave < n[i]) {
                 float* const to = out + at[i] + q * kWave;
@@ -322,7 +329,7 @@ __global__ __launch_bounds__(kTileWaves * 64) __attribute__((amdgpu_waves_per_eu
 
     // ---- what is left: rows whose columns do not ascend, and results that are not finite
     const bool again = __ballot(!(all_finite == 0.f)) != 0;
-    const SampledOut plain{out, 0};
+    const ScaledOut plain{out, scale};
 #pragma unroll 1
     for (int i = 0; i < kRowsPerWave; ++i) {
         int from = 0, done = 0, end = 0;
@@ -345,7 +352,7 @@ __global__ __launch_bounds__(kTileWaves * 64) __attribute__((amdgpu_waves_per_eu
     }
 }
 
-template <int SEGMENTS> static hipError_t launch_one(const SddmmArgs& x, const TilePlan& plan, hipStream_t stream)
+template <int SEGMENTS> static hipError_t launch_one(const SddmmArgs& x, float scale, const TilePlan& plan, hipStream_t stream)
 {
     const long long row_blocks = ceil_div(x.M, kTileRows), blocks = row_blocks * plan.ranges;
     if (blocks <= 0 || blocks > 0x7fffffffLL) return hipErrorInvalidConfiguration;
@@ -354,7 +361,7 @@ template <int SEGMENTS> static hipError_t launch_one(const SddmmArgs& x, const T
                              : streaming ? &sddmm_tiles_kernel<SEGMENTS, false, true> : &sddmm_tiles_kernel<SEGMENTS, false, false>;
     const int range_tiles = (int)ceil_div(ceil_div(x.K, kTileCols), plan.ranges);
     hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(kTileWaves * 64), 0, stream, x.M, x.K, x.D, x.nnz, (int)row_blocks, range_tiles,
-                       x.row_offsets, x.col_indices, x.lhs, x.rhs, x.out);
+                       x.row_offsets, x.col_indices, x.lhs, x.rhs, scale, x.out);
     return hipGetLastError();
 }
 
@@ -370,7 +377,7 @@ template <int SEGMENTS> static hipError_t launch_one(const SddmmArgs& x, const T
 //               slots, one on each unit, takes about 0.75 of a full one.
 TilePlan sddmm_tiles_choose(const DeviceInfo& dev, int M, int K, int D, int nnz)
 {
-    const TilePlan none{0};
+    const TilePlan none{0, 0.0};
     if (!rule_on(kRuleDenseGroups) || D < 17 || D > 128 || M <= 0 || K <= 0 || nnz <= 0 || nnz >= (1 << 29) || !dense_fits_buffer(K + 256ll, D)) return none;
     const double density = (double)nnz / ((double)M * K);
     const int segments = (int)ceil_div(D, 32);
@@ -387,7 +394,7 @@ TilePlan sddmm_tiles_choose(const DeviceInfo& dev, int M, int K, int D, int nnz)
         const double us = rounds * ((ranges > 1 ? 8.0 : 6.0) + (double)per * tile_us);
         if (us < best_us) {
             best_us = us;
-            best = TilePlan{(int)ranges};
+            best = TilePlan{(int)ranges, us};
         }
     }
     return best;
@@ -399,13 +406,13 @@ void sddmm_tile_shape(int* rows, int* columns)
     *columns = kTileCols;
 }
 
-hipError_t sddmm_tiles_launch(const SddmmArgs& x, const TilePlan& plan, hipStream_t stream)
+hipError_t sddmm_tiles_launch(const SddmmArgs& x, float scale, const TilePlan& plan, hipStream_t stream)
 {
     const int segments = (int)ceil_div(x.D, 32);
-    if (segments == 1) return launch_one<1>(x, plan, stream);
-    if (segments == 2) return launch_one<2>(x, plan, stream);
-    if (segments == 3) return launch_one<3>(x, plan, stream);
-    if (segments == 4) return launch_one<4>(x, plan, stream);
+    if (segments == 1) return launch_one<1>(x, scale, plan, stream);
+    if (segments == 2) return launch_one<2>(x, scale, plan, stream);
+    if (segments == 3) return launch_one<3>(x, scale, plan, stream);
+    if (segments == 4) return launch_one<4>(x, scale, plan, stream);
     return hipErrorInvalidValue;
 }
 

@@ -329,16 +329,19 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(2,
 // 194 (211) and 323; 32768 x 8192 at 0.3, N = 64 400 (399) and 340; 2000 x 4608 at 0.3, N = 3136 440 (488) and 703. Uneven rows (lognormal,
 // sigma 0.6) gain less, since a row of many pairs makes its wave come back to four rows and the others wait: 32768 x 8192 at 0.3 660 -> 545,
 // 12288 x 4096 at 0.3, N = 200 241 -> 240.
+double spmm_tiles_us(const DeviceInfo& dev, int M, int K, int N, int nnz)
+{
+    const double density = (double)nnz / ((double)M * K), slice_us = 2.95 + 7.0 * std::max(0.0, density - 0.3);
+    const long long slices = ceil_div(K, kSlice), rounds = ceil_div(ceil_div(M, kRows) * ceil_div(N, kCols), dev.cus);
+    return 6.0 + (double)K * N * 3e-6 + (double)rounds * (5.0 + (double)slices * slice_us);
+}
 bool spmm_tiles_choose(const DeviceInfo& dev, int M, int K, int N, int nnz, double other_us)
 {
     const Tuning& t = tuning();
     if (!rule_on(kRuleDenseGroups) || N < 4 || M <= 0 || K <= 0 || nnz <= 0 || nnz >= (1 << 29) || K > kMostColumns || !dense_fits_buffer(K, N)) return false;
     // (a schedule that was asked for by name)
     if (t.split_w > 0 || t.flat >= 0 || t.slices >= 0 || t.tile_major >= 0 || t.tile_width > 0 || t.plan_order > 0 || t.xcd_contiguous) return false;
-    const double density = (double)nnz / ((double)M * K);
-    const long long slices = ceil_div(K, kSlice), rounds = ceil_div(ceil_div(M, kRows) * ceil_div(N, kCols), dev.cus);
-    const double slice_us = 2.95 + 7.0 * std::max(0.0, density - 0.3);
-    return 6.0 + (double)K * N * 3e-6 + (double)rounds * (5.0 + (double)slices * slice_us) < 0.9 * other_us;
+    return spmm_tiles_us(dev, M, K, N, nnz) < 0.9 * other_us;
 }
 
 static long long fragments_of(int K, int N) { return ceil_div(N, 32) * ceil_div(K, kSlice) * kSteps; }

@@ -329,7 +329,7 @@ def advise(op, width, info: MatrixInfo) -> CallPlan:
 
 class Prepared:
     """What dlspm_advise said for one matrix, op and width, allocated and built (prepare()): pass as plan=... . A size without
-    memory is that of memory which each call takes from PyTorch's allocator (SpMM on dense tiles: B's parts)."""
+    memory is that of memory which each call takes from PyTorch's allocator (B's parts for dense tiles, the scores between two steps)."""
 
     def __init__(self, memory, size_and_hints, call_plan):
         self.memory, self.size_and_hints, self.call_plan = memory, size_and_hints, call_plan
@@ -342,8 +342,10 @@ def prepare(row_offsets, col_indices, K, op, width, info=None) -> Prepared:
     info = info if info is not None else analyze(row_offsets, col_indices, K)
     cp = advise(op, width, info)
     M = row_offsets.numel() - 1
-    if op == OP_SPMM and cp.build == BUILD_NOTHING and cp.hints & HINT_ROWS_EVEN:
-        return Prepared(None, cp.bytes | cp.hints, cp)
+    if cp.bytes and cp.build == BUILD_NOTHING and op != OP_SDDMM:
+        run = describe_schedule(op, M, K, width, col_indices.numel(), workspace_bytes=cp.bytes | cp.hints)["schedule"]
+        if run in ("dense_tiles", "two_steps"):
+            return Prepared(None, cp.bytes | cp.hints, cp)
     mem = torch.empty(((cp.bytes + 3) // 4,), dtype=torch.int32, device=row_offsets.device) if cp.bytes else None
     if cp.build == BUILD_ROW_PLAN:
         st = lib().dlspm_row_plan_build(M, _ptr(row_offsets, torch.int32, "row_offsets", M + 1), ctypes.c_void_p(mem.data_ptr()),
@@ -567,17 +569,20 @@ def describe_launch(op: int, M: int, K: int, N: int, nnz: int, rows_even: bool =
                     (int(x) for x in out)))
 
 
-SCHEDULES = ("row_blocks", "flat", "sliced", "row_plan", "cut_plan", "resident", "dense_groups", "dense_tiles")
+SCHEDULES = ("row_blocks", "flat", "sliced", "row_plan", "cut_plan", "resident", "dense_groups", "dense_tiles", "two_steps")
 
 
 def describe_schedule(op: int, M: int, K: int, N: int, nnz: int, plan=None, workspace_bytes: int = 0) -> dict:
     """The schedule that a call runs (dlspm_describe_schedule): {'schedule' (one of SCHEDULES), 'rows' per workgroup, 'slice_rows',
-    'chunks'}; on dense tiles also {'tile_columns'}, with 'rows' those of a tile (SDDMM: 'schedule' is the one without tiles). plan: what
+    'chunks'}; on dense tiles also {'tile_columns'}, with 'rows' those of a tile (SDDMM: 'schedule' is the one without tiles), and of
+    two steps {'second'}, the schedule of the second. plan: what
     prepare() returned; or workspace_bytes: the size, with hint bits, that the call passes."""
     out = (ctypes.c_int * 4)()
     st = lib().dlspm_describe_schedule(op, M, K, N, nnz, plan.size_and_hints if plan is not None else workspace_bytes, out)
     if st != OK:
         raise DlspmError(st, "dlspm_describe_schedule")
+    if SCHEDULES[out[0]] == "two_steps":
+        return {"schedule": "two_steps", "rows": out[1], "slice_rows": 0, "chunks": 0, "tile_columns": out[2], "second": SCHEDULES[out[3]]}
     if out[2] > 0 and (op == OP_SDDMM or SCHEDULES[out[0]] == "dense_tiles"):
         return {"schedule": SCHEDULES[out[0]], "rows": out[1], "slice_rows": 0, "chunks": 0, "tile_columns": out[2]}
     return {"schedule": SCHEDULES[out[0]], "rows": out[1], "slice_rows": out[2], "chunks": out[3]}

@@ -225,6 +225,7 @@ PyObject* call_fused(PyObject*, PyObject* const* args, Py_ssize_t npos, PyObject
             V->sizes() != Km->sizes() || Q->size(1) != Km->size(1) || Q->size(0) < c.M || Km->size(0) > kMostInt ||
             Km->size(1) > kMostInt || !c.output(a[6], {c.M, Km->size(1)}, *Q))
             return fallback(DLSPM_OP_FUSED, args, npos, kwnames);
+        c.own_memory(*Q);
         const int K = (int)Km->size(0), D = (int)Km->size(1);
         const float scale = a[5] ? (float)PyFloat_AS_DOUBLE(a[5]) : 1.0f;
         const float *q = static_cast<const float*>(address(*Q)), *k = static_cast<const float*>(address(*Km)),

@@ -47,7 +47,9 @@
  *         memory or a plan that comes with such a call is not used. Large ones under the even-rows hint are multiplied as dense
  *         tiles on the matrix cores where that is estimated to be faster still and the call has memory for it, which then
  *         holds B split into parts: dlspm_advise names the size (6.02 bytes per float of B, its rows rounded up to 128 and
- *         its columns to 32); less memory, or none, is as good as the hint alone.
+ *         its columns to 32); less memory, or none, is as good as the hint alone. The fused op on dense masks takes two
+ *         steps where they are estimated to be faster, SDDMM on dense tiles and SpMM, with memory for the scores between
+ *         them (4 bytes per nonzero, rounded up to 256, and behind them, under the hint, that of SpMM).
  *       DLSPM_HINT_ROW_PLAN: `workspace` holds the row plan of this matrix (dlspm_row_plan_build, below; at least
  *         dlspm_row_plan_bytes(M) bytes, else DLSPM_E_WORKSPACE) and the launch hands the rows out in the plan's order.
  *         The plan is only read.
@@ -358,7 +360,8 @@ int dlspm_describe_launch_rows(int op, int M, int K, int N_or_D, int nnz, int pa
  * size other than 0 stands for memory of that size). The compute entry points decide by the same function. schedule[4]
  * receives: [0] DLSPM_SCHEDULE_*, [1] rows per workgroup (0: flat schedule), and, where [0] is DLSPM_SCHEDULE_RESIDENT, [2] rows
  * of B per slice and [3] chunks of 64 nonzeros of a row that are loaded ahead (else 0). DLSPM_SCHEDULE_DENSE_TILES: [1] rows and [2]
- * columns of C per workgroup. SDDMM on dense tiles (masks dense enough: the matrix cores compute whole tiles and the sampled results
+ * columns of C per workgroup. DLSPM_SCHEDULE_TWO_STEPS: [1] rows and [2] columns of a tile of the first step, [3] the second one's
+ * schedule. SDDMM on dense tiles (masks dense enough: the matrix cores compute whole tiles and the sampled results
  * are picked from them): [1] rows and [2] columns of a tile, [0] the schedule that the call would run without
  * DLSPM_RULE_DENSE_GROUPS. The shapes that
  * dlspm_describe_launch_rows gives are those of DLSPM_SCHEDULE_ROW_BLOCKS and _FLAT (and, as far as the fields go, of
@@ -373,6 +376,7 @@ int dlspm_describe_launch_rows(int op, int M, int K, int N_or_D, int nnz, int pa
 #define DLSPM_SCHEDULE_RESIDENT     5  /* SpMM: slices of B in LDS                                                          */
 #define DLSPM_SCHEDULE_DENSE_GROUPS 6  /* fused: row blocks, sixteen rows whose columns form one run on the matrix cores    */
 #define DLSPM_SCHEDULE_DENSE_TILES  7  /* SpMM, even rows and memory: dense tiles on the matrix cores                       */
+#define DLSPM_SCHEDULE_TWO_STEPS    8  /* fused, with memory: SDDMM on dense tiles, then SpMM                                */
 int dlspm_describe_schedule(int op, int M, int K, int N_or_D, int nnz, size_t workspace_bytes, int* schedule);
 
 /*
