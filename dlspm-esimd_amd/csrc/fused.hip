@@ -54,7 +54,7 @@ __device__ __forceinline__ void fused_segment(Vec<VEC>* acc, int p, int q, int D
     if constexpr (kWave / G > 1) slots_sum<VEC, G, V2>(acc, lane);
 }
 
-constexpr int kDenseSpan = 304;  // (p of fused_dense_group: 20 KB of the 21 ... 24 KB of its kernels, six or seven workgroups per compute unit; their 82 ... 125 registers allow four or five waves per SIMD, as many workgroups)
+constexpr int kDenseSpan = 304;  // (p and Q of fused_dense_group: 24 ... 28 KB of the 25 ... 32 KB of its kernels, five or six workgroups per compute unit; their 82 ... 118 registers allow four to six waves per SIMD, as many workgroups)
 // the row-block shapes that fused_dense_group is built for: 33 ... 128 columns, four-wave workgroups
 constexpr bool dense_groups_built(int vec, int DS, int V2, int W, int R) { return vec == 4 && DS >= 2 && DS <= 4 && V2 == 1 && W == 4 && R <= 16; }
 
@@ -62,10 +62,11 @@ constexpr bool dense_groups_built(int vec, int DS, int V2, int W, int R) { retur
 // group computes them on the matrix cores, the others leave. What bounds the row-by-row path is the vector-memory path of
 // the compute unit, through which every row gathers its own rows of Kmat and V; here each of them is read once for all sixteen
 // and the time is that of the workgroups' chains of loads and, with four workgroups per compute unit, of the fp32 matrix cores (9
-// us; three operand sets in turn, row by row -> here: 16384 rows, 128 columns per row, D = 128: 69 -> 29.1 us, D = 64: 37 -> 17.0 us;
-// 38.6 and 21.4 while a row's columns were loaded 64 at a time, V two tiles ahead and a group led by one of its own workgroups).
+// us; three operand sets in turn, row by row -> here: 16384 rows, 128 columns per row, D = 128: 69 -> 24.6 us, D = 64: 37 -> 15.4 us;
+// 38.6 and 21.4 while a row's columns were loaded 64 at a time, V two tiles ahead and a group led by one of its own workgroups;
+// 28.2 and 16.9 while every wave loaded all of Q for itself and V was asked for behind the barrier).
 //   1  p[r][x] <- 1 where row r has column c0 + x (LDS; plain stores: LDS float atomics took 9 us of the first figure)
-//   2  16 x 16 tiles of Q Kmat^T by v_mfma_f32_16x16x4_f32, one wave per tile; p[r][x] <- scale x score where marked
+//   2  16 x 16 tiles of Q Kmat^T (Q in LDS) by v_mfma_f32_16x16x4_f32, one wave per tile; p[r][x] <- scale x score where marked
 //   3  O = p V by the same instruction, D / 4 columns of O per wave
 // A score is summed in eight chains of D / 8 products as the row-by-row path does, a row of O in four chains per kAhead tiles
 // whose sums are added: an error against 64 bits of 1.1e-7 ... 1.3e-7 (the row-by-row path: 1.3e-7 ... 2.4e-7 on the same calls; one
@@ -86,6 +87,7 @@ __device__ __forceinline__ bool fused_dense_group(int row0, int offsets, int M, 
     typedef float f4 __attribute__((ext_vector_type(4)));
     constexpr int kRows = 16, kStride = kDenseSpan + 4, NQ = 2 * DS, NT = DS <= 2 ? 1 : 2;
     __shared__ __attribute__((aligned(16))) float s_p[kRows * kStride];
+    __shared__ __attribute__((aligned(16))) float s_q[kRows * NQ * 16];  // four floats at a time: quad i of row r is (i * 16 + (r ^ (i & 15)))-th
     __shared__ int s_left, s_marks;
     if (row0 + kRows > M) return false;
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = lane & 15, kq = lane >> 4;
@@ -121,19 +123,23 @@ __device__ __forceinline__ bool fused_dense_group(int row0, int offsets, int M, 
     if constexpr (!LEADS) return true;
     const int tiles = (span + 15) >> 4;
 
-    // four consecutive floats of a row, the q-th sixteen of them dealt to the four k of the lanes (zero past D)
-    auto quad = [&](const float* a, int row, int q) -> f4 {
-        const int d = 16 * q + 4 * kq;
+    // four consecutive floats of a row (zero past D)
+    auto quad = [&](const float* a, int row, int d) -> f4 {
         const bool in = !MASKED || d < D;
         const Vec<4> x = Vec<4>::gload(a + (size_t)row * D + (in ? d : 0));
         return in ? f4{x.v.x, x.v.y, x.v.z, x.v.w} : f4{0.f, 0.f, 0.f, 0.f};
     };
-    f4 qf[NQ], kf[NQ];
+    constexpr int kQuads = 4 * NQ, kOwn = (kRows * kQuads + 255) / 256;  // of Q per row and thread
+    f4 own[kOwn], kf[NQ];
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) qf[q] = quad(Q, row0 + l, q);
+    for (int i = 0; i < kOwn; ++i) {
+        const int at_quad = i * 256 + threadIdx.x;
+        if (kRows * kQuads % 256 == 0 || at_quad < kRows * kQuads) own[i] = quad(Q, row0 + at_quad / kQuads, at_quad % kQuads * 4);
+    }
+    // the q-th sixteen floats of the tile's rows of Kmat are dealt to the four k of the lanes
     auto load_k = [&](int t) {
 #pragma unroll
-        for (int q = 0; q < NQ; ++q) kf[q] = quad(Kmat, c0 + min(16 * t + l, span - 1), q);
+        for (int q = 0; q < NQ; ++q) kf[q] = quad(Kmat, c0 + min(16 * t + l, span - 1), 16 * q + 4 * kq);
     };
     if (w < tiles) load_k(w);
     {
@@ -141,6 +147,11 @@ __device__ __forceinline__ bool fused_dense_group(int row0, int offsets, int M, 
         for (int x = l * 4; x < tiles * 16; x += 64) *reinterpret_cast<f4*>(mine + x) = f4{0.f, 0.f, 0.f, 0.f};
     }
     if (threadIdx.x == 0) s_left = s_marks = 0;
+#pragma unroll
+    for (int i = 0; i < kOwn; ++i) {
+        const int at_quad = i * 256 + threadIdx.x, q = at_quad % kQuads;
+        if (kRows * kQuads % 256 == 0 || at_quad < kRows * kQuads) *reinterpret_cast<f4*>(s_q + (q * 16 + ((at_quad / kQuads) ^ (q & 15))) * 4) = own[i];
+    }
     __syncthreads();
     {
 #pragma unroll
@@ -163,9 +174,19 @@ __device__ __forceinline__ bool fused_dense_group(int row0, int offsets, int M, 
         int marks = 0;
         for (int t = w; t < tiles; t += 4) {
             f4 part[8];
+            auto read_q = [&](int q) { return *reinterpret_cast<const f4*>(s_q + ((4 * q + kq) * 16 + (l ^ ((4 * q + kq) & 15))) * 4); };
+            f4 next_q = read_q(0);
 #pragma unroll
-            for (int i = 0; i < NQ * 4; ++i)
-                part[i % 8] = __builtin_amdgcn_mfma_f32_16x16x4f32(qf[i / 4][i % 4], kf[i / 4][i % 4], i < 8 ? f4{0.f, 0.f, 0.f, 0.f} : part[i % 8], 0, 0, 0);
+            for (int q = 0; q < NQ; ++q) {
+                const f4 of_q = next_q;
+                if (q + 1 < NQ) next_q = read_q(q + 1);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int i = 4 * q + j;
+                    part[i % 8] = __builtin_amdgcn_mfma_f32_16x16x4f32(of_q[j], kf[q][j], i < 8 ? f4{0.f, 0.f, 0.f, 0.f} : part[i % 8], 0, 0, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);  // (all of Q at once would spill)
+            }
             if (t + 4 < tiles) load_k(t + 4);
             const f4 score = ((part[0] + part[1]) + (part[2] + part[3])) + ((part[4] + part[5]) + (part[6] + part[7]));
 #pragma unroll
@@ -176,28 +197,8 @@ __device__ __forceinline__ bool fused_dense_group(int row0, int offsets, int M, 
                 *p = marked ? score[i] * scale : 0.f;
             }
         }
-        marks += __builtin_amdgcn_update_dpp(0, marks, kDppQuadSwap1, 0xF, 0xF, true);
-        marks += __builtin_amdgcn_update_dpp(0, marks, kDppQuadSwap2, 0xF, 0xF, true);
-        marks += __builtin_amdgcn_update_dpp(0, marks, kDppRowHalfMirror, 0xF, 0xF, true);
-        marks += __builtin_amdgcn_update_dpp(0, marks, kDppRowMirror, 0xF, 0xF, true);
-        if (l == 0) __hip_atomic_fetch_add(&s_marks, marks, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        __syncthreads();
+        // (V's first tiles are on their way while the waves with fewer tiles wait)
         const int d = min(w * 16 * NT + NT * l, D - NT);  // (lanes past D repeat the last columns and store nothing)
-        f4 acc[NT];
-#pragma unroll
-        for (int n = 0; n < NT; ++n) acc[n] = f4{0.f, 0.f, 0.f, 0.f};
-        f4 part[4][NT];
-        auto clear = [&]() {
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-#pragma unroll
-                for (int n = 0; n < NT; ++n) part[j][n] = f4{0.f, 0.f, 0.f, 0.f};
-        };
-        auto fold = [&]() {
-#pragma unroll
-            for (int n = 0; n < NT; ++n) acc[n] += (part[0][n] + part[1][n]) + (part[2][n] + part[3][n]);
-        };
-        clear();
         constexpr int kAhead = 4;  // tiles of V on their way, and of a chain
         float v[kAhead][4][NT];
         auto load_v = [&](int t, int to) {
@@ -214,6 +215,27 @@ __device__ __forceinline__ bool fused_dense_group(int row0, int offsets, int M, 
         };
 #pragma unroll
         for (int t = 0; t < kAhead; ++t) load_v(t, t);
+        marks += __builtin_amdgcn_update_dpp(0, marks, kDppQuadSwap1, 0xF, 0xF, true);
+        marks += __builtin_amdgcn_update_dpp(0, marks, kDppQuadSwap2, 0xF, 0xF, true);
+        marks += __builtin_amdgcn_update_dpp(0, marks, kDppRowHalfMirror, 0xF, 0xF, true);
+        marks += __builtin_amdgcn_update_dpp(0, marks, kDppRowMirror, 0xF, 0xF, true);
+        if (l == 0) __hip_atomic_fetch_add(&s_marks, marks, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        __syncthreads();
+        f4 acc[NT];
+#pragma unroll
+        for (int n = 0; n < NT; ++n) acc[n] = f4{0.f, 0.f, 0.f, 0.f};
+        f4 part[4][NT];
+        auto clear = [&]() {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int n = 0; n < NT; ++n) part[j][n] = f4{0.f, 0.f, 0.f, 0.f};
+        };
+        auto fold = [&]() {
+#pragma unroll
+            for (int n = 0; n < NT; ++n) acc[n] += (part[0][n] + part[1][n]) + (part[2][n] + part[3][n]);
+        };
+        clear();
         for (int t0 = 0; t0 < tiles; t0 += kAhead) {
 #pragma unroll
             for (int i = 0; i < kAhead; ++i) {

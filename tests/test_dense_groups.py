@@ -178,3 +178,16 @@ def test_groups_led_by_workgroups_of_other_rows(M, D):
     whole = np.array([[kind[(g * 16 + i) // 48] for i in range(16)] for g in range(M // 16)])
     assert differ[(whole == 0).all(axis=1)].any(axis=1).all()  # on the matrix cores
     assert not differ[(whole == 1).all(axis=1)].any()          # row by row
+
+
+@pytest.mark.parametrize("D", [36, 64, 68, 96, 100, 128])
+def test_widths_whole_and_ragged(D):
+    """Q goes through LDS a whole number of times per thread, or once and a half (D = 65 ... 96): every row of a group is there"""
+    ro, ci, rng = window(20003, 20003, 200, D, 0.02)
+    Q, Km, V = (rng.normal(size=(20003, D)).astype(np.float32) for _ in range(3))
+    got, other = run(ro, ci, Q, Km, V, 0.125)
+    differ = (got != other).any(axis=1)[:20000]
+    assert differ.mean() > 0.99
+    # row by row: each row's own error is that of its chains (as in test_no_less_precise_than_row_by_row, of one row: three times the mean)
+    off = np.linalg.norm(got - other, axis=1) / np.linalg.norm(other, axis=1)
+    assert off.max() <= 2e-6, off.max()
