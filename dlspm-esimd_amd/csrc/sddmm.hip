@@ -19,7 +19,7 @@
 
 namespace dlspm {
 
-// The same for one row shared by the W waves of a workgroup: the row is gone through in passes of `chunk` nonzeros, wave w
+// The dot products of one row (sddmm_segment) shared by the W waves of a workgroup: the row is gone through in passes of `chunk` nonzeros, wave w
 // taking the passes w, w + W, ... -- so that the waves go through the row's (ascending) columns together, and so that no
 // wave is left with a nearly empty pass of its own (an even split of 300 nonzeros over four waves is 64 + 11 each: two
 // passes; here it is two passes of 40). `chunk` is the row's length over the fewest passes per wave that passes of 64
