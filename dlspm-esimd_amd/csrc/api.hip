@@ -529,9 +529,10 @@ static SddmmCall sddmm_decide(const DeviceInfo& dev, int M, int K, int D, int nn
 }
 
 // The fused op as SDDMM on dense tiles and then SpMM, the scores in the caller's memory in between: where the masks are dense enough that
-// the scores of whole tiles cost less than the gathered ones, and both steps together take less than 0.95 of the fused kernels' time.
-// Estimates (us): those of the two steps, 2 for the second launch, and 2 + nnz x 0.0100 / 0.0162 / 0.0343 x 1e-3 for the fused kernels at
-// D <= 32 / 64 / 128 (8192 x 8192, D = 128 at 0.1 / 0.2 / 0.3 232 / 442 / 688, D = 32 at 0.3 200; 16384 x 4096, D = 64 at 0.2 218;
+// the scores of whole tiles cost less than the gathered ones, and both steps together take less than 0.92 of the fused kernels' time (10691 x 4000,
+// D = 95 at 0.14, and 2919 x 5655, D = 75 at 0.13, estimated at 0.95: 198 -> 207 and 71 -> 79).
+// Estimates (us): those of the two steps, 2 for the second launch, and 2 + nnz x 0.0100 / 0.0162 / 0.0315 / 0.0343 x 1e-3 for the fused kernels
+// at D <= 32 / 64 / 96 / 128 (8192 x 8192, D = 128 at 0.1 / 0.2 / 0.3 232 / 442 / 688, D = 32 at 0.3 200; 16384 x 4096, D = 64 at 0.2 218;
 // 24576 x 8192, D = 80 at 0.1 623). A second step of row blocks takes more than its estimate on uneven rows (4000 x 4090, D = 77 at 0.2,
 // lognormal: fused 96, two steps 118) and below D = 64 (8192 x 8192, D = 32 at 0.3 145, estimate 105). Measured, fused -> two steps: 8192 x 8192, D = 128 at 0.1 / 0.2 / 0.3 230 / 437 / 683 -> 206 / 261 / 325, with
 // lognormal rows at 0.3 747 -> 392; 16384 x 8192, D = 128 at 0.3 1357 -> 451; 16384 x 4096, D = 64 at 0.2 217 -> 144; 4096 x 4096, D = 128 at
@@ -556,8 +557,8 @@ static bool fused_two_steps(const DeviceInfo& dev, int M, int K, int D, int nnz,
     c.second = spmm_decide(dev, M, K, D, nnz, behind_scores(ws, nnz));
     const double second_us = c.second.schedule == DLSPM_SCHEDULE_DENSE_TILES ? spmm_tiles_us(dev, M, K, D, nnz) : c.second.resident.us;
     if (c.second.schedule == DLSPM_SCHEDULE_ROW_BLOCKS && (!ws.rows_even || D < 64)) return false;
-    const double fused_us = 2.0 + (double)nnz * (D <= 32 ? 1.00e-5 : D <= 64 ? 1.62e-5 : 3.43e-5);
-    return c.second.resident.us > 0.0 && c.tiles.us + second_us + 2.0 < 0.95 * fused_us;  // (no estimate: a schedule was asked for by name)
+    const double fused_us = 2.0 + (double)nnz * (D <= 32 ? 1.00e-5 : D <= 64 ? 1.62e-5 : D <= 96 ? 3.15e-5 : 3.43e-5);
+    return c.second.resident.us > 0.0 && c.tiles.us + second_us + 2.0 < 0.92 * fused_us;  // (no estimate: a schedule was asked for by name)
 }
 size_t fused_two_steps_bytes(const DeviceInfo& dev, int M, int K, int D, int nnz, bool rows_even)
 {
