@@ -13,8 +13,10 @@
 //     The products of a slice and the scatter of the next one are one stream of instructions, a product, four others and two writes in turn.
 //   * hi x hi of a slice's steps is added up in 32 bits and goes to 64 bits slice by slice; the five smaller products have sums of
 //     their own. The two halves of the steps meet in LDS at the end.
-// Rows whose columns do not ascend, results that are not finite, and values too small for their parts are computed once more from the
-// floats, row by row.
+// Values of B that are not finite have zeros for parts and are added at the end, to the rows that use them (one NaN in B, 16384 x 8192,
+// N = 128 at 0.3: 1601 us while it went through the products and made every row of its column one to compute again, now 245).
+// Rows whose columns do not ascend, other results that are not finite, and values too small for their parts are computed once more
+// from the floats, row by row.
 // Measured (us, three operand sets in turn, resident -> tiles): 32768 x 8192, N = 128 at 0.2 / 0.3 527 / 647 -> 392 / 420; 16384 x 8192 at 0.2 / 0.3 / 0.5
 // 266 / 327 / 496 -> 204 / 206 / 291; 4096 x 4096, N = 512 at 0.5 245 -> 134; 16384 x 2048, N = 256 at 0.3 173 -> 113; 2000 x 4608, N = 3136 at 0.3
 // 703 -> 440. Against 64 bits the results are off by 3.0 ... 3.4e-8, the resident schedule's by 6.9 ... 7.1e-8.
@@ -36,8 +38,12 @@ constexpr int kTileWaves = 8, kTileThreads = kTileWaves * 64;
 constexpr int kFragmentBytes = 3 * kWave * 16;
 
 // ---- B: split once, in the order in which the products read it: [strip of 32 columns][step][part][lane][8]
+// A value that is not finite, or that bf16 rounds to infinity, would make every result of its column NaN, through the zeros of A as
+// well: its parts are zeros, and the rows that have its column get it from the float (spmm_tiles_kernel). Per strip and step, in a word:
+// bits 0 ... 31 the columns with a nonzero value below 2^-109, 32 ... 47 the rows of B with a value that has no parts.
+constexpr unsigned kTooLarge = 0xfeff0000u;  // twice the bits of a value, from this on: no parts
 __global__ __launch_bounds__(256) void split_dense_kernel(int K, int N, int steps, const float* __restrict__ B, bf16x8* __restrict__ parts,
-                                                          unsigned long long* __restrict__ too_small)
+                                                          unsigned long long* __restrict__ notes)
 {
     const int lane = threadIdx.x & 63, l = lane & 31, h = lane >> 5;
     const long long fragment = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -45,8 +51,14 @@ __global__ __launch_bounds__(256) void split_dense_kernel(int K, int N, int step
     if (strip * 32 >= N) return;
     const int n = strip * 32 + l, k0 = 16 * step + 8 * h;
     float x[8];
+    unsigned without = 0;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) x[j] = n < N && k0 + j < K ? B[(size_t)(k0 + j) * N + n] : 0.f;
+    for (int j = 0; j < 8; ++j) {
+        x[j] = n < N && k0 + j < K ? B[(size_t)(k0 + j) * N + n] : 0.f;
+        const bool none = (__float_as_uint(x[j]) << 1) >= kTooLarge;
+        without |= none ? 1u << j : 0u;
+        x[j] = none ? 0.f : x[j];
+    }
     unsigned least;
     const Parts p = split_parts(x, least);
     bf16x8* const to = parts + fragment * 3 * kWave + lane;
@@ -54,9 +66,15 @@ __global__ __launch_bounds__(256) void split_dense_kernel(int K, int N, int step
     to[kWave] = p.mid;
     to[2 * kWave] = p.lo;
     const unsigned long long few = __ballot(least < kTooSmall);
-    if (lane == 0) too_small[fragment] = few;
+    unsigned long long note = (unsigned)few | (unsigned)(few >> 32);
+    if (__ballot(without != 0) != 0)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const unsigned long long in = __ballot((without >> j & 1) != 0);
+            note |= (unsigned long long)((unsigned)in != 0 ? 1 : 0) << (32 + j) | (unsigned long long)((unsigned)(in >> 32) != 0 ? 1 : 0) << (40 + j);
+        }
+    if (lane == 0) notes[fragment] = note;
 }
-
 
 constexpr int kRows = 64, kCols = 128;                     // of C per workgroup
 constexpr int kSlice = 128, kSteps = kSlice / 16;          // columns of A worked on at a time, in steps of sixteen
@@ -64,11 +82,19 @@ constexpr int kRowBytes = kSlice * 2 + 16, kPartBytes = kRows * kRowBytes, kBuff
 constexpr int kMostColumns = 1 << 22;                      // (a strip's parts are read as a buffer)
 constexpr int kMine = kSteps / 2;                          // steps per wave: two waves share a strip
 constexpr int kAhead = 2;                                  // steps of B loaded ahead
+// the end, in the same LDS: the sums of one way (then what values of B without parts add), and behind them
+constexpr int kSumBytes = 4 * 32 * kWave * (int)sizeof(double), kLoad = 4 * kWave;
+struct EndLds {
+    int again[kRows];  // the row is computed from the floats
+    unsigned without;  // some strip of the tile has values of B without parts
+};
+constexpr int kMarkSteps = (kSumBytes - kRows * kCols * (int)sizeof(float)) / (int)sizeof(unsigned short);
+static_assert(kMarkSteps % kTileThreads == 0, "steps that share a mark are one thread's");
 
 __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void spmm_tiles_kernel(
     int M, int K, int N, int nnz, int col_tiles, int streaming, const int* __restrict__ row_offsets, const int* __restrict__ col_indices,
     const float* __restrict__ values, const float* __restrict__ B, const bf16x8* __restrict__ parts,
-    const unsigned long long* __restrict__ too_small, float* __restrict__ C)
+    const unsigned long long* __restrict__ notes, float* __restrict__ C)
 {
     typedef unsigned u4 __attribute__((ext_vector_type(4)));
     extern __shared__ __attribute__((aligned(16))) char shared[];
@@ -236,89 +262,180 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(2,
         __syncthreads();
     }
 
-    // ---- the two ways' sums
-    double* const sums = reinterpret_cast<double*>(shared);
-    int* const again = reinterpret_cast<int*>(shared + 4 * 32 * kWave * 8);  // per row
+    // (the thread's place once more: kept through the loop, it would be spilled)
+    int thread = threadIdx.x;
+    asm("" : "+v"(thread));
+    {
+        const int t = thread, lane = t & 63, l = lane & 31, h = lane >> 5, l16 = lane & 15, own_row = 8 * w + (lane >> 4);
+        // ---- the two ways' sums
+        double* const sums = reinterpret_cast<double*>(shared);
+        EndLds& end = *reinterpret_cast<EndLds*>(shared + kSumBytes);
 #pragma unroll
-    for (int i = 0; i < 32; ++i) {
-        total[i / 16][i % 16] += (double)sum[i / 16][i % 16] + (double)small[i / 16][i % 16];
-        if (way > 0) sums[(strip * 32 + i) * kWave + lane] = total[i / 16][i % 16];
-    }
+        for (int i = 0; i < 32; ++i) {
+            total[i / 16][i % 16] += (double)sum[i / 16][i % 16] + (double)small[i / 16][i % 16];
+            if (way > 0) sums[(strip * 32 + i) * kWave + lane] = total[i / 16][i % 16];
+        }
 #pragma unroll
-    for (int g = 0; g < 2; ++g) {
-        const unsigned long long bad = __ballot(wrong[g] || tiny || p[g] < e[g]);
-        if (l16 == 0) again[own_row + 4 * g] = (bad >> (lane & 48) & 0xffff) != 0 ? 1 : 0;
-    }
-    __syncthreads();
-    if (way == 0) {
-        unsigned long long few = 0;  // columns (twice 32) of the strip with a value of B that its parts do not hold
-        for (int i = lane; i < steps; i += kWave) few |= too_small[(size_t)min(col0 / 32 + strip, (N - 1) / 32) * steps + i];
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) few |= __shfl_xor(few, o);
-        // Such a value is off by 2^-134 at most: of no account for results from 2^34 times what that can come to on.
+        for (int g = 0; g < 2; ++g) {
+            const unsigned long long bad = __ballot(wrong[g] || tiny || p[g] < e[g]);
+            if (l16 == 0) end.again[own_row + 4 * g] = (bad >> (lane & 48) & 0xffff) != 0 ? 1 : 0;
+        }
+        if (t == 0) end.without = 0;
+        __syncthreads();
+        const unsigned long long* const strip_notes = notes + (size_t)min(col0 / 32 + strip, (N - 1) / 32) * steps;
+        unsigned few = 0;  // columns of the strip with a value of B that its parts do not hold
         float bound = 0.f;
-        if (few != 0) {
-            float most = 0.f;
-            for (int i = row_offsets[row0] + lane; i < row_offsets[min(row0 + kRows, M)]; i += kWave) most = fmaxf(most, fabsf(values[i]));
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) most = fmaxf(most, __shfl_xor(most, o));
-            bound = (float)K * most * 0x1p-100f;
-        }
-#pragma unroll
-        for (int r = 0; r < 2; ++r) {
-            bool bad = false;
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                total[r][i] += sums[(strip * 32 + 16 * r + i) * kWave + lane];
-                const float x = (float)total[r][i];
-                const int n = 8 * (i / 4) + 4 * h + i % 4;
-                bad = bad || (col0 + 32 * strip + n < N && (!(fabsf(x) < __builtin_inff()) || ((few >> n | few >> (32 + n)) & 1 && !(fabsf(x) >= bound))));
+        if (way == 0) {
+            unsigned without = 0;
+            for (int i = lane; i < steps; i += kWave) {
+                const unsigned long long note = strip_notes[i];
+                few |= (unsigned)note;
+                without |= (unsigned)(note >> 32) & 0xffffu;
             }
-            if (bad) again[32 * r + l] = 1;
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) {
+                few |= __shfl_xor(few, o);
+                without |= __shfl_xor(without, o);
+            }
+            if (lane == 0 && without != 0) end.without = 1;
+            // A value below 2^-109 is off by 2^-134 at most in its parts: of no account for results from 2^34 times what that can come to on.
+            if (few != 0) {
+                float most = 0.f;
+                for (int i = row_offsets[row0] + lane; i < row_offsets[min(row0 + kRows, M)]; i += kWave) most = fmaxf(most, fabsf(values[i]));
+#pragma unroll
+                for (int o = 32; o > 0; o >>= 1) most = fmaxf(most, __shfl_xor(most, o));
+                bound = (float)K * most * 0x1p-100f;
+            }
+#pragma unroll
+            for (int i = 0; i < 32; ++i) total[i / 16][i % 16] += sums[(strip * 32 + i) * kWave + lane];
         }
-    }
-    __syncthreads();
-    if (way == 0)
+        __syncthreads();
+        if (way == 0) {
 #pragma unroll
-        for (int r = 0; r < 2; ++r)
-            if (row0 + 32 * r + l < M && again[32 * r + l] == 0)
+            for (int r = 0; r < 2; ++r) {
+                bool bad = false;
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const int n = col0 + 32 * strip + 8 * q + 4 * h;
-                    float* const to = C + (size_t)(row0 + 32 * r + l) * N + n;
-                    const Vec<4> x{make_float4((float)total[r][4 * q], (float)total[r][4 * q + 1], (float)total[r][4 * q + 2], (float)total[r][4 * q + 3])};
-                    if (n + 3 < N) x.gstore(to, streaming != 0);
-                    else {
-                        if (n < N) to[0] = x.v.x;
-                        if (n + 1 < N) to[1] = x.v.y;
-                        if (n + 2 < N) to[2] = x.v.z;
-                    }
+                for (int i = 0; i < 16; ++i) {
+                    const float x = fabsf((float)total[r][i]);
+                    const int n = 8 * (i / 4) + 4 * h + i % 4;
+                    const float least = (few >> n & 1) != 0 ? bound : 0.f;
+                    bad |= (col0 + 32 * strip + n < N) & !((x >= least) & (x < __builtin_inff()));
                 }
-    // ---- rows whose columns do not ascend, and results that the parts do not give: from the floats, in CSR order, in 64 bits
-    for (int i = w; i < kRows; i += kTileWaves) {
-        if (again[i] == 0 || row0 + i >= M) continue;
-        const int from = __builtin_amdgcn_readfirstlane(row_offsets[row0 + i]), to = __builtin_amdgcn_readfirstlane(row_offsets[row0 + i + 1]);
-        const float* const b0 = B + min(col0 + lane, N - 1);
-        const float* const b1 = B + min(col0 + lane + kWave, N - 1);
-        double x0 = 0.0, x1 = 0.0;
-        for (int j = from; j < to; j += kWave) {
-            const int count = min(to - j, kWave), column = col_indices[min(j + lane, to - 1)];
-            const unsigned value = __float_as_uint(values[min(j + lane, to - 1)]);
-            auto add = [&](int k) {
-                const size_t row = (size_t)__builtin_amdgcn_readlane(column, k) * N;
-                const double v = __uint_as_float(__builtin_amdgcn_readlane(value, k));
-                x0 = fma(v, (double)b0[row], x0);
-                x1 = fma(v, (double)b1[row], x1);
-            };
-            int k = 0;
-            for (; k + 8 <= count; k += 8)
-#pragma unroll
-                for (int u = 0; u < 8; ++u) add(k + u);
-            for (; k < count; ++k) add(k);
+                if (bad) end.again[32 * r + l] = 1;
+            }
         }
-        float* const to_row = C + (size_t)(row0 + i) * N + col0;
-        if (col0 + lane < N) to_row[lane] = (float)x0;
-        if (col0 + lane + kWave < N) to_row[lane + kWave] = (float)x1;
+        __syncthreads();
+
+        // ---- two columns of a row of the tile per lane
+        const int c0 = col0 + 2 * lane, c0_at = min(c0, N - 2);
+        const bool in0 = c0 < N, in1 = c0 + 1 < N;
+        typedef float f2 __attribute__((ext_vector_type(2), aligned(4)));
+        auto load_two = [&](int column) {
+            f2 b = *reinterpret_cast<const f2*>(B + (size_t)column * N + c0_at);
+            b.x = c0 == c0_at ? b.x : b.y;
+            return b;
+        };
+        // ---- what the values of B without parts add: to the rows that have their columns, and to no others
+        float* const extra = reinterpret_cast<float*>(shared);  // [row][column of the tile]
+        if (end.without != 0) {  // (uniform)
+            unsigned short* const of_step = reinterpret_cast<unsigned short*>(extra + kRows * kCols);  // which rows of B, per step modulo kMarkSteps
+            for (int at = t; at < min(steps, kMarkSteps); at += kTileThreads) {
+                unsigned long long any = 0;
+                for (int i = at; i < steps; i += kMarkSteps)
+#pragma unroll
+                    for (int q = 0; q < kCols / 32; ++q) any |= notes[(size_t)min(col0 / 32 + q, (N - 1) / 32) * steps + i];
+                of_step[at] = (unsigned short)(any >> 32);
+            }
+            __syncthreads();
+            for (int i = w; i < kRows; i += kTileWaves) {
+                double x0 = 0.0, x1 = 0.0;
+                if (end.again[i] == 0 && row0 + i < M) {
+                    const int from = __builtin_amdgcn_readfirstlane(row_offsets[row0 + i]), to = __builtin_amdgcn_readfirstlane(row_offsets[row0 + i + 1]);
+                    bool large = false;  // a finite value: the sum is wanted as a whole
+                    constexpr int kLoads = 4;
+                    for (int j = from; j < to; j += kLoads * kLoad) {
+                        u4 k[kLoads];
+#pragma unroll
+                        for (int q = 0; q < kLoads; ++q)
+                            k[q] = __builtin_bit_cast(u4, __builtin_amdgcn_raw_buffer_load_b128(columns_buffer, (unsigned)(j + q * kLoad + 4 * lane) * 4u, 0, 0));
+                        unsigned hits = 0;  // of the lane's pairs
+#pragma unroll
+                        for (int i = 0; i < 4 * kLoads; ++i) {
+                            const unsigned mine = j + i / 4 * kLoad + 4 * lane + i % 4 < to ? 1u : 0u, column = k[i / 4][i % 4];
+                            hits |= ((unsigned)of_step[mine * (column >> 4) % kMarkSteps] >> (column & 15) & mine) << i;
+                        }
+                        for (unsigned long long left; (left = __ballot(hits != 0)) != 0;) {
+                            const int of = __builtin_ctzll(left), i = __builtin_ctz(__builtin_amdgcn_readlane(hits, of)), at = j + i / 4 * kLoad + 4 * of + i % 4;
+                            if (lane == of) hits &= hits - 1;
+                            const f2 b = load_two(col_indices[at]);
+                            const double v = values[at];
+                            const bool none0 = in0 && (__float_as_uint(b.x) << 1) >= kTooLarge, none1 = in1 && (__float_as_uint(b.y) << 1) >= kTooLarge;
+                            large = large || (none0 && fabsf(b.x) < __builtin_inff()) || (none1 && fabsf(b.y) < __builtin_inff());
+                            if (none0) x0 = fma(v, (double)b.x, x0);
+                            if (none1) x1 = fma(v, (double)b.y, x1);
+                        }
+                        // (nothing changes any more)
+                        if (__ballot(large) != 0 || __ballot((in0 && x0 == x0) || (in1 && x1 == x1)) == 0) break;
+                    }
+                    if (__ballot(large) != 0) end.again[i] = 1;
+                }
+                *reinterpret_cast<float2*>(extra + i * kCols + 2 * lane) = make_float2((float)x0, (float)x1);
+            }
+            __syncthreads();
+        }
+        if (way == 0)
+#pragma unroll
+            for (int r = 0; r < 2; ++r)
+                if (row0 + 32 * r + l < M && end.again[32 * r + l] == 0)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const int at = 32 * strip + 8 * q + 4 * h, n = col0 + at;
+                        float* const to = C + (size_t)(row0 + 32 * r + l) * N + n;
+                        Vec<4> x{make_float4((float)total[r][4 * q], (float)total[r][4 * q + 1], (float)total[r][4 * q + 2], (float)total[r][4 * q + 3])};
+                        if (end.without != 0) {
+                            const float4 y = *reinterpret_cast<const float4*>(extra + (32 * r + l) * kCols + at);
+                            x.v = make_float4(x.v.x + y.x, x.v.y + y.y, x.v.z + y.z, x.v.w + y.w);
+                        }
+                        if (n + 3 < N) x.gstore(to, streaming != 0);
+                        else {
+                            if (n < N) to[0] = x.v.x;
+                            if (n + 1 < N) to[1] = x.v.y;
+                            if (n + 2 < N) to[2] = x.v.z;
+                        }
+                    }
+        // ---- rows whose columns do not ascend, and results that the parts do not give: from the floats, in CSR order, in 64 bits
+        for (int i = w; i < kRows; i += kTileWaves) {
+            if (end.again[i] == 0 || row0 + i >= M) continue;
+            const int from = __builtin_amdgcn_readfirstlane(row_offsets[row0 + i]), to = __builtin_amdgcn_readfirstlane(row_offsets[row0 + i + 1]);
+            double x0 = 0.0, x1 = 0.0;
+            int next_column = from < to ? col_indices[min(from + lane, to - 1)] : 0;
+            float next_value = from < to ? values[min(from + lane, to - 1)] : 0.f;
+            for (int j = from; j < to; j += kWave) {
+                const int count = min(to - j, kWave), column = next_column;
+                const int2 value = __builtin_bit_cast(int2, (double)next_value);  // (a conversion takes as long as four products)
+                next_column = col_indices[min(j + kWave + lane, to - 1)];
+                next_value = values[min(j + kWave + lane, to - 1)];
+                constexpr int kFlight = 16;
+                auto add = [&](const f2& b, int k) {
+                    const double v = __builtin_bit_cast(double, make_int2(__builtin_amdgcn_readlane(value.x, k), __builtin_amdgcn_readlane(value.y, k)));
+                    x0 = fma(v, (double)b.x, x0);
+                    x1 = fma(v, (double)b.y, x1);
+                };
+                int k = 0;
+                for (; k + kFlight <= count; k += kFlight) {
+                    f2 b[kFlight];
+#pragma unroll
+                    for (int u = 0; u < kFlight; ++u) b[u] = load_two(__builtin_amdgcn_readlane(column, k + u));
+#pragma unroll
+                    for (int u = 0; u < kFlight; ++u) add(b[u], k + u);
+                }
+#pragma unroll 1
+                for (; k < count; ++k) add(load_two(__builtin_amdgcn_readlane(column, k)), k);
+            }
+            float* const to_row = C + (size_t)(row0 + i) * N + c0;
+            if (in0) to_row[0] = (float)x0;
+            if (in1) to_row[1] = (float)x1;
+        }
     }
 }
 
@@ -361,12 +478,12 @@ hipError_t spmm_tiles_launch(const SpmmArgs& x, void* memory, hipStream_t stream
     const long long fragments = fragments_of(x.K, x.N), blocks = (ceil_div(x.M, kRows) + 7) / 8 * 8 * col_tiles;
     if (blocks > 0x7fffffffLL || fragments > 0x7fffffffLL) return hipErrorInvalidConfiguration;
     bf16x8* const parts = static_cast<bf16x8*>(memory);
-    unsigned long long* const too_small = reinterpret_cast<unsigned long long*>(static_cast<char*>(memory) + fragments * kFragmentBytes);
-    hipLaunchKernelGGL(split_dense_kernel, dim3((unsigned)ceil_div(fragments, 4)), dim3(256), 0, stream, x.K, x.N, steps, x.B, parts, too_small);
+    unsigned long long* const notes = reinterpret_cast<unsigned long long*>(static_cast<char*>(memory) + fragments * kFragmentBytes);
+    hipLaunchKernelGGL(split_dense_kernel, dim3((unsigned)ceil_div(fragments, 4)), dim3(256), 0, stream, x.K, x.N, steps, x.B, parts, notes);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     constexpr size_t lds = 2 * kBuffer;
-    static_assert(lds >= 4 * 32 * kWave * sizeof(double) + kRows * sizeof(int), "the sums of one way, and a word per row");
+    static_assert(lds >= kSumBytes + sizeof(EndLds), "what the kernel ends with");
     // (once per device, as spmm_resident_launch)
     static std::atomic<unsigned long long> allowed[2];
     int device = 0;
@@ -381,7 +498,7 @@ hipError_t spmm_tiles_launch(const SpmmArgs& x, void* memory, hipStream_t stream
     const int stream_rule = tuning().stream_results;
     const bool streaming = stream_rule < 0 ? (long long)x.M * x.N >= 1024 * 1024 : stream_rule != 0;  // (as dense_rows_window)
     hipLaunchKernelGGL(spmm_tiles_kernel, dim3((unsigned)blocks), dim3(kTileThreads), lds, stream, x.M, x.K, x.N, x.nnz, col_tiles, streaming ? 1 : 0,
-                       x.row_offsets, x.col_indices, x.values, x.B, parts, too_small, x.C);
+                       x.row_offsets, x.col_indices, x.values, x.B, parts, notes, x.C);
     return hipGetLastError();
 }
 

@@ -197,3 +197,45 @@ def test_one_plan_on_two_streams_and_in_a_graph():
         other = dl.spmm(*args, dense[1 - i], plan=plan)
         torch.cuda.synchronize()
         assert torch.equal(out, want[i]) and torch.equal(other, want[1 - i])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("what", ["a row", "scattered", "everything", "one column", "explicit zeros", "large"])
+@pytest.mark.parametrize("M,K,N,density", [SIZES[0], SIZES[2], SIZES[5]])
+def test_values_of_B_that_have_no_parts(what, M, K, N, density):
+    """Infinities, NaN and values that bf16 rounds to infinity reach the rows that use them, in the columns that hold them, as from
+    slices of B; all other results are what they are with zeros in their place."""
+    ro, ci, va, B, rng = matrix(M, K, N, density, 21)
+    bad = np.zeros(B.shape, bool)
+    if what in ("a row", "explicit zeros"):
+        bad[K - 2] = True
+    elif what == "scattered":
+        bad[rng.integers(0, K, 40), rng.integers(0, N, 40)] = True
+    elif what == "everything":
+        bad[:] = True
+    elif what == "one column":
+        bad[:, N - 1] = True
+    else:
+        bad[rng.integers(0, K, 5), rng.integers(0, N, 5)] = True
+    B[bad] = np.float32(3.4e38) if what == "large" else rng.choice(np.array([np.inf, -np.inf, np.nan, 3.4e38], np.float32), bad.sum(), p=[0.4, 0.3, 0.2, 0.1])
+    if what == "explicit zeros":
+        va[::3] = 0.0
+    elif what == "large":
+        va *= np.float32(0.1)  # (finite results)
+    with np.errstate(all="ignore"):
+        got, other = run(ro, ci, va, B)
+    fine = np.isfinite(other)
+    assert fine.any() == (what != "everything") and (what == "large" or not fine.all())
+    if what == "large":
+        assert fine.all() and np.isfinite(got).all()
+        off, norm = np.linalg.norm((got - other) / 1e38, axis=0), np.linalg.norm(other / 1e38, axis=0)
+        assert (off <= 3e-7 * norm + 1e-38).all()
+        return
+    # (a sum that overflows on the way only, from slices of B in 32 bits, is what it is in 64 bits here)
+    sums = ~fine & np.isfinite(got)
+    assert sums.sum() <= 1e-3 * got.size and np.array_equal(np.isfinite(got) & ~sums, fine)
+    assert np.array_equal(np.isnan(got[~sums]), np.isnan(other[~sums]))
+    infinite = np.isinf(other) & ~sums
+    assert np.array_equal(got[infinite], other[infinite])
+    small = fine & (np.abs(other) < 1e30)
+    assert np.linalg.norm(np.where(small, got - other, 0)) <= 3e-7 * np.linalg.norm(np.where(small, other, 0)) + 1e-38
