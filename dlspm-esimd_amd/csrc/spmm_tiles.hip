@@ -15,8 +15,9 @@
 //     their own. The two halves of the steps meet in LDS at the end.
 // Values of B that are not finite have zeros for parts and are added at the end, to the rows that use them (one NaN in B, 16384 x 8192,
 // N = 128 at 0.3: 1601 us while it went through the products and made every row of its column one to compute again, now 245).
-// Rows whose columns do not ascend, other results that are not finite, and values too small for their parts are computed once more
-// from the floats, row by row.
+// Rows whose columns do not ascend, other results that are not finite, and results that are not large against what values too small for
+// their parts may have lost are computed once more from the floats, row by row (three values of 1e-36 in every row of that matrix: 206
+// us; 1598 while every row with one was computed again).
 // Measured (us, three operand sets in turn, resident -> tiles): 32768 x 8192, N = 128 at 0.2 / 0.3 527 / 647 -> 392 / 420; 16384 x 8192 at 0.2 / 0.3 / 0.5
 // 266 / 327 / 496 -> 204 / 206 / 291; 4096 x 4096, N = 512 at 0.5 245 -> 134; 16384 x 2048, N = 256 at 0.3 173 -> 113; 2000 x 4608, N = 3136 at 0.3
 // 703 -> 440. Against 64 bits the results are off by 3.0 ... 3.4e-8, the resident schedule's by 6.9 ... 7.1e-8.
@@ -40,7 +41,8 @@ constexpr int kFragmentBytes = 3 * kWave * 16;
 // ---- B: split once, in the order in which the products read it: [strip of 32 columns][step][part][lane][8]
 // A value that is not finite, or that bf16 rounds to infinity, would make every result of its column NaN, through the zeros of A as
 // well: its parts are zeros, and the rows that have its column get it from the float (spmm_tiles_kernel). Per strip and step, in a word:
-// bits 0 ... 31 the columns with a nonzero value below 2^-109, 32 ... 47 the rows of B with a value that has no parts.
+// bits 0 ... 31 the columns with a nonzero value below 2^-109, 32 ... 47 the rows of B with a value that has no parts, 48 ... 55 the
+// exponent of the largest of the others.
 constexpr unsigned kTooLarge = 0xfeff0000u;  // twice the bits of a value, from this on: no parts
 __global__ __launch_bounds__(256) void split_dense_kernel(int K, int N, int steps, const float* __restrict__ B, bf16x8* __restrict__ parts,
                                                           unsigned long long* __restrict__ notes)
@@ -50,7 +52,7 @@ __global__ __launch_bounds__(256) void split_dense_kernel(int K, int N, int step
     const int strip = (int)(fragment / steps), step = (int)(fragment - (long long)strip * steps);
     if (strip * 32 >= N) return;
     const int n = strip * 32 + l, k0 = 16 * step + 8 * h;
-    float x[8];
+    float x[8], most = 0.f;
     unsigned without = 0;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
@@ -58,6 +60,7 @@ __global__ __launch_bounds__(256) void split_dense_kernel(int K, int N, int step
         const bool none = (__float_as_uint(x[j]) << 1) >= kTooLarge;
         without |= none ? 1u << j : 0u;
         x[j] = none ? 0.f : x[j];
+        most = fmaxf(most, fabsf(x[j]));
     }
     unsigned least;
     const Parts p = split_parts(x, least);
@@ -66,7 +69,9 @@ __global__ __launch_bounds__(256) void split_dense_kernel(int K, int N, int step
     to[kWave] = p.mid;
     to[2 * kWave] = p.lo;
     const unsigned long long few = __ballot(least < kTooSmall);
-    unsigned long long note = (unsigned)few | (unsigned)(few >> 32);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) most = fmaxf(most, __shfl_xor(most, o));
+    unsigned long long note = (unsigned)few | (unsigned)(few >> 32) | (unsigned long long)(__float_as_uint(most) >> 23) << 48;
     if (__ballot(without != 0) != 0)
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
@@ -86,7 +91,8 @@ constexpr int kAhead = 2;                                  // steps of B loaded 
 constexpr int kSumBytes = 4 * 32 * kWave * (int)sizeof(double), kLoad = 4 * kWave;
 struct EndLds {
     int again[kRows];  // the row is computed from the floats
-    unsigned without;  // some strip of the tile has values of B without parts
+    int tiny[kRows];   // ... has a value below 2^-109
+    unsigned without, few, most;  // some strip of the tile has values of B without parts, below 2^-109; the bits of the rows' largest value
 };
 constexpr int kMarkSteps = (kSumBytes - kRows * kCols * (int)sizeof(float)) / (int)sizeof(unsigned short);
 static_assert(kMarkSteps % kTileThreads == 0, "steps that share a mark are one thread's");
@@ -109,7 +115,7 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(2,
     const __amdgpu_buffer_rsrc_t values_buffer = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(values), 0, nnz * 4, 0x00020000);
     int p[2], e[2], n[2], at[2][4];
     u4 c[2], a[2];
-    bool wrong[2] = {false, false}, tiny = false;
+    bool wrong[2] = {false, false}, tiny[2] = {false, false};
     auto load_pairs = [&](int g) {
         const unsigned from = (unsigned)(p[g] + 4 * l16) * 4u;
         c[g] = __builtin_bit_cast(u4, __builtin_amdgcn_raw_buffer_load_b128(columns_buffer, from, 0, 0));
@@ -164,7 +170,7 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(2,
             py[kPartBytes] = (unsigned short)(lo >> 16);
             least = min(least, min((a[g][i] << 1) - 1u, (a[g][i + 1] << 1) - 1u));
         }
-        tiny |= least < kTooSmall;
+        tiny[g] |= least < kTooSmall;
     };
     auto clear = [&](int buffer) {
 #pragma unroll
@@ -277,48 +283,71 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(2,
         }
 #pragma unroll
         for (int g = 0; g < 2; ++g) {
-            const unsigned long long bad = __ballot(wrong[g] || tiny || p[g] < e[g]);
-            if (l16 == 0) end.again[own_row + 4 * g] = (bad >> (lane & 48) & 0xffff) != 0 ? 1 : 0;
+            const unsigned long long bad = __ballot(wrong[g] || p[g] < e[g]), few = __ballot(tiny[g]);
+            if (l16 == 0) {
+                end.again[own_row + 4 * g] = (bad >> (lane & 48) & 0xffff) != 0 ? 1 : 0;
+                end.tiny[own_row + 4 * g] = (few >> (lane & 48) & 0xffff) != 0 ? 1 : 0;
+            }
         }
-        if (t == 0) end.without = 0;
+        if (t == 0) end.without = end.few = end.most = 0;
         __syncthreads();
         const unsigned long long* const strip_notes = notes + (size_t)min(col0 / 32 + strip, (N - 1) / 32) * steps;
         unsigned few = 0;  // columns of the strip with a value of B that its parts do not hold
-        float bound = 0.f;
+        float bound = 0.f, bound_tiny = 0.f;
         if (way == 0) {
-            unsigned without = 0;
+            unsigned without = 0, exponent = 0;
             for (int i = lane; i < steps; i += kWave) {
                 const unsigned long long note = strip_notes[i];
                 few |= (unsigned)note;
                 without |= (unsigned)(note >> 32) & 0xffffu;
+                exponent = max(exponent, (unsigned)(note >> 48));
             }
 #pragma unroll
             for (int o = 32; o > 0; o >>= 1) {
                 few |= __shfl_xor(few, o);
                 without |= __shfl_xor(without, o);
+                exponent = max(exponent, (unsigned)__shfl_xor((int)exponent, o));
             }
-            if (lane == 0 && without != 0) end.without = 1;
+            if (lane == 0) {
+                if (few != 0) end.few = 1;
+                if (without != 0) end.without = 1;
+            }
             // A value below 2^-109 is off by 2^-134 at most in its parts: of no account for results from 2^34 times what that can come to on.
-            if (few != 0) {
-                float most = 0.f;
-                for (int i = row_offsets[row0] + lane; i < row_offsets[min(row0 + kRows, M)]; i += kWave) most = fmaxf(most, fabsf(values[i]));
-#pragma unroll
-                for (int o = 32; o > 0; o >>= 1) most = fmaxf(most, __shfl_xor(most, o));
-                bound = (float)K * most * 0x1p-100f;
-            }
+            bound_tiny = ldexpf((float)K, (int)exponent - 126 - 100);
 #pragma unroll
             for (int i = 0; i < 32; ++i) total[i / 16][i % 16] += sums[(strip * 32 + i) * kWave + lane];
         }
         __syncthreads();
+        if (end.few != 0) {  // (uniform) the largest value of the 64 rows
+            const int from = row_offsets[row0], to = row_offsets[min(row0 + kRows, M)];
+            unsigned most = 0;
+            for (int j = from + w * 2 * kLoad; j < to; j += kTileWaves * 2 * kLoad) {
+                u4 x[2];
+#pragma unroll
+                for (int q = 0; q < 2; ++q)
+                    x[q] = __builtin_bit_cast(u4, __builtin_amdgcn_raw_buffer_load_b128(values_buffer, (unsigned)(j + q * kLoad + 4 * lane) * 4u, 0, 0));
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const unsigned v = x[i / 4][i % 4] & 0x7fffffffu;  // (a row with an infinity has no finite result to be bounded)
+                    if (j + i / 4 * kLoad + 4 * lane + i % 4 < to && v < 0x7f800000u) most = max(most, v);
+                }
+            }
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) most = max(most, (unsigned)__shfl_xor((int)most, o));
+            if (lane == 0) __hip_atomic_fetch_max(&end.most, most, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            __syncthreads();
+            bound = (float)K * __uint_as_float(end.most) * 0x1p-100f;
+        }
         if (way == 0) {
 #pragma unroll
             for (int r = 0; r < 2; ++r) {
+                const float least_row = end.tiny[32 * r + l] != 0 ? bound_tiny : 0.f;
                 bool bad = false;
 #pragma unroll
                 for (int i = 0; i < 16; ++i) {
                     const float x = fabsf((float)total[r][i]);
                     const int n = 8 * (i / 4) + 4 * h + i % 4;
-                    const float least = (few >> n & 1) != 0 ? bound : 0.f;
+                    const float least = fmaxf(least_row, (few >> n & 1) != 0 ? bound : 0.f);
                     bad |= (col0 + 32 * strip + n < N) & !((x >= least) & (x < __builtin_inff()));
                 }
                 if (bad) end.again[32 * r + l] = 1;

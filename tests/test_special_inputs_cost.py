@@ -64,3 +64,16 @@ def test_spmm_values_of_B_that_are_not_finite(spmm_case, what):
     else:
         B[100] = float("inf")
     assert time_us(lambda: dl.spmm(ro, ci, values, B, plan=plan)) <= 1.6 * ordinary
+
+
+# nonzero values below 2^-109 (softmax weights among them): results that are large against what such values can lose stay as they are
+@pytest.mark.parametrize("what", ["three of A in every row", "every 50th row of B"])
+def test_spmm_values_too_small_for_their_parts(spmm_case, what):
+    ro, ci, values, B, plan, ordinary = spmm_case
+    if what == "three of A in every row":
+        values = values.clone()
+        values[::400] = 1e-36
+    else:
+        B = B.clone()
+        B[::50] = 1e-36
+    assert time_us(lambda: dl.spmm(ro, ci, values, B, plan=plan)) <= 1.4 * ordinary

@@ -239,3 +239,32 @@ def test_values_of_B_that_have_no_parts(what, M, K, N, density):
     assert np.array_equal(got[infinite], other[infinite])
     small = fine & (np.abs(other) < 1e30)
     assert np.linalg.norm(np.where(small, got - other, 0)) <= 3e-7 * np.linalg.norm(np.where(small, other, 0)) + 1e-38
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("small", [1e-33, 1e-36, 1e-44])
+@pytest.mark.parametrize("where", ["A", "B", "both", "A, results of few terms"])
+def test_values_too_small_for_their_parts(where, small):
+    """Values below 2^-109 lose up to 2^-134 in their parts, which no result may show: the large ones because they are large, the small
+    ones because they are computed from the floats."""
+    M, K, N, density = SIZES[2]
+    ro, ci, va, B, rng = matrix(M, K, N, density, 33)
+    if where != "B":
+        va[rng.random(ci.size) < 0.02] = small
+    if where in ("B", "both"):
+        B[rng.random(B.shape) < 0.02] = small
+    if where == "A, results of few terms":  # whole columns of results that only such values make
+        B[:, 7:40] = 0.0
+        B[3, 7:40] = rng.normal(size=33)
+        va[ci == 3] = np.where(rng.random((ci == 3).sum()) < 0.5, small, va[ci == 3])
+    got, other = run(ro, ci, va, B)
+    dense = np.zeros((M, K))
+    dense[np.repeat(np.arange(M), np.diff(ro)), ci] = va
+    want = dense @ B.astype(np.float64)
+    # every result by itself: rounded once, or 2^-22 of what its terms come to together, or half of the smallest float
+    terms = np.abs(dense) @ np.abs(B).astype(np.float64)
+    assert (np.abs(got - want) <= 2.0 ** -22 * terms + 2.0 ** -149).all()
+    few = (terms > 0) & (terms < 1e-30)
+    assert few.any() == (where == "A, results of few terms")
+    # (down to the smallest ones, which one term makes: exact but for the rounding of the product)
+    assert (np.abs(got - want)[few] <= 2.0 ** -23 * terms[few] + 2.0 ** -149).all()
