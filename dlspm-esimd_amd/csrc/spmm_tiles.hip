@@ -268,11 +268,10 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(2,
         __syncthreads();
     }
 
-    // (the thread's place once more: kept through the loop, it would be spilled)
-    int thread = threadIdx.x;
-    asm("" : "+v"(thread));
     {
-        const int t = thread, lane = t & 63, l = lane & 31, h = lane >> 5, l16 = lane & 15, own_row = 8 * w + (lane >> 4);
+        // (the thread's place once more: kept through the loop, it would be spilled)
+        const int lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), t = w * kWave + lane, l = lane & 31, h = lane >> 5, l16 = lane & 15;
+        const int own_row = 8 * w + (lane >> 4);
         // ---- the two ways' sums
         double* const sums = reinterpret_cast<double*>(shared);
         EndLds& end = *reinterpret_cast<EndLds*>(shared + kSumBytes);
