@@ -806,7 +806,8 @@ __device__ __forceinline__ void sddmm_rounds_load(int D, int g, const float* __r
 // (lanes past the chunk return an unspecified value that the caller must not store). `c` is the lane's
 // column index (0 past the chunk). `lq` holds the lhs row as laid out by the caller:
 // lq[s] = lhs_row[(s*G1 + g)*VEC ..] (Vec::gload_clip), zero past D. With DS = 0 the row is re-read from lhs_row.
-template <int VEC, int G1, int DS, int MASKED>
+// FLIGHT: accesses issued together (more than the usual eight where few waves share a SIMD).
+template <int VEC, int G1, int DS, int MASKED, int FLIGHT = 8>
 __device__ __forceinline__ float sddmm_chunk(int D, int lane, int cnt, int c, const float* __restrict__ lhs_row,
                                              const Vec<VEC>* lq, const float* __restrict__ rhs)
 {
@@ -817,7 +818,7 @@ __device__ __forceinline__ float sddmm_chunk(int D, int lane, int cnt, int c, co
     const int rounds = (cnt + P - 1) / P;  // <= G1
     float res = 0.f;
     if constexpr (DS > 0) {
-        constexpr int U = DS >= 8 ? 1 : 8 / DS;  // rounds whose loads are issued together
+        constexpr int U = DS >= FLIGHT ? 1 : FLIGHT / DS < G1 ? FLIGHT / DS : G1;  // rounds whose loads are issued together
         int t = 0;
         for (; t + U <= rounds; t += U) {
             VecT x[U][DS];

@@ -34,11 +34,12 @@ static inline SampledOut sampled_out(const SddmmArgs& x)
     return SampledOut{x.out, (forced < 0 ? by_rule : forced != 0) ? 1 : 0};
 }
 
-// out[j] = <lhs_row, rhs[col_indices[j]]> for the nonzeros j in [p, q) of one row (p < q, wave-uniform).
-template <int VEC, int G1, int DS, int MASKED, typename Out>
+// out[j] = <lhs_row, rhs[col_indices[j]]> for the nonzeros j in [p, q) of one row (p < q, wave-uniform), 64 at a time: all of
+// them, or (several waves in turn) every `step`-th 64.
+template <int VEC, int G1, int DS, int MASKED, int FLIGHT = 8, typename Out>
 __device__ __forceinline__ void sddmm_segment(int p, int q, int D, const int* __restrict__ col_indices,
                                               const float* __restrict__ lhs_row, const float* __restrict__ rhs,
-                                              Out out, int lane)
+                                              Out out, int lane, int step = 1)
 {
     using VecT = Vec<VEC>;
     const int g = lane % G1;
@@ -54,11 +55,11 @@ __device__ __forceinline__ void sddmm_segment(int p, int q, int D, const int* __
     // 64 column indices per pass, one per lane; the next 64 are requested (index clamped, no condition) before
     // the rhs rows of the current ones
     int c_nxt = col_indices[min(p + lane, q - 1)];
-    for (int base = p; base < q; base += kWave) {
+    for (int base = p; base < q; base += step * kWave) {
         const int c = base + lane < q ? c_nxt : 0;
-        c_nxt = col_indices[min(base + kWave + lane, q - 1)];
+        c_nxt = col_indices[min(base + step * kWave + lane, q - 1)];
         const int cnt = min(kWave, q - base);
-        const float o = sddmm_chunk<VEC, G1, DS, MASKED>(D, lane, cnt, c, lhs_row, lq, rhs);
+        const float o = sddmm_chunk<VEC, G1, DS, MASKED, FLIGHT>(D, lane, cnt, c, lhs_row, lq, rhs);
         if (base + lane < q) out.store(base + lane, o);
     }
 }

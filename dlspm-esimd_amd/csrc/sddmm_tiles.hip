@@ -10,6 +10,10 @@
 //     a prefix of them, and their results go to their slots. A row's position is carried from tile to tile; where a range does not
 //     begin with the row it is found by a binary search. Any position is a correct one: what a row has left at the end of a range,
 //     because its columns do not ascend, is computed as in sddmm.hip, and so are results that are not finite (dense_tiles.hpp).
+//   * Rows whose first 64 columns do not ascend are left out of the tiles. A workgroup that finds more than half of its rows to be
+//     such gathers all of them instead, otherwise its waves share them behind the tiles (us, gathering kernels / all rows shuffled /
+//     every sixteenth, at 8192 x 8192: D = 128 at 0.2 250 / 274 / 126, D = 64 at 0.2 125 / 137 / 78, D = 32 at 0.3 110 / 119 / 61; while the wave
+//     of such a row finished it alone: 1565 / 307, 654 / 158, 481 / 131; 2048 x 2048 at 0.3, D = 128, 24 / 31 / 16, was 187 / 62).
 //   * Up to D = 32 two workgroups share a compute unit, one sampling while the other computes. Above, the parts of lhs take the
 //     LDS of the second one, and the splits of a step of sixteen, the loads and the passage through LDS stand between the products
 //     of the step before it instead.
@@ -57,6 +61,8 @@ template <> struct Stage<0> {};
 template <int STAGES, int PARTS> struct __attribute__((aligned(16))) TileLds : Stage<STAGES> {
     float scores[kTileRows * kTileCols];
     bf16x8 lhs_parts[PARTS][kWave];
+    int first[kTileRows], end[kTileRows], done[kTileRows];  // nonzeros of the rows in the range of columns, and how far the tiles got
+    int unordered[kTileWaves];  // how many rows of a wave
 };
 
 struct ScaledOut {
@@ -117,12 +123,16 @@ __global__ __launch_bounds__(kTileWaves * 64) __attribute__((amdgpu_waves_per_eu
     load_rhs(0, 0);
 
     // ---- the rows' nonzeros in the range of columns
-    int* const bounds = reinterpret_cast<int*>(lds.scores);
+    const __amdgpu_buffer_rsrc_t columns = __builtin_amdgcn_make_buffer_rsrc(const_cast<int*>(col_indices), 0, nnz * 4, 0x00020000);
+    const int offsets = row_offsets[min(row0 + w * kRowsPerWave + min(lane, kRowsPerWave), M)];  // of the wave's rows
+    const int searched = min(row0 + (t & (kTileRows - 1)), M), from = row_offsets[searched], to = row_offsets[min(searched + 1, M)];
+    int leading[kRowsPerWave];
+#pragma unroll
+    for (int i = 0; i < kRowsPerWave; ++i)
+        leading[i] = __builtin_amdgcn_raw_buffer_load_b32(columns, (unsigned)(__builtin_amdgcn_readlane(offsets, i) + lane) * 4u, 0, 0);
     if (t < 2 * kTileRows) {
-        const int row = min(row0 + (t & (kTileRows - 1)), M);
-        const int from = row_offsets[row], to = row_offsets[min(row + 1, M)];
         const int column = t < kTileRows ? first_column : columns_end;
-        bounds[t] = column == 0 ? from : column >= K ? to : first_not_below(col_indices, from, to, column);
+        (t < kTileRows ? lds.first : lds.end)[t & (kTileRows - 1)] = column == 0 ? from : column >= K ? to : first_not_below(col_indices, from, to, column);
     }
     // ---- the parts of lhs: lane l holds row l % 32, floats 16 ks + 8 (l / 32) ... + 7
     auto split_lhs = [&](int row, int ks) {
@@ -146,14 +156,35 @@ __global__ __launch_bounds__(kTileWaves * 64) __attribute__((amdgpu_waves_per_eu
         const int i = 3 * (rt * KS + ks);
         return Parts{lds.lhs_parts[i][lane], lds.lhs_parts[i + 1][lane], lds.lhs_parts[i + 2][lane]};
     };
-    __syncthreads();
-    int p[kRowsPerWave], e[kRowsPerWave], begin[kRowsPerWave];
+    // Columns that do not ascend are told from the row's first 64, the same for every range of columns. Such rows (a bit each) are
+    // left out of the tiles; the ranges share them evenly.
+    int unordered = 0;
 #pragma unroll
     for (int i = 0; i < kRowsPerWave; ++i) {
-        begin[i] = p[i] = __builtin_amdgcn_readfirstlane(bounds[w * kRowsPerWave + i]);
-        e[i] = __builtin_amdgcn_readfirstlane(bounds[kTileRows + w * kRowsPerWave + i]);
+        const int length = __builtin_amdgcn_readlane(offsets, i + 1) - __builtin_amdgcn_readlane(offsets, i), next = __builtin_amdgcn_update_dpp(0, leading[i], 0x130, 0xf, 0xf, true);  // wave_shl:1
+        if (__ballot(lane < min(length, kWave) - 1 && leading[i] > next) != 0) unordered |= 1 << i;
     }
-    const __amdgpu_buffer_rsrc_t columns = __builtin_amdgcn_make_buffer_rsrc(const_cast<int*>(col_indices), 0, nnz * 4, 0x00020000);
+    if (lane == 0) lds.unordered[w] = __builtin_popcount(unordered);
+    __syncthreads();
+    const int length = lane_get(offsets, lane + 1) - offsets;
+    if (unordered != 0 && lane < kRowsPerWave && (unordered >> lane & 1)) {
+        const int ranges = (int)(gridDim.x / (unsigned)row_blocks), share = (length - 1) / ranges + 1;
+        lds.first[w * kRowsPerWave + lane] = offsets + min(share * range, length);
+        lds.end[w * kRowsPerWave + lane] = offsets + min(share * (range + 1), length);
+    }
+    const int my_first = lds.first[w * kRowsPerWave + (lane & (kRowsPerWave - 1))], my_end = lds.end[w * kRowsPerWave + (lane & (kRowsPerWave - 1))];
+    const int counts = lds.unordered[lane & (kTileWaves - 1)];
+    int p[kRowsPerWave], e[kRowsPerWave];
+#pragma unroll
+    for (int i = 0; i < kRowsPerWave; ++i) {
+        p[i] = __builtin_amdgcn_readlane(my_first, i);
+        e[i] = unordered >> i & 1 ? p[i] : __builtin_amdgcn_readlane(my_end, i);
+    }
+    int rows_unordered = 0;
+    if (__ballot(counts != 0) != 0)
+#pragma unroll
+        for (int i = 0; i < kTileWaves; ++i) rows_unordered += __builtin_amdgcn_readlane(counts, i);
+    const bool gather = rows_unordered > kTileRows / 2;  // (uniform) all rows are gathered: their tiles would cost more than they save
     int c[kRowsPerWave][kAhead];
     auto load_columns = [&](int i) {
 #pragma unroll
@@ -161,7 +192,6 @@ __global__ __launch_bounds__(kTileWaves * 64) __attribute__((amdgpu_waves_per_eu
     };
 #pragma unroll
     for (int i = 0; i < kRowsPerWave; ++i) load_columns(i);
-    __syncthreads();  // (`bounds` is read)
 
     // ---- the wave's part of a tile: 64 rows x 32 columns
     // the products of one step with the parts q0, q1 of the lhs rows 0 ... 31, 32 ... 63, smallest first; hi x hi into `sum`
@@ -320,7 +350,7 @@ __global__ __launch_bounds__(kTileWaves * 64) __attribute__((amdgpu_waves_per_eu
         }
     };
 
-    for (int tile = 0; tile < tiles; ++tile) {
+    for (int tile = 0; tile < (gather ? 0 : tiles); ++tile) {
         if constexpr (kTwoPerUnit) compute_short(tile);
         else compute_long(tile);
         __syncthreads();
@@ -328,26 +358,47 @@ __global__ __launch_bounds__(kTileWaves * 64) __attribute__((amdgpu_waves_per_eu
     }
 
     // ---- what is left: rows whose columns do not ascend, and results that are not finite
-    const bool again = __ballot(!(all_finite == 0.f)) != 0;
     const ScaledOut plain{out, scale};
-#pragma unroll 1
-    for (int i = 0; i < kRowsPerWave; ++i) {
-        int from = 0, done = 0, end = 0;
+    const int at_end = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));  // (the lane; kept through the loop, it would be spilled)
+    auto gathered = [&](int row, int from, int to, int step) {
+        sddmm_segment<4, 8, SEGMENTS, FULL ? kExactWidth : kMaskedBySelect, kTwoPerUnit ? 8 : 16>(from, to, D, col_indices, lhs + (size_t)(row0 + row) * D, rhs,
+                                                                                                 plain, at_end, step);
+    };
+    int left = 0;
 #pragma unroll
-        for (int j = 0; j < kRowsPerWave; ++j)
-            if (j == i) {
-                from = begin[j];
-                done = p[j];
-                end = e[j];
-            }
-        const float* lhs_row = lhs + (size_t)(row0 + w * kRowsPerWave + i) * D;
-        if (done < end) sddmm_segment<4, 8, 0, kMaskedBySelect>(done, end, D, col_indices, lhs_row, rhs, plain, lane);
-        if (!again) continue;
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");  // (this wave's own stores)
-        for (int at = from; at < done; at += kWave) {
-            const float x = out[min(at + lane, done - 1)];
-            if (__ballot(!(fabsf(x) < __builtin_inff())) != 0)
-                sddmm_segment<4, 8, 0, kMaskedBySelect>(at, min(at + kWave, done), D, col_indices, lhs_row, rhs, plain, lane);
+    for (int i = 0; i < kRowsPerWave; ++i) {
+        const int row = w * kRowsPerWave + i;
+        if (at_end == 0) lds.done[row] = (unordered >> i & 1) != 0 ? lds.first[row] : p[i];
+        left |= e[i] - p[i];
+    }
+    if ((rows_unordered | left) != 0) {
+        // all rows: whole ones, dealt to the waves of the row block's workgroups; some: each by all waves, 64 nonzeros in turn; rows
+        // that are found not to ascend on the way: by their own wave
+        const bool shared = rows_unordered != 0 && !gather;
+        if (shared) __syncthreads();
+        const unsigned ranges = gridDim.x / (unsigned)row_blocks, row = at_end;  // (a row per lane)
+        const int from = gather ? row_offsets[min(row0 + at_end, M)] : lds.done[row], to = gather ? row_offsets[min(row0 + at_end + 1, M)] : lds.end[row];
+        const bool mine = gather ? row % ranges == (unsigned)range && row / ranges % kTileWaves == (unsigned)w : shared || row / kRowsPerWave == (unsigned)w;
+        int turn = shared ? w : 0;
+        for (unsigned long long rows = __ballot(mine && from < to); rows != 0; rows &= rows - 1) {
+            const int at = __builtin_ctzll(rows), p_row = __builtin_amdgcn_readlane(from, at), e_row = __builtin_amdgcn_readlane(to, at);
+            const int own = p_row + turn * kWave;
+            // (the lines of its columns, all at once)
+            const int touched = gather ? col_indices[min(own + 32 * at_end, e_row - 1)] : 0;
+            if (own < e_row) gathered(at, own, e_row, shared ? kTileWaves : 1);
+            asm volatile("" : : "v"(touched));
+            if (shared) turn = (turn - (e_row - p_row + kWave - 1) / kWave) & (kTileWaves - 1);
+        }
+        if (gather) return;
+    }
+    if (__ballot(!(all_finite == 0.f)) == 0) return;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");  // (this wave's own stores)
+#pragma unroll 1
+    for (int row = w * kRowsPerWave; row < (w + 1) * kRowsPerWave; ++row) {
+        const int done = __builtin_amdgcn_readfirstlane(lds.done[row]);
+        for (int at = __builtin_amdgcn_readfirstlane(lds.first[row]); at < done; at += kWave) {
+            const float x = out[min(at + at_end, done - 1)];
+            if (__ballot(!(fabsf(x) < __builtin_inff())) != 0) gathered(row, at, min(at + kWave, done), 1);
         }
     }
 }

@@ -157,3 +157,28 @@ def test_the_same_bits_whatever_comes_with_the_call(torch_cuda):
     # operands on any float
     shifted = torch.empty(lhs.numel() + 1, device="cuda")[1:].view(M, D).copy_(lhs), torch.empty(rhs.numel() + 3, device="cuda")[3:].view(K, D).copy_(rhs)
     assert torch.equal(dl.sddmm(ro, ci, *shifted), first)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K,D,density", [(4096, 4096, 32, 0.9), (1500, 2300, 64, 0.9), (1000, 2000, 127, 0.9), (300, 30000, 100, 0.4), (40000, 300, 128, 0.5)])
+@pytest.mark.parametrize("kind", ["a tenth of the rows", "every row", "behind the first 64", "one row in four, descending"])
+def test_how_many_rows_ascend(torch_cuda, M, K, D, density, kind):
+    """Few rows that do not ascend are shared by the waves behind the tiles, more than half of a tile's are gathered in its place, and
+    rows found out on the way are finished by their wave: every nonzero once, with several ranges of columns too."""
+    torch = torch_cuda
+    ro, ci, row = mask(torch, M, K, density, 13)
+    lhs, rhs = operands(torch, M, K, D, 14)
+    at = torch.arange(ci.numel(), device="cuda")
+    first, end = ro[:-1].long()[row], ro[1:].long()[row]
+    if kind == "one row in four, descending":
+        ci = torch.where(row % 4 == 1, ci[first + end - 1 - at], ci)
+    else:
+        some = row % 10 == 3 if kind == "a tenth of the rows" else at - first >= 64 if kind == "behind the first 64" else row >= 0
+        key = torch.where(some, torch.rand(ci.numel(), device="cuda", dtype=torch.float64) * 0.4 + 0.1, (at - first).double() * 1e-9)
+        ci = ci[(row.double() + key).argsort()]
+    on, off = both(torch, ro, ci.contiguous(), lhs, rhs)
+    want = exact(torch, lhs, rhs, row, ci)
+    terms = exact(torch, lhs.abs(), rhs.abs(), row, ci)
+    assert bool(((on.double() - want).abs() <= 2.0 ** -22 * terms).all())
+    # (a row's last nonzeros and its neighbour's first ones are written by different waves: none into the other's)
+    assert bool(((on - off).abs() <= 2.0 ** -21 * terms).all())
