@@ -5,9 +5,9 @@
 // in 32 bits and do 16 times the multiplications per clock that they do in fp32: six for one is still 2.7 times the fp32 rate.
 // Errors against 64 bits, operands of normal distribution, the sums' order as in the kernels: dot products of 32 / 64 / 128
 // 3.8e-8 / 5.0e-8 / 5.0e-8, eight chains of fp32 fma 6.2e-8 / 7.2e-8 / 8.8e-8 (2.5e-8: rounded once).
-// What the parts cannot hold shows in the result: an infinity, a NaN or a value that rounds to infinity in bf16 makes it NaN or
-// infinite, and so does a nonzero value below 2^-109, whose last part would be below bf16's smallest: it is replaced by NaN.
-// The kernels compute results that are not finite once more, row by row, from the floats themselves.
+// What the parts cannot hold: an infinity, a NaN or a value that rounds to infinity in bf16 makes the result NaN or infinite, and the
+// last part of a nonzero value below 2^-109 would be below bf16's smallest, which loses up to 2^-134 of it. The kernels compute
+// results that are not finite, and those that are not large against what such values can lose, from the floats themselves.
 #pragma once
 
 #include "common.hpp"
@@ -42,15 +42,12 @@ __device__ __forceinline__ Parts split_parts(const float* x, unsigned& least)
     }
     return Parts{__builtin_bit_cast(bf16x8, hi), __builtin_bit_cast(bf16x8, mid), __builtin_bit_cast(bf16x8, lo)};
 }
-// ... with NaN in the place of a part where a value is too small
-__device__ __forceinline__ Parts split_parts(const float* x)
+// ... and the lanes with a value that is too small among those of `few`
+__device__ __forceinline__ Parts split_parts(const float* x, unsigned long long& few)
 {
-    typedef unsigned u4 __attribute__((ext_vector_type(4)));
     unsigned least;
-    Parts p = split_parts(x, least);
-    u4 hi = __builtin_bit_cast(u4, p.hi);
-    hi[0] = least < kTooSmall ? 0x7fc07fc0u : hi[0];
-    p.hi = __builtin_bit_cast(bf16x8, hi);
+    const Parts p = split_parts(x, least);
+    few |= __ballot(least < kTooSmall);
     return p;
 }
 

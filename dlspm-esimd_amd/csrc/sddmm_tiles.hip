@@ -10,10 +10,13 @@
 //     a prefix of them, and their results go to their slots. A row's position is carried from tile to tile; where a range does not
 //     begin with the row it is found by a binary search. Any position is a correct one: what a row has left at the end of a range,
 //     because its columns do not ascend, is computed as in sddmm.hip, and so are results that are not finite (dense_tiles.hpp).
-//   * Rows whose first 64 columns do not ascend are left out of the tiles. A workgroup that finds more than half of its rows to be
+//   * Rows whose first 64 columns do not ascend, and rows of lhs with a nonzero value below 2^-109, are left out of the tiles. A workgroup that finds more than half of its rows to be
 //     such gathers all of them instead, otherwise its waves share them behind the tiles (us, gathering kernels / all rows shuffled /
 //     every sixteenth, at 8192 x 8192: D = 128 at 0.2 250 / 274 / 126, D = 64 at 0.2 125 / 137 / 78, D = 32 at 0.3 110 / 119 / 61; while the wave
 //     of such a row finished it alone: 1565 / 307, 654 / 158, 481 / 131; 2048 x 2048 at 0.3, D = 128, 24 / 31 / 16, was 187 / 62).
+//   * Such a value in a row of rhs is noted for the end, where results of its column that are small enough to show what its parts lost,
+//     and results that are not finite, are gathered: a value of 1e-36 in every row of rhs takes the three from 104 / 66 / 56 to 133 / 92 /
+//     80 us (1175 / 605 / 388 while its parts were NaN and every result of the column was computed again).
 //   * Up to D = 32 two workgroups share a compute unit, one sampling while the other computes. Above, the parts of lhs take the
 //     LDS of the second one, and the splits of a step of sixteen, the loads and the passage through LDS stand between the products
 //     of the step before it instead.
@@ -38,6 +41,7 @@ namespace dlspm {
 constexpr int kTileWaves = 8, kTileRows = 64, kTileCols = 32 * kTileWaves;
 constexpr int kRowsPerWave = kTileRows / kTileWaves;
 constexpr int kAhead = 2;  // columns of a row loaded ahead, times 64
+constexpr int kFewWords = 32 * kTileWaves;
 
 // Element (row, col) of a tile lies at row * kTileCols + (col ^ turned(row)): eight lanes that write four columns each of eight
 // rows fall on all banks
@@ -56,13 +60,16 @@ __device__ __forceinline__ int first_not_below(const int* __restrict__ col_indic
     return p;
 }
 
+// (in front of the scores: an LDS access holds an offset of 64 KiB, and behind them every part would take an address register of its own)
+template <int PARTS> struct LhsParts { bf16x8 lhs_parts[PARTS][kWave]; };
 template <int N> struct Stage { float stage[N][32 * 32]; };
 template <> struct Stage<0> {};
-template <int STAGES, int PARTS> struct __attribute__((aligned(16))) TileLds : Stage<STAGES> {
+template <int STAGES, int PARTS> struct __attribute__((aligned(16))) TileLds : LhsParts<PARTS>, Stage<STAGES> {
     float scores[kTileRows * kTileCols];
-    bf16x8 lhs_parts[PARTS][kWave];
     int first[kTileRows], end[kTileRows], done[kTileRows];  // nonzeros of the rows in the range of columns, and how far the tiles got
-    int unordered[kTileWaves];  // how many rows of a wave
+    unsigned long long apart[kTileWaves];  // rows that each wave has found to be none for the tiles
+    unsigned few[kFewWords];               // columns of the range, modulo 32 kFewWords, whose row of rhs has a value below 2^-109
+    int any_few;
 };
 
 struct ScaledOut {
@@ -135,19 +142,19 @@ __global__ __launch_bounds__(kTileWaves * 64) __attribute__((amdgpu_waves_per_eu
         (t < kTileRows ? lds.first : lds.end)[t & (kTileRows - 1)] = column == 0 ? from : column >= K ? to : first_not_below(col_indices, from, to, column);
     }
     // ---- the parts of lhs: lane l holds row l % 32, floats 16 ks + 8 (l / 32) ... + 7
-    auto split_lhs = [&](int row, int ks) {
-        const float* from = lhs + (size_t)min(row0 + row, M - 1) * D;
+    unsigned long long apart = 0;
+    for (int i = w; i < 2 * KS; i += kTileWaves) {
+        const float* from = lhs + (size_t)min(row0 + 32 * (i / KS) + l, M - 1) * D;
         float x[8];
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
-            const int d = 16 * ks + 8 * h + 4 * q;
+            const int d = 16 * (i % KS) + 8 * h + 4 * q;
             const Vec<4> v = FULL ? Vec<4>::gload(from + d) : d < D ? Vec<4>::gload_clip(from, d, D) : Vec<4>::zero();
             x[4 * q] = v.v.x, x[4 * q + 1] = v.v.y, x[4 * q + 2] = v.v.z, x[4 * q + 3] = v.v.w;
         }
-        return split_parts(x);
-    };
-    for (int i = w; i < 2 * KS; i += kTileWaves) {
-        const Parts q = split_lhs(32 * (i / KS) + l, i % KS);
+        unsigned long long few = 0;
+        const Parts q = split_parts(x, few);
+        apart |= (unsigned long long)((unsigned)few | (unsigned)(few >> 32)) << 32 * (i / KS);
         lds.lhs_parts[3 * i + 0][lane] = q.hi;
         lds.lhs_parts[3 * i + 1][lane] = q.mid;
         lds.lhs_parts[3 * i + 2][lane] = q.lo;
@@ -156,35 +163,41 @@ __global__ __launch_bounds__(kTileWaves * 64) __attribute__((amdgpu_waves_per_eu
         const int i = 3 * (rt * KS + ks);
         return Parts{lds.lhs_parts[i][lane], lds.lhs_parts[i + 1][lane], lds.lhs_parts[i + 2][lane]};
     };
-    // Columns that do not ascend are told from the row's first 64, the same for every range of columns. Such rows (a bit each) are
-    // left out of the tiles; the ranges share them evenly.
+    // Rows that are left out of the tiles: those whose columns do not ascend, told by the first 64, and rows of lhs with a value below
+    // 2^-109. Every range of columns comes to the same ones; they share their nonzeros evenly.
     int unordered = 0;
 #pragma unroll
     for (int i = 0; i < kRowsPerWave; ++i) {
-        const int length = __builtin_amdgcn_readlane(offsets, i + 1) - __builtin_amdgcn_readlane(offsets, i), next = __builtin_amdgcn_update_dpp(0, leading[i], 0x130, 0xf, 0xf, true);  // wave_shl:1
+        const int length = __builtin_amdgcn_readlane(offsets, i + 1) - __builtin_amdgcn_readlane(offsets, i);
+        const int next = __builtin_amdgcn_update_dpp(0, leading[i], 0x130, 0xf, 0xf, true);  // wave_shl:1
         if (__ballot(lane < min(length, kWave) - 1 && leading[i] > next) != 0) unordered |= 1 << i;
     }
-    if (lane == 0) lds.unordered[w] = __builtin_popcount(unordered);
+    if (lane == 0) lds.apart[w] = apart | (unsigned long long)unordered << w * kRowsPerWave;
+    if (t < kFewWords) lds.few[t] = 0;
+    if (t == 0) lds.any_few = 0;
     __syncthreads();
-    const int length = lane_get(offsets, lane + 1) - offsets;
-    if (unordered != 0 && lane < kRowsPerWave && (unordered >> lane & 1)) {
-        const int ranges = (int)(gridDim.x / (unsigned)row_blocks), share = (length - 1) / ranges + 1;
-        lds.first[w * kRowsPerWave + lane] = offsets + min(share * range, length);
-        lds.end[w * kRowsPerWave + lane] = offsets + min(share * (range + 1), length);
+    const unsigned long long found = lds.apart[lane & (kTileWaves - 1)];
+    apart = 0;
+    if (__ballot(found != 0) != 0) {
+#pragma unroll
+        for (int i = 0; i < kTileWaves; ++i)
+            apart |= (unsigned)__builtin_amdgcn_readlane((int)found, i) | (unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(found >> 32), i) << 32;
+        const int length = lane_get(offsets, lane + 1) - offsets, row = w * kRowsPerWave + (lane & (kRowsPerWave - 1));
+        if (lane < kRowsPerWave && (apart >> row & 1) != 0) {
+            const int ranges = (int)(gridDim.x / (unsigned)row_blocks), share = (length - 1) / ranges + 1;
+            lds.first[row] = offsets + min(share * range, length);
+            lds.end[row] = offsets + min(share * (range + 1), length);
+        }
     }
+    const unsigned mine_apart = (unsigned)(apart >> w * kRowsPerWave) & ((1u << kRowsPerWave) - 1);
     const int my_first = lds.first[w * kRowsPerWave + (lane & (kRowsPerWave - 1))], my_end = lds.end[w * kRowsPerWave + (lane & (kRowsPerWave - 1))];
-    const int counts = lds.unordered[lane & (kTileWaves - 1)];
     int p[kRowsPerWave], e[kRowsPerWave];
 #pragma unroll
     for (int i = 0; i < kRowsPerWave; ++i) {
         p[i] = __builtin_amdgcn_readlane(my_first, i);
-        e[i] = unordered >> i & 1 ? p[i] : __builtin_amdgcn_readlane(my_end, i);
+        e[i] = mine_apart >> i & 1 ? p[i] : __builtin_amdgcn_readlane(my_end, i);
     }
-    int rows_unordered = 0;
-    if (__ballot(counts != 0) != 0)
-#pragma unroll
-        for (int i = 0; i < kTileWaves; ++i) rows_unordered += __builtin_amdgcn_readlane(counts, i);
-    const bool gather = rows_unordered > kTileRows / 2;  // (uniform) all rows are gathered: their tiles would cost more than they save
+    const bool gather = __builtin_popcountll(apart) > kTileRows / 2;  // (uniform) all rows are gathered: their tiles would cost more than they save
     int c[kRowsPerWave][kAhead];
     auto load_columns = [&](int i) {
 #pragma unroll
@@ -219,6 +232,12 @@ __global__ __launch_bounds__(kTileWaves * 64) __attribute__((amdgpu_waves_per_eu
                 *reinterpret_cast<float4*>(lds.scores + (32 * rt + l) * kTileCols + 32 * w + ((8 * q + 4 * h) ^ turned(l))) =
                     make_float4(sum[rt][4 * q], sum[rt][4 * q + 1], sum[rt][4 * q + 2], sum[rt][4 * q + 3]);
     };
+    // the lanes whose rows of rhs have a value below 2^-109, for the end
+    auto note_few = [&](int tile, unsigned long long few) {
+        if (few == 0) return;
+        lds.few[(tile * kTileWaves + w) % kFewWords] |= (unsigned)few | (unsigned)(few >> 32);
+        lds.any_few = 1;
+    };
     // D <= 32: the small products of both steps come first, in one accumulator
     auto compute_short = [&](int tile) {
         f32x16 sum[2] = {};
@@ -227,11 +246,12 @@ __global__ __launch_bounds__(kTileWaves * 64) __attribute__((amdgpu_waves_per_eu
         load_rhs(tile + 1, 0);
         Parts r[2];
         float x[2][8];
+        unsigned long long few = 0;
         get(x[0], 0);
         get(x[1], 1);
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) {
-            r[ks] = split_parts(x[ks]);
+            r[ks] = split_parts(x[ks], few);
             multiply(r[ks], lhs_at(0, ks), lhs_at(1, ks), sum, nullptr);
         }
 #pragma unroll
@@ -240,22 +260,26 @@ __global__ __launch_bounds__(kTileWaves * 64) __attribute__((amdgpu_waves_per_eu
             for (int rt = 0; rt < 2; ++rt) sum[rt] = mfma(r[ks].hi, lhs_at(rt, ks).hi, sum[rt]);
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         write_scores(sum);
+        note_few(tile, few);
     };
     // D > 32: `ready` and `of_lhs` are the parts of the step at hand, `next` the floats of the one after it. Between the products
     // stand the split of the next step, the segment after it on its way through LDS, and the loads of the one behind that
     Parts ready, of_lhs[2];
+    unsigned long long few_ahead = 0;
     float next[8];
     if constexpr (!kTwoPerUnit) {
         put();
         float x[8];
         get(x, 0);
         get(next, 1);
-        ready = split_parts(x);
+        ready = split_parts(x, few_ahead);
         of_lhs[0] = lhs_at(0, 0), of_lhs[1] = lhs_at(1, 0);
         load_rhs(0, 1);
     }
     auto compute_long = [&](int tile) {
         f32x16 small[2] = {}, sum[2] = {};
+        unsigned long long few = few_ahead;
+        few_ahead = 0;
 #pragma unroll
         for (int s = 0; s < SEGMENTS; ++s) {
             float staged[2][8];
@@ -268,10 +292,10 @@ __global__ __launch_bounds__(kTileWaves * 64) __attribute__((amdgpu_waves_per_eu
                     put();
                     get(staged[0], 0);
                     get(staged[1], 1);
-                    ready = split_parts(next);
+                    ready = split_parts(next, few);
                     load_rhs(tile + (s + 2) / SEGMENTS, (s + 2) % SEGMENTS);
                 } else {
-                    ready = split_parts(staged[0]);
+                    ready = split_parts(staged[0], s + 1 < SEGMENTS ? few : few_ahead);
 #pragma unroll
                     for (int i = 0; i < 8; ++i) next[i] = staged[1][i];
                 }
@@ -289,6 +313,7 @@ __global__ __launch_bounds__(kTileWaves * 64) __attribute__((amdgpu_waves_per_eu
         sum[1] += small[1];
         __syncthreads();  // (the previous tile has been read)
         write_scores(sum);
+        note_few(tile, few);
     };
 
     // ---- the sampled ones. All reads, then all loads for the next tile, then all stores: loads and stores complete in order
@@ -368,13 +393,13 @@ __global__ __launch_bounds__(kTileWaves * 64) __attribute__((amdgpu_waves_per_eu
 #pragma unroll
     for (int i = 0; i < kRowsPerWave; ++i) {
         const int row = w * kRowsPerWave + i;
-        if (at_end == 0) lds.done[row] = (unordered >> i & 1) != 0 ? lds.first[row] : p[i];
+        if (at_end == 0) lds.done[row] = (mine_apart >> i & 1) != 0 ? lds.first[row] : p[i];
         left |= e[i] - p[i];
     }
-    if ((rows_unordered | left) != 0) {
+    if (apart != 0 || left != 0) {
         // all rows: whole ones, dealt to the waves of the row block's workgroups; some: each by all waves, 64 nonzeros in turn; rows
         // that are found not to ascend on the way: by their own wave
-        const bool shared = rows_unordered != 0 && !gather;
+        const bool shared = apart != 0 && !gather;
         if (shared) __syncthreads();
         const unsigned ranges = gridDim.x / (unsigned)row_blocks, row = at_end;  // (a row per lane)
         const int from = gather ? row_offsets[min(row0 + at_end, M)] : lds.done[row], to = gather ? row_offsets[min(row0 + at_end + 1, M)] : lds.end[row];
@@ -391,14 +416,46 @@ __global__ __launch_bounds__(kTileWaves * 64) __attribute__((amdgpu_waves_per_eu
         }
         if (gather) return;
     }
-    if (__ballot(!(all_finite == 0.f)) == 0) return;
+    // Parts of values below 2^-109 are off by 2^-134 at most, which does not show in a result from 2^34 times what that can come to on:
+    // smaller ones of such a column are gathered too.
+    const bool any_few = __builtin_amdgcn_readfirstlane(lds.any_few) != 0;
+    if (__ballot(!(all_finite == 0.f)) == 0 && !any_few) return;
+    float bound = 0.f;
+    if (any_few) {
+        unsigned most = 0;
+#pragma unroll 1
+        for (int i = 0; i < 2 * KS; ++i) {
+            const uint4 hi = __builtin_bit_cast(uint4, lds.lhs_parts[3 * i][at_end]);
+            for (unsigned x : {hi.x, hi.x << 16, hi.y, hi.y << 16, hi.z, hi.z << 16, hi.w, hi.w << 16}) {
+                x &= 0x7fff0000u;
+                most = max(most, x < 0x7f800000u ? x : 0u);
+            }
+        }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) most = max(most, (unsigned)__shfl_xor((int)most, o));
+        bound = (float)D * __uint_as_float(most) * 0x1p-99f * fabsf(scale);
+    }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");  // (this wave's own stores)
+    constexpr int kLoads = 4;
 #pragma unroll 1
     for (int row = w * kRowsPerWave; row < (w + 1) * kRowsPerWave; ++row) {
         const int done = __builtin_amdgcn_readfirstlane(lds.done[row]);
-        for (int at = __builtin_amdgcn_readfirstlane(lds.first[row]); at < done; at += kWave) {
-            const float x = out[min(at + at_end, done - 1)];
-            if (__ballot(!(fabsf(x) < __builtin_inff())) != 0) gathered(row, at, min(at + kWave, done), 1);
+        for (int at = __builtin_amdgcn_readfirstlane(lds.first[row]); at < done; at += kLoads * kWave) {
+            float x[kLoads];
+            int column[kLoads];
+            unsigned bad = 0;
+#pragma unroll
+            for (int q = 0; q < kLoads; ++q) {
+                x[q] = out[min(at + q * kWave + at_end, done - 1)];
+                column[q] = col_indices[min(at + q * kWave + at_end, done - 1)];
+            }
+#pragma unroll
+            for (int q = 0; q < kLoads; ++q) {
+                const unsigned of_few = lds.few[((unsigned)(column[q] - first_column) >> 5) % kFewWords] >> (column[q] - first_column & 31) & 1;
+                const float least = of_few != 0 ? bound : 0.f;
+                bad |= (__ballot(!(fabsf(x[q]) >= least && fabsf(x[q]) < __builtin_inff())) != 0 ? 1u : 0u) << q;
+            }
+            if (bad != 0) gathered(row, at + __builtin_ctz(bad) * kWave, min(at + (32 - __builtin_clz(bad)) * kWave, done), 1);
         }
     }
 }

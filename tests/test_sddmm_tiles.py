@@ -182,3 +182,53 @@ def test_how_many_rows_ascend(torch_cuda, M, K, D, density, kind):
     assert bool(((on.double() - want).abs() <= 2.0 ** -22 * terms).all())
     # (a row's last nonzeros and its neighbour's first ones are written by different waves: none into the other's)
     assert bool(((on - off).abs() <= 2.0 ** -21 * terms).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K,D,density", [(4096, 4096, 32, 0.9), (16448, 9000, 32, 0.3), (1500, 2300, 64, 0.9), (1000, 2000, 127, 0.9), (300, 30000, 100, 0.4)])
+@pytest.mark.parametrize("small", [1e-33, 1e-36, 1e-44])
+@pytest.mark.parametrize("where", ["rhs", "lhs", "both", "rhs, results of few terms"])
+def test_values_too_small_for_their_parts(torch_cuda, M, K, D, density, small, where):
+    """Values below 2^-109: rows of lhs with one are gathered, results of a row of rhs with one unless they are large against what its
+    parts may have lost. Every result by itself, the smallest ones too."""
+    torch = torch_cuda
+    ro, ci, row = mask(torch, M, K, density, 23)
+    lhs, rhs = operands(torch, M, K, D, 24)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(25)
+    few = lambda n: torch.rand((n, D), device="cuda", generator=g) < 0.004  # noqa: E731
+    if where != "rhs" and not where.endswith("terms"):
+        lhs[few(M)] = small
+    if where != "lhs":
+        rhs[few(K)] = small
+    if where.endswith("terms"):  # columns whose results are made by such a value alone, in one row of lhs out of three by nothing
+        rhs[5::19] = 0.0
+        rhs[5::19, 3] = small
+        lhs[::3, 3] = 0.0
+    on, off = both(torch, ro, ci, lhs, rhs)
+    want, terms = exact(torch, lhs, rhs, row, ci), exact(torch, lhs.abs(), rhs.abs(), row, ci)
+    # (the gathering kernels round to multiples of 2^-149 as often as there are products)
+    assert bool(((on.double() - want).abs() <= 2.0 ** -22 * terms + D * 2.0 ** -149).all())
+    alone = (terms > 0) & (terms < 1e-30)
+    assert bool(alone.any()) == where.endswith("terms")
+    assert bool(((on.double() - want).abs()[alone] <= 2.0 ** -23 * terms[alone] + 2.0 ** -149).all())
+    assert error(on, want) <= 1.02 * error(off, want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K,D,density", [(4096, 4096, 32, 0.9), (1500, 2300, 64, 0.9)])
+def test_results_that_are_not_finite_run_by_run(torch_cuda, M, K, D, density):
+    """What is gathered again is the run of 64s between the first and the last result that asks for it, of 256: at the ends of rows, of
+    ranges and of such runs."""
+    torch = torch_cuda
+    ro, ci, row = mask(torch, M, K, density, 33)
+    lhs, rhs = operands(torch, M, K, D, 34)
+    columns = torch.tensor([0, 63, 64, 255, 256, 700, K - 1], device="cuda")
+    rhs[columns] = torch.tensor([1.0, float("inf"), float("nan"), 3.4e38, 1.0, float("-inf"), float("nan")], device="cuda")[:, None]
+    rhs[columns, 1:] = rhs[columns, 1:] * torch.sign(operands(torch, 7, 7, D - 1, 35)[0])
+    lhs[::7] = float("nan")
+    on, off = both(torch, ro, ci, lhs, rhs)
+    assert bool((on.isnan() == off.isnan()).all())
+    assert bool((on[on.isinf()] == off[on.isinf()]).all()) and bool((on.isinf() == off.isinf()).all())
+    fine = on.isfinite()
+    assert float((on - off)[fine].norm() / off[fine].norm()) <= 1e-6

@@ -102,3 +102,21 @@ def test_sddmm_columns_that_do_not_ascend(D, density):
     gathered = time_us(lambda: dl.sddmm(ro, all_, lhs, rhs))
     dl.set_tuning()
     assert took <= 1.35 * gathered
+
+
+# the gathering kernels' times are the bound: 250 / 125 / 110 us
+@pytest.mark.parametrize("D,density", [(32, 0.3), (64, 0.2), (128, 0.2)])
+@pytest.mark.parametrize("what", ["a tiny value in every row of rhs", "one NaN in rhs", "a tiny value in every row of lhs"])
+def test_sddmm_values_without_parts(D, density, what):
+    M = K = 8192
+    ro, ci, row = mask(M, K, density, 3)
+    lhs, rhs = normal(M, D), normal(K, D)
+    if what == "one NaN in rhs":
+        rhs[100, 3] = float("nan")
+    else:
+        (rhs if what.endswith("rhs") else lhs)[:, 5] = 1e-36
+    took = time_us(lambda: dl.sddmm(ro, ci, lhs, rhs))
+    dl.set_tuning(rules_off=dl.RULES["dense_groups"])
+    gathered = time_us(lambda: dl.sddmm(ro, ci, lhs, rhs))
+    dl.set_tuning()
+    assert took <= (1.35 if what.endswith("lhs") else 1.0) * gathered
