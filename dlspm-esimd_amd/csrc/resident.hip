@@ -146,6 +146,40 @@ __device__ __forceinline__ void resident_part_chunk(const char* tiles, const int
     (void)(resident_lane<L>(tiles, at, lane_bytes, a, sum, lanes) && ...);
 }
 
+// What is left of a wave's four rows, sixteen lanes each, whose columns do not ascend: from memory, in CSR order, in 64 bits. Sixteen
+// pairs of a row at a time and eight of their rows of B on their way together (16384 x 8192 at density 0.3, N = 128, all rows shuffled: 2962
+// -> 1149 us; one nonzero after the other before). Written with selects and without a branch around it: either made the compiler order
+// the loop over the slices for fewer registers, 3 ... 4 % slower.
+template <int... L>
+__device__ __forceinline__ void gather_rest(int p, int end, int l, int N, const int* __restrict__ col_indices, const float* __restrict__ values,
+                                            const float* __restrict__ B, RowSum& sum, std::integer_sequence<int, L...>)
+{
+    auto pair = [&](int j) { return max(min(j + l, end - 1), 0); };
+    int column = col_indices[pair(p)];
+    float value = values[pair(p)];
+    for (; __ballot(p < end) != 0; p += 16) {
+        const int c = column;
+        const float a = value;
+        column = col_indices[pair(p + 16)];
+        value = values[pair(p + 16)];
+        auto some = [&](auto first) {  // eight of the sixteen
+            constexpr int kFirst = decltype(first)::value;
+            const Vec<4> b[] = {Vec<4>::gload(B + (size_t)row_bcast<kFirst + L>(c) * N)...};
+            auto add = [&](int i, float v) {
+                const bool in = p + kFirst + i < end;
+                sum.x = in ? fma((double)v, (double)b[i].v.x, sum.x) : sum.x;
+                sum.y = in ? fma((double)v, (double)b[i].v.y, sum.y) : sum.y;
+                sum.z = in ? fma((double)v, (double)b[i].v.z, sum.z) : sum.z;
+                sum.w = in ? fma((double)v, (double)b[i].v.w, sum.w) : sum.w;
+            };
+            (add(L, __int_as_float(row_bcast<kFirst + L>(__float_as_int(a)))), ...);
+        };
+        some(std::integral_constant<int, 0>{});
+        __builtin_amdgcn_sched_barrier(0);  // (eight rows of B take the registers there are)
+        some(std::integral_constant<int, 8>{});
+    }
+}
+
 // QC: chunks of 64 pairs of a row that are loaded ahead (a slice's share of a row is to fit them: what exceeds it is loaded
 // when it is needed, with nothing to hide the latency behind). CHAINS: see ChunkSum.
 template <int RR, int QC, int CHAINS>
@@ -340,20 +374,15 @@ __global__ __launch_bounds__(kResidentThreads) void spmm_resident_kernel(int M, 
         __syncthreads();
     }
 
+    // (the lane's place once more: kept through the loop, it would be spilled)
+    const int l_end = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)) & 15, col_end = min(ct * kResidentTile + l_end * 4, N - 4);
 #pragma unroll
     for (int rr = 0; rr < RR; ++rr) {
-        if (row[rr] >= M) continue;
         RowSum& sum = total[rr];
-        for (int j = p[rr]; j < end[rr]; ++j) {
-            const double v = values[j];
-            const Vec<4> b = Vec<4>::gload(B + (size_t)col_indices[j] * N + col);
-            sum.x = fma(v, (double)b.v.x, sum.x);
-            sum.y = fma(v, (double)b.v.y, sum.y);
-            sum.z = fma(v, (double)b.v.z, sum.z);
-            sum.w = fma(v, (double)b.v.w, sum.w);
-        }
+        gather_rest(p[rr], end[rr], l_end, N, col_indices, values, B + col_end, sum, std::make_integer_sequence<int, 8>{});
+        if (row[rr] >= M) continue;
         const Vec<4> out{make_float4((float)sum.x, (float)sum.y, (float)sum.z, (float)sum.w)};
-        if (ct * kResidentTile + l * 4 < N) out.gstore(C + (size_t)row[rr] * N + col, streaming != 0);
+        if (ct * kResidentTile + l_end * 4 < N) out.gstore(C + (size_t)row[rr] * N + col_end, streaming != 0);
     }
 }
 

@@ -120,3 +120,18 @@ def test_sddmm_values_without_parts(D, density, what):
     gathered = time_us(lambda: dl.sddmm(ro, ci, lhs, rhs))
     dl.set_tuning()
     assert took <= (1.35 if what.endswith("lhs") else 1.0) * gathered
+
+
+# The row-block kernels do not care about the order of columns (350 us here). From slices of B such rows are gathered at the end of the
+# workgroup that has them: 560 us, and 455 with every sixteenth row like that (890 and 740 while that was one nonzero after the other).
+def test_spmm_columns_that_do_not_ascend():
+    M, K, N = 16384, 4096, 128
+    ro, ci, row = mask(M, K, 0.3, 5)
+    values, B = normal(ci.numel()), normal(K, N)
+    assert dl.describe_schedule(dl.OP_SPMM, M, K, N, ci.numel())["schedule"] == "resident"
+    few, all_ = shuffled(ci, row, row % 16 == 0), shuffled(ci, row, row >= 0)
+    took, took_few = (time_us(lambda: dl.spmm(ro, c, values, B)) for c in (all_, few))
+    dl.set_tuning(rules_off=dl.RULES["resident_slices"])
+    blocks, blocks_few = (time_us(lambda: dl.spmm(ro, c, values, B)) for c in (all_, few))
+    dl.set_tuning()
+    assert took <= 2.0 * blocks and took_few <= 1.8 * blocks_few
