@@ -16,8 +16,9 @@ namespace {
 
 constexpr int kEighths = 8;  // the row blocks are dealt to eight XCDs; DLSPM_HINT_BANDED gives each a contiguous eighth
 // stats: [0] longest row, [1] rows without nonzeros, [2] widest row (largest - smallest column + 1),
-// [3 .. 10] smallest column of each eighth of the rows, [11 .. 18] largest, [19 .. 26] nonzeros of each eighth
-constexpr int kStats = 3 + 3 * kEighths;
+// [3 .. 10] smallest column of each eighth of the rows, [11 .. 18] largest, [19 .. 26] nonzeros of each eighth,
+// [27] rows whose columns do not ascend strictly, [28] nonzeros of the heaviest 64 rows
+constexpr int kUnordered = 3 + 3 * kEighths, kHeaviest = kUnordered + 1, kStats = kHeaviest + 1, kHeavyRows = 64;
 
 // Where the kernel leaves its figures: one of 64 slots of a static device array (32 ints each), taken for the length of
 // one call, and the same slot of a pinned host array (8 KiB per device, allocated at the first call on that device and
@@ -107,7 +108,7 @@ __global__ __launch_bounds__(256) void analyze_kernel(int M, int K, int rows_per
     const long long first = wave * rows_per_wave;
     if (first >= M) return;
     const int last = (int)min(first + rows_per_wave, (long long)M);
-    int longest = 0, empty = 0, widest = 0;
+    int longest = 0, empty = 0, widest = 0, unordered = 0;
     int cur = eighth_of(first, M), lo = 0x7fffffff, hi = -1;
     auto flush = [&]() {
         if (lane == 0 && hi >= 0) {
@@ -128,11 +129,17 @@ __global__ __launch_bounds__(256) void analyze_kernel(int M, int K, int rows_per
         longest = max(longest, len);
         empty += len == 0 ? 1 : 0;
         int rlo = 0x7fffffff, rhi = -1;
+        bool ascends = true;
+        int last = (int)0x80000000;  // of the 64 before
         for (int p = rs + lane; p < re; p += kWave) {
-            const int c = min(max(col_indices[p], 0), max(K - 1, 0));
+            const int at = col_indices[p];
+            ascends = ascends && __builtin_amdgcn_update_dpp(last, at, 0x138, 0xf, 0xf, false) < at;  // wave_shr:1
+            last = __builtin_amdgcn_readlane(at, kWave - 1);
+            const int c = min(max(at, 0), max(K - 1, 0));
             rlo = min(rlo, c);
             rhi = max(rhi, c);
         }
+        unordered += __ballot(!ascends) != 0 ? 1 : 0;
         rlo = wave_min_int(rlo);
         rhi = wave_max_int(rhi);
         if (rhi >= 0) {
@@ -146,7 +153,14 @@ __global__ __launch_bounds__(256) void analyze_kernel(int M, int K, int rows_per
         if (longest > 0) atomicMax(&stats[0], longest);
         if (empty > 0) atomicAdd(&stats[1], empty);
         if (widest > 0) atomicMax(&stats[2], widest);
+        if (unordered > 0) atomicAdd(&stats[kUnordered], unordered);
     }
+    int heaviest = 0;
+    const long long waves = ((long long)M + rows_per_wave - 1) / rows_per_wave;
+    for (long long r = (wave * kWave + lane) * kHeavyRows; r < M; r += waves * kWave * kHeavyRows)
+        heaviest = max(heaviest, row_offsets[min(r + kHeavyRows, (long long)M)] - row_offsets[r]);
+    heaviest = wave_max_int(heaviest);
+    if (lane == 0 && heaviest > 0) atomicMax(&stats[kHeaviest], heaviest);
     if (wave == 0 && lane < kEighths) {  // the nonzeros of each eighth, from the offsets at its ends
         const long long a = (long long)lane * M / kEighths, b = (long long)(lane + 1) * M / kEighths;
         stats[3 + 2 * kEighths + lane] = max(row_offsets[b] - row_offsets[a], 0);
@@ -167,7 +181,10 @@ int dlspm_analyze(int M, int K, int nnz, const int* row_offsets, const int* col_
     if ((long long)nnz > (long long)M * K) return DLSPM_E_INVALID_ARG;
     if (M > 0 && !row_offsets) return DLSPM_E_INVALID_ARG;
     if (nnz > 0 && !col_indices) return DLSPM_E_INVALID_ARG;
-    *info = dlspm_matrix_info{M, K, nnz, 0, 0, 0, 0, 0};
+    *info = dlspm_matrix_info{};
+    info->M = M;
+    info->K = K;
+    info->nnz = nnz;
     if (M == 0) return DLSPM_OK;
     const DeviceInfo& dev = device_info();
     if (!dev.present || !dev.gfx950) return DLSPM_E_NO_DEVICE;
@@ -214,6 +231,8 @@ int dlspm_analyze(int M, int K, int nnz, const int* row_offsets, const int* col_
         total += h[3 + 2 * kEighths + x];
     }
     info->eighths_cover_permille = K > 0 ? (int)std::min<long long>(cover * 1000 / K, 1000ll * kEighths) : 0;
+    info->unordered_rows = h[kUnordered];
+    info->heaviest_64_rows = h[kHeaviest];
     info->eighths_nnz_permille = total > 0 ? (int)std::min<long long>(heaviest * 1000 * kEighths / total, 1000ll * kEighths) : 0;
     return DLSPM_OK;
 }
@@ -247,8 +266,20 @@ int dlspm_advise(int op, int N_or_D, const dlspm_matrix_info* info, dlspm_call_p
         plan->hints = DLSPM_HINT_BANDED | (even ? DLSPM_HINT_ROWS_EVEN : 0);
         return DLSPM_OK;
     }
+    // Rows whose columns do not ascend are gathered one by one, behind what dense tiles and slices of B in LDS do for the others
+    // (fused, all rows shuffled, the schedules below / two steps: 16384 x 4096 at 0.2, D = 64 224 / 320 us, 12288 x 2048 at 0.3, D = 128 240 / 518,
+    // 32768 x 8192 at 0.3, D = 32 900 / 1570): not more than one in sixteen, except in place of column slices, which want them to ascend
+    // too (8192 x 8192, D = 128 at 0.2 / 0.3 955 / 657 and 1423 / 958, 16384 x 8192 at 0.2 1888 / 1520).
+    const bool ascend = 16ll * info->unordered_rows <= M;
+    int slices = 0;
+    (void)dlspm_describe_slices(op, M, K, N_or_D, nnz, &slices, nullptr);
+    // Workgroups that own 64 rows and more end when the heaviest does. Heaviest 64 rows / mean, and the time of the row plan or slices / of two
+    // steps: all nonzeros in full rows at the top (5.0) 16384 x 8192 at 0.2, D = 128 838 / 1217, (3.3) 12288 x 2048 at 0.3 236 / 305, 32768 x 8192
+    // at 0.3, D = 32 860 / 1299; a triangle (2.0) 860 / 667, 239 / 216, and at D = 32 862 / 918; full rows anywhere (1.6) 985 / 678,
+    // 237 / 198, at D = 32 856 / 862; lognormal rows, sigma 1 (1.5) 885 / 550, 215 / 150.
+    const double heavy = info->heaviest_64_rows > 0 ? (double)info->heaviest_64_rows * M / (64.0 * nnz) : info->eighths_nnz_permille * 1e-3;
     // 2. the fused op on dense masks: memory for the scores between its two steps (never less than what the call would refuse)
-    if (op == DLSPM_OP_FUSED) {
+    if (op == DLSPM_OP_FUSED && (ascend || slices > 0) && (even || heavy <= (N_or_D <= 32 ? 1.5 : 2.5))) {
         const size_t bytes = fused_two_steps_bytes(dev, M, K, N_or_D, nnz, even);
         if (bytes > 0) {
             plan->bytes = std::max(bytes, dlspm_workspace_bytes(op, M, K, N_or_D, nnz));
@@ -278,7 +309,7 @@ int dlspm_advise(int op, int N_or_D, const dlspm_matrix_info* info, dlspm_call_p
         return DLSPM_OK;
     }
     // 4. even rows on dense tiles: memory for the parts of B
-    if (op == DLSPM_OP_SPMM && even && spmm_tiles_choose(dev, M, K, N_or_D, nnz, spmm_resident_choose(dev, M, K, N_or_D, nnz, true, false).us)) {
+    if (op == DLSPM_OP_SPMM && even && ascend && spmm_tiles_choose(dev, M, K, N_or_D, nnz, spmm_resident_choose(dev, M, K, N_or_D, nnz, true, false).us)) {
         plan->bytes = spmm_tiles_bytes(K, N_or_D);
         plan->hints = DLSPM_HINT_ROWS_EVEN;
         return DLSPM_OK;

@@ -99,11 +99,12 @@ RULES = {"eight_waves_few_rows": 1, "sixteen_waves_tall_long_rows": 2, "more_wav
 
 class MatrixInfo(ctypes.Structure):
     """dlspm_matrix_info of include/dlspm_hip.h."""
-    _fields_ = [(n, ctypes.c_int) for n in ("M", "K", "nnz", "max_row_len", "empty_rows", "max_col_span",
-                                            "eighths_cover_permille", "eighths_nnz_permille")]
+    _shape = ("M", "K", "nnz", "max_row_len", "empty_rows", "max_col_span", "eighths_cover_permille", "eighths_nnz_permille")
+    _fields_ = [(n, ctypes.c_int) for n in (*_shape, "unordered_rows", "heaviest_64_rows")]
 
     def as_dict(self):
-        return {n: getattr(self, n) for n, _ in self._fields_}
+        """the matrix's shape: all figures but the last two, which only dense tiles ask for"""
+        return {n: getattr(self, n) for n in self._shape}
 
 
 class CallPlan(ctypes.Structure):

@@ -281,3 +281,52 @@ def test_no_memory_is_asked_for_that_the_call_does_not_look_at(dl):
                 assert cp.bytes == 0 and run == with_memory
                 seen["memory"] += 1
     assert min(seen.values()) > 20, seen
+
+
+@pytest.mark.gpu
+def test_analyze_counts_rows_out_of_order_and_the_heaviest_64(dl):
+    import torch
+
+    rng = np.random.default_rng(5)
+    for kind, M, K, density in [("uniform", 1000, 777, 0.1), ("skewed", 5000, 2048, 0.02), ("empty_rows", 333, 500, 0.3), ("empty", 64, 64, 0.0),
+                                ("full", 40, 100, 1.0), ("uniform", 7, 5000, 0.5), ("skewed", 100000, 512, 0.02), ("uniform", 65, 300, 0.4)]:
+        ro, ci = random_csr(rng, M, K, kind, density)
+        heaviest = max(int(ro[min(i + 64, M)] - ro[i]) for i in range(0, M, 64))
+        lens, want = np.diff(ro), 0
+        for r in rng.choice(M, min(M, 40), replace=False):
+            a, b, what = ro[r], ro[r + 1], rng.integers(3)
+            if lens[r] >= 2 and what == 0:  # the last two change places
+                ci[b - 2], ci[b - 1] = ci[b - 1], ci[b - 2]
+            elif lens[r] >= 2 and what == 1:  # the first comes twice
+                ci[a + 1] = ci[a]
+            elif lens[r] >= 70 and what == 2:  # from the 64th on to the 65th
+                ci[a + 64] = ci[a + 3]
+        for r in range(M):
+            want += int((np.diff(ci[ro[r]:ro[r + 1]]) <= 0).any())
+        got = dl.analyze(dev(torch, ro), dev(torch, ci), K)
+        assert (got.unordered_rows, got.heaviest_64_rows) == (want, heaviest), (kind, M, K)
+
+
+def test_tiles_are_for_rows_that_ascend_and_share_the_work(dl):
+    """Memory for dense tiles and for the fused op's two steps: not for matrices whose rows do not ascend, nor (two steps) where a few
+    rows that lie together hold the nonzeros."""
+    M, K, D = 12288, 2048, 128
+    nnz = int(M * K * 0.3)
+    mean_64 = nnz * 64 // M
+
+    def advice(op, longest, unordered=0, heaviest=0, eighths=1000, width=D, M=M, K=K, nnz=nnz):
+        info = dl.MatrixInfo(M, K, nnz, longest, 0, K, 8000, eighths, unordered, heaviest)
+        return dl.advise(op, width, info)
+
+    scores = nnz * 4
+    fused = lambda *a, **kw: advice(dl.OP_FUSED, *a, **kw).bytes >= scores  # noqa: E731
+    assert fused(700) and fused(700, M // 16) and not fused(700, M // 16 + 1) and not fused(700, M)
+    uneven = K  # (a full row)
+    assert fused(uneven) and fused(uneven, 0, 2 * mean_64) and not fused(uneven, 0, 3 * mean_64) and not fused(uneven, M, 2 * mean_64)
+    assert not fused(uneven, eighths=3300) and fused(uneven, 0, 2 * mean_64, eighths=3300)
+    assert advice(dl.OP_FUSED, uneven, 0, 3 * mean_64).build != dl.BUILD_NOTHING  # (the row plan, as without tiles)
+    large = dict(M=32768, K=8192, nnz=32768 * 2457, width=32)
+    assert advice(dl.OP_FUSED, 8192, 0, 64 * 2457 * 5 // 4, **large).bytes >= 32768 * 2457 * 4
+    assert advice(dl.OP_FUSED, 8192, 0, 64 * 2457 * 2, **large).bytes < 32768 * 2457 * 4
+    spmm = dict(M=16384, K=8192, nnz=16384 * 2457, width=128)
+    assert advice(dl.OP_SPMM, 2700, **spmm).bytes > 0 and advice(dl.OP_SPMM, 2700, 1024, **spmm).bytes > 0 and advice(dl.OP_SPMM, 2700, 1025, **spmm).bytes == 0
