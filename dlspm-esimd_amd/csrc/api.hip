@@ -528,13 +528,21 @@ static SddmmCall sddmm_decide(const DeviceInfo& dev, int M, int K, int D, int nn
     return c;
 }
 
-// The fused op as SDDMM on dense tiles and then SpMM, the scores in the caller's memory in between: where the masks are dense enough that
-// the scores of whole tiles cost less than the gathered ones, and both steps together take less than 0.92 of the fused kernels' time (10691 x 4000,
-// D = 95 at 0.14, and 2919 x 5655, D = 75 at 0.13, estimated at 0.95: 198 -> 207 and 71 -> 79).
-// Estimates (us): those of the two steps, 2 for the second launch, and 2 + nnz x 0.0100 / 0.0162 / 0.0315 / 0.0343 x 1e-3 for the fused kernels
-// at D <= 32 / 64 / 96 / 128 (8192 x 8192, D = 128 at 0.1 / 0.2 / 0.3 232 / 442 / 688, D = 32 at 0.3 200; 16384 x 4096, D = 64 at 0.2 218;
-// 24576 x 8192, D = 80 at 0.1 623). A second step of row blocks takes more than its estimate on uneven rows (4000 x 4090, D = 77 at 0.2,
-// lognormal: fused 96, two steps 118) and below D = 64 (8192 x 8192, D = 32 at 0.3 145, estimate 105). Measured, fused -> two steps: 8192 x 8192, D = 128 at 0.1 / 0.2 / 0.3 230 / 437 / 683 -> 206 / 261 / 325, with
+// The fused op as SDDMM on dense tiles and then SpMM, the scores in the caller's memory in between, where the masks are dense enough that
+// both steps together are estimated to take less time than the fused kernels. Whether SDDMM alone would run on tiles is another question:
+// gathering also feeds the fused kernels' second stage. Estimates (us):
+//   two steps  those of the steps, and 2 for the second launch. 1.05 of the measured time in the geometric mean over the 73 of 173 sizes
+//              (Bernoulli and lognormal rows, M = 2000 ... 33000, K = 1200 ... 9100, D = 24 ... 128, density 0.06 ... 0.5) where the second runs
+//              from slices of B in LDS or on tiles.
+//   fused      2 + nnz x 0.0100 / 0.0162 / 0.0290 / 0.0343 x 1e-3 at D <= 32 / 64 / 96 / 128 (8192 x 8192, D = 128 at 0.1 / 0.2 / 0.3 232 / 442 /
+//              688, D = 32 at 0.3 200; 16384 x 4096, D = 64 at 0.2 218; measured / estimated 0.91 ... 1.32 in nine of ten).
+// A second step of row blocks is for even rows and D from 64 on (lognormal rows, 4000 x 4090, D = 77 at 0.2: fused 96, two steps 118; 8192 x 8192,
+// D = 32 at 0.3: 145, estimate 105). Its time goes by workgroups of four rows per compute unit, the fused row blocks' too (2291 x 3228, 2.2
+// of them, D = 96 at 0.36: three rounds, 94 -> 86; 2096 x 7374 in column slices, D = 128 at 0.44: 229 -> 244, not taken), and the two are
+// near each other: from 0.95 on. Of the 173 sizes 78 are taken, at 0.31 ... 1.02 of the time of the schedule before (two above 0.96); seven
+// of the others would gain more than 5 %. Below M = 8192 at density 0.1, D = 128, 230 -> 206; above it 129 row blocks in two ranges
+// of columns are a second round for two compute units, and two steps lose (8321 x 8180 at 0.11 289 -> 317).
+// Measured, fused -> two steps: 8192 x 8192, D = 128 at 0.1 / 0.2 / 0.3 230 / 437 / 683 -> 206 / 261 / 325, with
 // lognormal rows at 0.3 747 -> 392; 16384 x 8192, D = 128 at 0.3 1357 -> 451; 16384 x 4096, D = 64 at 0.2 217 -> 144; 4096 x 4096, D = 128 at
 // 0.3 165 -> 140; 12288 x 2048, D = 128 at 0.3 235 -> 112; 32768 x 8192, D = 32 at 0.3 890 -> 622.
 static size_t scores_bytes(int nnz) { return ((size_t)nnz * sizeof(float) + 255) / 256 * 256; }
@@ -552,13 +560,20 @@ static WorkspaceArg behind_scores(const WorkspaceArg& ws, int nnz)
 static bool fused_two_steps(const DeviceInfo& dev, int M, int K, int D, int nnz, const WorkspaceArg& ws, FusedCall& c)
 {
     if (!ws.mem || ws.bytes < scores_bytes(nnz)) return false;
-    c.tiles = sddmm_tiles_choose(dev, M, K, D, nnz);
+    c.tiles = sddmm_tiles_plan(dev, M, K, D, nnz);
     if (c.tiles.ranges == 0) return false;
     c.second = spmm_decide(dev, M, K, D, nnz, behind_scores(ws, nnz));
-    const double second_us = c.second.schedule == DLSPM_SCHEDULE_DENSE_TILES ? spmm_tiles_us(dev, M, K, D, nnz) : c.second.resident.us;
-    if (c.second.schedule == DLSPM_SCHEDULE_ROW_BLOCKS && (!ws.rows_even || D < 64)) return false;
-    const double fused_us = 2.0 + (double)nnz * (D <= 32 ? 1.00e-5 : D <= 64 ? 1.62e-5 : D <= 96 ? 3.15e-5 : 3.43e-5);
-    return c.second.resident.us > 0.0 && c.tiles.us + second_us + 2.0 < 0.92 * fused_us;  // (no estimate: a schedule was asked for by name)
+    if (c.second.resident.us <= 0.0) return false;  // (no estimate: a schedule was asked for by name)
+    double second_us = c.second.schedule == DLSPM_SCHEDULE_DENSE_TILES ? spmm_tiles_us(dev, M, K, D, nnz) : c.second.resident.us;
+    double fused_us = 2.0 + (double)nnz * (D <= 32 ? 1.00e-5 : D <= 64 ? 1.62e-5 : D <= 96 ? 2.90e-5 : 3.43e-5);
+    if (c.second.schedule == DLSPM_SCHEDULE_ROW_BLOCKS) {
+        if (!ws.rows_even || D < 64) return false;
+        const double rounds = M / (4.0 * dev.cus), whole = std::ceil(rounds) / rounds;
+        const bool slices = fused_slice_plan(dev, M, K, D, nnz, fused_choose(dev, M, D, nnz, true)).slices > 0;
+        second_us *= whole;
+        if (!slices) fused_us *= 0.95 * whole;
+    }
+    return c.tiles.us + second_us + 2.0 < fused_us;
 }
 size_t fused_two_steps_bytes(const DeviceInfo& dev, int M, int K, int D, int nnz, bool rows_even)
 {

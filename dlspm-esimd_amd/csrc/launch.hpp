@@ -245,7 +245,8 @@ struct TilePlan {
     int ranges;
     double us;  // estimated time
 };
-TilePlan sddmm_tiles_choose(const DeviceInfo& dev, int M, int K, int D, int nnz);
+TilePlan sddmm_tiles_plan(const DeviceInfo& dev, int M, int K, int D, int nnz);    // the best ranges
+TilePlan sddmm_tiles_choose(const DeviceInfo& dev, int M, int K, int D, int nnz);  // ... where SDDMM runs on them
 void sddmm_tile_shape(int* rows, int* columns);
 hipError_t sddmm_tiles_launch(const SddmmArgs& x, float scale, const TilePlan& plan, hipStream_t stream);  // (the results times scale)
 hipError_t sddmm_flat_launch(const SddmmArgs& x, const SddmmShape& s, int chunk, hipStream_t stream);

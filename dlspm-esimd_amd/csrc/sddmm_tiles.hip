@@ -473,10 +473,10 @@ template <int SEGMENTS> static hipError_t launch_one(const SddmmArgs& x, float s
     return hipGetLastError();
 }
 
-// Tiles for these sizes, or ranges == 0: where their estimated time is below 0.9 of the gathering kernels', whatever the call brings
-// with it and whatever schedule the tuning
-// overrides name (so that the bits of a result depend on the sizes alone; DLSPM_RULE_DENSE_GROUPS switches tiles off). Both estimates (us) are fits to one operand set worked on over
-// and over:
+// The ranges of columns with which tiles are estimated to take the least time, and that time (sddmm_tiles_plan; ranges == 0: not for
+// these sizes), and whether SDDMM runs on them: where it is below 0.9 of the gathering kernels', whatever the call brings with it and
+// whatever schedule the tuning overrides name (so that the bits of a result depend on the sizes alone; DLSPM_RULE_DENSE_GROUPS switches
+// tiles off). Both estimates (us) are fits to one operand set worked on over and over:
 //   gathering   2 + nnz (2.2 + 0.122 D) 1e-6, D rounded up to a whole access of eight lanes, a fifth more where lanes past D are masked
 //               one by one (a twenty-fifth up to D = 24; 8192 x 8192 at density 0.1, D = 32 / 50 / 64 / 128 38 / 82 / 63 / 125, estimate
 //               43 / 79 / 69 / 121);
@@ -487,17 +487,14 @@ template <int SEGMENTS> static hipError_t launch_one(const SddmmArgs& x, float s
 //               each unit, take about 0.75 of a full one's.
 // 56 masks of 500 ... 8200 rows near the line, gathering / tiles: 0.91 ... 2.7; the five below 1.1 were D = 17 ... 22 on 2000 ... 6000 rows
 // (2952 x 1702 at 0.47, D = 19, lognormal rows, 14.7 / 16.6), for which the additions up to D = 32 are.
-TilePlan sddmm_tiles_choose(const DeviceInfo& dev, int M, int K, int D, int nnz)
+TilePlan sddmm_tiles_plan(const DeviceInfo& dev, int M, int K, int D, int nnz)
 {
-    const TilePlan none{0, 0.0};
-    if (!rule_on(kRuleDenseGroups) || D < 17 || D > 128 || M <= 0 || K <= 0 || nnz <= 0 || nnz >= (1 << 29) || !dense_fits_buffer(K + 256ll, D)) return none;
+    TilePlan best{0, 0.0};
+    if (!rule_on(kRuleDenseGroups) || D < 17 || D > 128 || M <= 0 || K <= 0 || nnz <= 0 || nnz >= (1 << 29) || !dense_fits_buffer(K + 256ll, D)) return best;
     const double density = (double)nnz / ((double)M * K);
     const int segments = (int)ceil_div(D, 32);
     const long long row_blocks = ceil_div(M, kTileRows), tiles = ceil_div(K, kTileCols), slots = (segments == 1 ? 2ll : 1ll) * dev.cus;
     const double tile_us = segments == 1 ? 4.4 + 6.0 * density + 12.0 * std::max(0.0, density - 0.3) : 0.1 + 1.42 * segments + 5.5 * density;
-    const double gathered = 32.0 * segments * (D % 4 == 0 ? 1.0 : D <= 24 ? 1.04 : 1.2);
-    TilePlan best = none;
-    double best_us = 0.9 * (2.0 + (double)nnz * (2.2 + 0.122 * gathered) * 1e-6);
     for (long long wanted = 1; wanted <= tiles && wanted <= 64; ++wanted) {
         const long long per = ceil_div(tiles, wanted), ranges = ceil_div(tiles, per), units = row_blocks * ranges;
         double rounds = (double)(units / slots);
@@ -505,12 +502,15 @@ TilePlan sddmm_tiles_choose(const DeviceInfo& dev, int M, int K, int D, int nnz)
         if (last > 0.0) rounds += segments > 1 ? 1.0 : 0.75 + 0.5 * std::max(0.0, last - 0.5);
         const double start_us = (ranges > 1 ? 8.0 : 6.0) + (segments == 1 ? 1.0 : 0.0);
         const double us = (double)ceil_div(units, slots) * start_us + rounds * (double)per * tile_us;
-        if (us < best_us) {
-            best_us = us;
-            best = TilePlan{(int)ranges, us};
-        }
+        if (best.ranges == 0 || us < best.us) best = TilePlan{(int)ranges, us};
     }
     return best;
+}
+TilePlan sddmm_tiles_choose(const DeviceInfo& dev, int M, int K, int D, int nnz)
+{
+    const TilePlan best = sddmm_tiles_plan(dev, M, K, D, nnz);
+    const double gathered = 32.0 * (double)ceil_div(D, 32) * (D % 4 == 0 ? 1.0 : D <= 24 ? 1.04 : 1.2);
+    return best.us < 0.9 * (2.0 + (double)nnz * (2.2 + 0.122 * gathered) * 1e-6) ? best : TilePlan{0, 0.0};
 }
 
 void sddmm_tile_shape(int* rows, int* columns)

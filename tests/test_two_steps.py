@@ -170,3 +170,20 @@ def test_one_plan_on_two_streams_and_in_a_graph():
         other = dl.fused(*args, *sets[1 - i], 0.5, plan=plan)
         torch.cuda.synchronize()
         assert torch.equal(out, want[i]) and torch.equal(other, want[1 - i])
+
+
+def test_the_rule_holds_beside_powers_of_two():
+    """At density 0.1, D = 128 up to 8192 rows (as many row blocks, in two ranges of columns, as there are compute units), and not where
+    the next row block begins a second round."""
+    def runs(M, K, D, density, even=True):
+        info = dl.MatrixInfo(M, K, int(M * K * density), int(K * density * 1.2) if even else K, 0, K, 8000, 1000)
+        cp = dl.advise(dl.OP_FUSED, D, info)
+        return dl.describe_schedule(dl.OP_FUSED, M, K, D, info.nnz, workspace_bytes=cp.bytes | cp.hints)["schedule"] == "two_steps"
+
+    rng = np.random.default_rng(3)
+    assert all(runs(8192 - int(a), 8192 - int(b), 128, d) for a, b, d in zip(rng.integers(0, 64, 200), rng.integers(0, 64, 200), rng.uniform(0.0985, 0.1015, 200)))
+    assert not runs(8321, 8180, 128, 0.113) and not runs(8578, 8015, 120, 0.098)
+    # one size each of a second step from slices of B, on tiles and of row blocks, and those that measured slower
+    assert runs(17343, 3729, 128, 0.132) and runs(16075, 7628, 128, 0.305) and runs(4822, 6818, 96, 0.241) and runs(4676, 7785, 128, 0.212)
+    assert not runs(2096, 7374, 128, 0.44) and not runs(7808, 7995, 96, 0.087) and not runs(23879, 3669, 64, 0.113) and not runs(17071, 7498, 32, 0.251)
+    assert not runs(12772, 3715, 96, 0.135, even=False) and runs(28641, 1244, 64, 0.254, even=False)
