@@ -448,7 +448,7 @@ def test_sddmm_results_beyond_the_l2_are_streamed(torch_cuda, dl, oracle):
     """More results than one and a half L2s hold (here 9.4 million = 38 MB; an MI355X's L2 is 4 MiB) are stored with the
     non-temporal hint; the bits must be those of ordinary stores under every schedule: row blocks, the
     even-rows hint, a row plan, and the flat schedule forced by tuning, all against the multi-threaded oracle and equal
-    to each other."""
+    to each other. (Dense tiles, which such masks run on by themselves, are switched off: their sums have another order.)"""
     torch = torch_cuda
     M, K, D = 8192, 8192, 32
     ro, ci = dl.make_pattern(dl.PATTERN_BERNOULLI, 71, M, K, 0.14)
@@ -459,11 +459,13 @@ def test_sddmm_results_beyond_the_l2_are_streamed(torch_cuda, dl, oracle):
     want = oracle.sddmm(ro, ci, lhs, rhs, omp=True)
     ro_d, ci_d, lhs_d, rhs_d = (dev(torch, x) for x in (ro, ci, lhs, rhs))
     first = None
-    for name in ("null", "rows_even", "plan", "flat"):
-        if name == "flat":
-            dl.set_tuning(flat=1)
-        got = dl.sddmm(ro_d, ci_d, lhs_d, rhs_d, workspace=dl.ROWS_EVEN if name == "rows_even" else None,
-                       plan=dl.row_plan(ro_d) if name == "plan" else None).cpu().numpy()
+    for name, runs in (("null", "row_blocks"), ("rows_even", "row_blocks"), ("plan", "row_plan"), ("flat", "flat")):
+        plan = dl.row_plan(ro_d) if name == "plan" else None
+        size = {"rows_even": dl.HINT_ROWS_EVEN, "plan": dl.row_plan_bytes(M) | dl.HINT_ROW_PLAN}.get(name, 0)
+        dl.set_tuning(rules_off=dl.RULES["dense_groups"], flat={"null": 0, "flat": 1}.get(name, -1))
+        run = dl.describe_schedule(dl.OP_SDDMM, M, K, D, ci.size, workspace_bytes=size)
+        assert run["schedule"] == runs and "tile_columns" not in run
+        got = dl.sddmm(ro_d, ci_d, lhs_d, rhs_d, workspace=dl.ROWS_EVEN if name == "rows_even" else None, plan=plan).cpu().numpy()
         dl.set_tuning()
         assert oracle.rel_frobenius(got, want) <= TOL, name
         first = got if first is None else first

@@ -232,3 +232,28 @@ def test_results_that_are_not_finite_run_by_run(torch_cuda, M, K, D, density):
     assert bool((on[on.isinf()] == off[on.isinf()]).all()) and bool((on.isinf() == off.isinf()).all())
     fine = on.isfinite()
     assert float((on - off)[fine].norm() / off[fine].norm()) <= 1e-6
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K,D,density", [(4100, 4097, 32, 0.9), (4097, 4095, 17, 0.9), (2111, 2303, 64, 0.9), (1985, 4095, 63, 0.6), (1023, 2048, 96, 0.9), (1087, 2817, 128, 0.7),
+                                           (1000, 2000, 127, 0.9)])
+def test_hinted_stores_change_no_bit(torch_cuda, M, K, D, density):
+    """Results that go past the caches and those that do not, of kernels of their own for both, at every number of segments and for
+    whole and ragged widths; columns that do not ascend and a NaN among them (whose results are stored by the row)."""
+    torch = torch_cuda
+    ro, ci, row = mask(torch, M, K, density, 43)
+    lhs, rhs = operands(torch, M, K, D, 44)
+    rhs[K // 2] = float("nan")
+    at = torch.arange(ci.numel(), device="cuda")
+    first, end = ro[:-1].long()[row], ro[1:].long()[row]
+    ci = torch.where(row % 11 == 2, ci[first + end - 1 - at], ci)
+    got = []
+    for stream in (0, 1):
+        dl.set_tuning(stream_results=stream)
+        assert "tile_columns" in dl.describe_schedule(dl.OP_SDDMM, M, K, D, ci.numel())
+        out = torch.full((ci.numel() + 64,), 7.0, device="cuda")
+        dl.sddmm(ro, ci, lhs, rhs, out=out[:ci.numel()])
+        assert bool((out[ci.numel():] == 7.0).all())
+        got.append(out[:ci.numel()].view(torch.int32))
+    dl.set_tuning()
+    assert torch.equal(*got) and bool((got[0].view(torch.float32).isnan() == (ci == K // 2)).all())
