@@ -474,9 +474,9 @@ template <int SEGMENTS> static hipError_t launch_one(const SddmmArgs& x, float s
 }
 
 // The ranges of columns with which tiles are estimated to take the least time, and that time (sddmm_tiles_plan; ranges == 0: not for
-// these sizes), and whether SDDMM runs on them: where it is below 0.9 of the gathering kernels', whatever the call brings with it and
-// whatever schedule the tuning overrides name (so that the bits of a result depend on the sizes alone; DLSPM_RULE_DENSE_GROUPS switches
-// tiles off). Both estimates (us) are fits to one operand set worked on over and over:
+// these sizes, or tuning overrides name a schedule), and whether SDDMM runs on them: where it is below 0.9 of the gathering kernels',
+// whatever the call brings with it (so that the bits of a result depend on the sizes alone). Both estimates (us) are fits to one operand
+// set worked on over and over:
 //   gathering   2 + nnz (2.2 + 0.122 D) 1e-6, D rounded up to a whole access of eight lanes, a fifth more where lanes past D are masked
 //               one by one (a twenty-fifth up to D = 24; 8192 x 8192 at density 0.1, D = 32 / 50 / 64 / 128 38 / 82 / 63 / 125, estimate
 //               43 / 79 / 69 / 121);
@@ -490,6 +490,8 @@ template <int SEGMENTS> static hipError_t launch_one(const SddmmArgs& x, float s
 TilePlan sddmm_tiles_plan(const DeviceInfo& dev, int M, int K, int D, int nnz)
 {
     TilePlan best{0, 0.0};
+    const Tuning& t = tuning();
+    if (t.split_w > 0 || t.flat >= 0 || t.flat_chunk > 0 || t.slices >= 0 || t.plan_order > 0 || t.xcd_contiguous) return best;  // (a schedule that was asked for by name)
     if (!rule_on(kRuleDenseGroups) || D < 17 || D > 128 || M <= 0 || K <= 0 || nnz <= 0 || nnz >= (1 << 29) || !dense_fits_buffer(K + 256ll, D)) return best;
     const double density = (double)nnz / ((double)M * K);
     const int segments = (int)ceil_div(D, 32);

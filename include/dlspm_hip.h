@@ -398,7 +398,9 @@ int dlspm_describe_slices(int op, int M, int K, int N_or_D, int nnz, int* slices
  * rules themselves unless the environment said otherwise when the library first looked, once per process:
  * DLSPM_SPLIT="W,R", DLSPM_FLAT, DLSPM_FLAT_CHUNK, DLSPM_SLICES, DLSPM_TILE_MAJOR, DLSPM_TILE_WIDTH, DLSPM_PLAN_ORDER,
  * DLSPM_XCD_CONTIGUOUS, DLSPM_STREAM_RESULTS
- * (so that the drivers can be swept from a shell). No launch reads the environment. An override that names a shape
+ * (so that the drivers can be swept from a shell). An override that names a schedule (split, flat, slices, tiles of columns, the
+ * order of a plan or of the row blocks) also keeps a call from the schedules that the sizes alone choose: slices of B in LDS, dense
+ * tiles, two steps. No launch reads the environment. An override that names a shape
  * the kernels are not built for is ignored. dlspm_workspace_bytes and the describe calls follow the overrides, so
  * set them before sizing a workspace. No counterpart in the reference (its knobs are -D macros, SPMM/spmmesimd.hpp:17-21).
  */

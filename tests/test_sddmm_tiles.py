@@ -68,6 +68,22 @@ def test_where_tiles_are_chosen():
     assert "tile_columns" not in case(24576, 8192, 32, 0.2)
 
 
+@pytest.mark.parametrize("named,runs,size", [({"flat": 0}, "row_blocks", 0), ({"flat": 1}, "flat", 0), ({"slices": 4}, "sliced", 1 << 40), ({"split": (4, 2)}, "flat", 0),
+                                             ({"split": (4, 2), "flat": 0}, "row_blocks", 0), ({"xcd_contiguous": 1}, "flat", 0), ({"flat_chunk": 512}, "flat", 0)])
+def test_a_schedule_asked_for_by_name_runs(named, runs, size):
+    """Tuning overrides that name a schedule of the gathering kernels get it, as for SpMM; the fused op's two steps need tiles."""
+    M, K, D, nnz = 24576, 8192, 32, int(24576 * 8192 * 0.2)
+    tiles = lambda: "tile_columns" in dl.describe_schedule(dl.OP_SDDMM, M, K, D, nnz, workspace_bytes=size)  # noqa: E731
+    assert tiles()
+    dl.set_tuning(**named)
+    run, fused = dl.describe_schedule(dl.OP_SDDMM, M, K, D, nnz, workspace_bytes=size), dl.describe_schedule(dl.OP_FUSED, 16384, 8192, 128, 16384 * 2457, workspace_bytes=1 << 40)
+    dl.set_tuning()
+    assert run["schedule"] == runs and "tile_columns" not in run and fused["schedule"] != "two_steps"
+    dl.set_tuning(stream_results=1)  # (not a schedule)
+    assert tiles()
+    dl.set_tuning()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,K,D,density", [(4097, 4095, 17, 0.9), (4100, 4097, 32, 0.9), (4095, 3841, 31, 0.95), (24576, 2048, 32, 0.25), (1983, 4097, 33, 0.9),
                                            (1985, 4095, 63, 0.6), (2111, 2303, 64, 0.9), (2049, 2305, 65, 0.5), (1023, 2048, 96, 0.9), (1025, 2304, 97, 0.6),
