@@ -323,7 +323,8 @@ class Probe:
 
         out = {"plain_call": one(None, 0), "empty_kernel_launch": empty(), "calls": calls}
         if prepared is not None:
-            out["prepared_call"] = one(prepared.memory.data_ptr() if prepared.memory is not None else None, prepared.size_and_hints)
+            pointer, size = prepared.for_call()
+            out["prepared_call"] = one(pointer, size)
         return out
 
     def gather_ceiling(self, torch, use_graph=True):
@@ -459,7 +460,7 @@ def measure(dl, torch, np, c, args, probe, steps, warmup, replays, ceiling_gbps,
     if not args.no_null:
         # the plain drop-in call (workspace = NULL, 0) in the same kind of graph, and what the preparation costs once per matrix
         k = min(steps, 500)
-        if prep is not None and (prep.memory is not None or prep.call_plan.hints):
+        if prep is not None and (prep.call_plan.bytes or prep.call_plan.hints):
             plain, _ = make_step(dl, torch, c, False)
             without = time_steps(torch, plain, k, min(warmup, 50), replays, not args.no_graph)
             r["null_call_us"] = round(without["per_step_s"] * 1e6, 3)

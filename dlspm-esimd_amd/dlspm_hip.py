@@ -335,6 +335,14 @@ class Prepared:
     def __init__(self, memory, size_and_hints, call_plan):
         self.memory, self.size_and_hints, self.call_plan = memory, size_and_hints, call_plan
 
+    def for_call(self):
+        """(pointer, size with hint bits) for one call of a compute entry point on the current stream. The pointer keeps memory of the
+        call's own; without room for that the pointer is None and the size holds the hints alone."""
+        if self.memory is not None:
+            return ctypes.c_void_p(self.memory.data_ptr()), self.size_and_hints
+        pointer, size = _own_memory(self.size_and_hints & ~HINT_MASK)
+        return pointer, self.size_and_hints & HINT_MASK | size
+
 
 def prepare(row_offsets, col_indices, K, op, width, info=None) -> Prepared:
     """The lead path of a caller: dlspm_analyze (unless `info` is given) -> dlspm_advise -> allocate -> build."""
@@ -442,10 +450,8 @@ def _workspace_args(workspace, plan, M, banded=False):
     if isinstance(plan, Prepared):
         if workspace is not None:
             raise ValueError("pass what prepare() returned or a workspace, not both")
-        if plan.memory is not None:
-            return ctypes.c_void_p(plan.memory.data_ptr()), plan.size_and_hints | hint
-        pointer, size = _own_memory(plan.size_and_hints & ~HINT_MASK)
-        return pointer, plan.size_and_hints & HINT_MASK | size | hint
+        pointer, size = plan.for_call()
+        return pointer, size | hint
     if isinstance(plan, CutPlan):
         if workspace is not None:
             raise ValueError("pass a row plan or a workspace, not both")

@@ -205,6 +205,7 @@ PyObject* call_sddmm(PyObject*, PyObject* const* args, Py_ssize_t npos, PyObject
             rhs->dim() != 2 || lhs->size(1) != rhs->size(1) || lhs->size(0) < c.M || rhs->size(0) > kMostInt ||
             rhs->size(1) > kMostInt || !c.output(a[4], {c.nnz}, *lhs))
             return fallback(DLSPM_OP_SDDMM, args, npos, kwnames);
+        c.own_memory(*lhs);
         const int K = (int)rhs->size(0), D = (int)rhs->size(1);
         const float *l = static_cast<const float*>(address(*lhs)), *r = static_cast<const float*>(address(*rhs));
         return c.run("sddmm_csr_f32", [&](void* stream) {

@@ -268,3 +268,26 @@ def test_values_too_small_for_their_parts(where, small):
     assert few.any() == (where == "A, results of few terms")
     # (down to the smallest ones, which one term makes: exact but for the rounding of the product)
     assert (np.abs(got - want)[few] <= 2.0 ** -23 * terms[few] + 2.0 ** -149).all()
+
+
+@pytest.mark.gpu
+def test_memory_for_a_call_of_the_c_entry_point():
+    """Prepared.for_call(): what a caller of the entry point passes, as the benchmark's host leg does, runs the schedule that
+    dlspm_describe_schedule names for the plan; a plan of another op is given memory by both kinds of Python call."""
+    import ctypes
+
+    import torch
+
+    M, K, N, density = SIZES[7]
+    ro, ci, va, B, rng = matrix(M, K, N, density, 2)
+    args = [torch.from_numpy(a).cuda() for a in (ro, ci, va, B)]
+    plan = dl.prepare(*args[:2], K, dl.OP_SPMM, N)
+    pointer, size = plan.for_call()
+    assert pointer.value and size == plan.size_and_hints
+    out, address = torch.empty((M, N), device="cuda"), lambda t: ctypes.c_void_p(t.data_ptr())
+    st = dl.lib().spmm_csr_f32(M, K, N, ci.size, *(address(t) for t in args), address(out), pointer, size, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert st == dl.OK and torch.equal(out, dl.spmm(*args, plan=plan)) and not torch.equal(out, dl.spmm(*args, workspace=dl.ROWS_EVEN))
+    lhs, rhs = torch.randn((M, 256), device="cuda"), torch.randn((K, 256), device="cuda")
+    assert torch.equal(dl.sddmm(*args[:2], lhs, rhs, plan=plan), dl._sddmm(*args[:2], lhs, rhs, plan=plan))
+    held = dl.prepare(*args[:2], K, dl.OP_SDDMM, 256)
+    assert held.memory is None or held.for_call()[0].value == held.memory.data_ptr()
