@@ -110,6 +110,9 @@ struct Call {
             memory = scratch.data_ptr();
         } catch (const c10::OutOfMemoryError&) {
             size_and_hints &= DLSPM_HINT_MASK;
+        } catch (...) {
+            Py_DECREF(result);
+            throw;
         }
     }
     // `given`, or a new tensor on `like`'s device

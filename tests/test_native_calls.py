@@ -150,3 +150,45 @@ def test_a_result_that_does_not_fit_is_out_of_memory(name):
     finally:
         torch.cuda.set_per_process_memory_fraction(1.0)
     assert not getattr(dl, name)(*args).any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["spmm", "fused"])
+def test_without_room_for_the_memory_of_a_call_it_runs_on_the_hints_alone(name):
+    """The memory that prepare() leaves to each call is for speed: a call whose own result has room runs without it, by both kinds of
+    call, with the bits of the call that passes the hints alone."""
+    import torch
+
+    M, K, N = (4096, 8192, 512) if name == "spmm" else (12288, 2048, 128)
+    keep = torch.rand((M, K), device="cuda") < 0.4
+    ro = torch.zeros(M + 1, dtype=torch.int32, device="cuda")
+    ro[1:] = keep.sum(1).cumsum(0)
+    ci = keep.nonzero()[:, 1].to(torch.int32)
+    del keep
+    r = lambda *s: torch.randn(s, device="cuda")  # noqa: E731
+    args = (ro, ci, r(ci.numel()), r(K, N)) if name == "spmm" else (ro, ci, r(M, N), r(K, N), r(K, N), 0.5)
+    plan = dl.prepare(ro, ci, K, dl.OP_SPMM if name == "spmm" else dl.OP_FUSED, N)
+    size = plan.size_and_hints & ~dl.HINT_MASK
+    assert plan.memory is None and size > 24 << 20 and plan.size_and_hints & dl.HINT_MASK == dl.HINT_ROWS_EVEN
+    calls = (getattr(dl, "_" + name), getattr(dl, name))
+    with_memory, hints_alone = calls[1](*args, plan=plan), calls[1](*args, workspace=dl.ROWS_EVEN)
+    assert not torch.equal(with_memory, hints_alone)
+    out = torch.empty_like(hints_alone)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    try:
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (2 << 20)) / total)
+        taken = []
+        with pytest.raises(torch.OutOfMemoryError):
+            while True:  # (what is free among the blocks in use)
+                taken.append(torch.empty((size,), dtype=torch.uint8, device="cuda"))
+        for call in calls:
+            out.zero_()
+            call(*args, out=out, plan=plan)
+            assert torch.equal(out, hints_alone), call
+        del taken
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    for call in calls:
+        assert torch.equal(call(*args, plan=plan), with_memory)
