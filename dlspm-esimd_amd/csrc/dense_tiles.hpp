@@ -4,7 +4,7 @@
 // floats is six of the nine products of the parts; the three left out are below 2^-26 of it. The matrix cores add up bf16 products
 // in 32 bits and do 16 times the multiplications per clock that they do in fp32: six for one is still 2.7 times the fp32 rate.
 // Errors against 64 bits, operands of normal distribution, the sums' order as in the kernels: dot products of 32 / 64 / 128
-// 3.8e-8 / 5.0e-8 / 5.0e-8, eight chains of fp32 fma 6.2e-8 / 7.2e-8 / 8.8e-8 (2.5e-8: rounded once).
+// 3.8e-8 / 4.3e-8 / 5.2e-8, eight chains of fp32 fma 6.2e-8 / 7.2e-8 / 8.8e-8 (2.5e-8: rounded once).
 // What the parts cannot hold: an infinity, a NaN or a value that rounds to infinity in bf16 makes the result NaN or infinite, and the
 // last part of a nonzero value below 2^-109 would be below bf16's smallest, which loses up to 2^-134 of it. The kernels compute
 // results that are not finite, and those that are not large against what such values can lose, from the floats themselves.

@@ -23,7 +23,9 @@
 // Measured (us, gathering kernels -> tiles): 24576 x 8192 at density 0.2, D = 32, three operand sets in turn 237 -> 163; one set, plain
 // calls: 8192 x 8192, D = 32 at 0.3 115 -> 58, D = 64 at 0.2 / 0.3 131 / 194 -> 69 / 74, D = 128 at 0.1 / 0.2 / 0.3 134 / 255 / 386 -> 109 /
 // 108 / 116; 30000 x 4093 at 0.2, D = 50 304 -> 139; 2048 x 2048 at 0.3, D = 128 24.7 -> 14.2. Against 64 bits the results are off by
-// 3.8 / 4.6 / 5.0 / 6.5e-8 at D = 32 / 50 / 64 / 128, the gathering kernels' by 6.2 / 6.9 / 7.2 / 8.8e-8.
+// 3.8 / 4.3 / 4.8 / 5.2e-8 at D = 32 / 64 / 96 / 128, the gathering kernels' by 6.2 / 7.2 / 8.0 / 8.8e-8; operands of one sign 3.4 / 3.8 / 3.9 /
+// 4.4e-8 and 4.1 / 4.2 / 4.3 / 4.5e-8. For the latter hi x hi has two chains of every second step above D = 32, and the last step's goes
+// behind the small products: in one chain of all steps the sums grow as they go, and so do their roundings (3.4 / 5.2 / 5.7 / 6.9e-8).
 // What bounds it: D = 128, the products (a wave spends 6 of the 7 us of a tile in them; 3 at the rate of products of constants, 4.5 at
 // what a large bf16 product of random numbers reaches here, 1.2 ... 1.35 PFLOP/s of 2.5: the chip lowers its clocks); D = 32, the
 // turns of computing (1.5 ... 2.5 us of 4 ... 5), waiting at the barrier and sampling, which two workgroups overlap only in part.
@@ -207,11 +209,11 @@ __global__ __launch_bounds__(kTileWaves * 64) __attribute__((amdgpu_waves_per_eu
     for (int i = 0; i < kRowsPerWave; ++i) load_columns(i);
 
     // ---- the wave's part of a tile: 64 rows x 32 columns
-    // the products of one step with the parts q0, q1 of the lhs rows 0 ... 31, 32 ... 63, smallest first; hi x hi into `sum`
+    // the products of one step with the parts q0, q1 of the lhs rows 0 ... 31, 32 ... 63, smallest first; hi x hi into `sum`, or none
     auto multiply = [&](const Parts& r, const Parts& q0, const Parts& q1, f32x16* small, f32x16* sum) {
         small[0] = mfma(r.lo, q0.hi, small[0]);
         small[1] = mfma(r.lo, q1.hi, small[1]);
-        if (sum) {
+        if (sum && sum != small) {
             sum[0] = mfma(r.hi, q0.hi, sum[0]);
             sum[1] = mfma(r.hi, q1.hi, sum[1]);
         }
@@ -223,6 +225,10 @@ __global__ __launch_bounds__(kTileWaves * 64) __attribute__((amdgpu_waves_per_eu
         small[1] = mfma(r.mid, q1.hi, small[1]);
         small[0] = mfma(r.hi, q0.mid, small[0]);
         small[1] = mfma(r.hi, q1.mid, small[1]);
+        if (sum == small) {
+            sum[0] = mfma(r.hi, q0.hi, sum[0]);
+            sum[1] = mfma(r.hi, q1.hi, sum[1]);
+        }
     };
     auto write_scores = [&](const f32x16* sum) {
 #pragma unroll
@@ -277,7 +283,7 @@ __global__ __launch_bounds__(kTileWaves * 64) __attribute__((amdgpu_waves_per_eu
         load_rhs(0, 1);
     }
     auto compute_long = [&](int tile) {
-        f32x16 small[2] = {}, sum[2] = {};
+        f32x16 small[2] = {}, sum[2][2] = {};
         unsigned long long few = few_ahead;
         few_ahead = 0;
 #pragma unroll
@@ -299,7 +305,7 @@ __global__ __launch_bounds__(kTileWaves * 64) __attribute__((amdgpu_waves_per_eu
 #pragma unroll
                     for (int i = 0; i < 8; ++i) next[i] = staged[1][i];
                 }
-                multiply(now, q0, q1, small, sum);
+                multiply(now, q0, q1, small, ks == KS - 1 ? small : sum[step]);
 #pragma unroll
                 for (int g = 0; g < 12; ++g) {
                     __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one product,
@@ -309,10 +315,11 @@ __global__ __launch_bounds__(kTileWaves * 64) __attribute__((amdgpu_waves_per_eu
                 __builtin_amdgcn_sched_barrier(0);  // (across steps the compiler would move loads far ahead, and spill)
             }
         }
-        sum[0] += small[0];
-        sum[1] += small[1];
+        f32x16 scores[2];
+#pragma unroll
+        for (int rt = 0; rt < 2; ++rt) scores[rt] = (small[rt] + sum[1][rt]) + sum[0][rt];
         __syncthreads();  // (the previous tile has been read)
-        write_scores(sum);
+        write_scores(scores);
         note_few(tile, few);
     };
 

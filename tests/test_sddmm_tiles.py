@@ -273,3 +273,27 @@ def test_hinted_stores_change_no_bit(torch_cuda, M, K, D, density):
         got.append(out[:ci.numel()].view(torch.int32))
     dl.set_tuning()
     assert torch.equal(*got) and bool((got[0].view(torch.float32).isnan() == (ci == K // 2)).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("what", ["both signs", "one sign", "unordered"])
+@pytest.mark.parametrize("M,K,D,density", [(16384, 64, 128, 0.9), (16384, 200, 64, 0.9), (4100, 4097, 32, 0.9), (2111, 2303, 64, 0.9), (1087, 2817, 128, 0.7),
+                                           (1983, 4097, 33, 0.9), (2049, 2305, 65, 0.5), (1025, 2304, 97, 0.6), (1000, 2000, 127, 0.9)])
+def test_a_single_tile_and_operands_of_one_sign(torch_cuda, M, K, D, density, what):
+    """Masks narrower than a tile, where waves lie beyond the last column; operands of one sign, where a bias in the rounding of the
+    matrix cores' sums would add up."""
+    torch = torch_cuda
+    ro, ci, row = mask(torch, M, K, density, 53)
+    lhs, rhs = operands(torch, M, K, D, 54)
+    if what == "one sign":
+        lhs, rhs = lhs.abs(), rhs.abs()
+    elif what == "unordered":
+        at = torch.arange(ci.numel(), device="cuda")
+        ci = torch.where(row % 3 == 0, ci[ro[:-1].long()[row] + ro[1:].long()[row] - 1 - at], ci).contiguous()
+    on, off = both(torch, ro, ci, lhs, rhs)
+    want, terms = exact(torch, lhs, rhs, row, ci), exact(torch, lhs.abs(), rhs.abs(), row, ci)
+    assert bool(((on.double() - want).abs() <= 2.0 ** -22 * terms).all())
+    assert error(on, want) <= error(off, want)
+    if what == "one sign":
+        # (were the sums not rounded to nearest, the mean would not be far below the errors)
+        assert 10 * abs(float(((on.double() - want) / want).mean())) <= error(off, want)
