@@ -291,3 +291,31 @@ def test_memory_for_a_call_of_the_c_entry_point():
     assert torch.equal(dl.sddmm(*args[:2], lhs, rhs, plan=plan), dl._sddmm(*args[:2], lhs, rhs, plan=plan))
     held = dl.prepare(*args[:2], K, dl.OP_SDDMM, 256)
     assert held.memory is None or held.for_call()[0].value == held.memory.data_ptr()
+
+
+# one slice and two: nothing is left to place behind the first fill, and every load of B ahead is of the same slice
+ONE_SLICE = [(16384, 100, 1024, 0.9), (16384, 128, 256, 0.9), (16384, 200, 1024, 0.5)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("what", ["ascending", "unordered", "one sign"])
+@pytest.mark.parametrize("M,K,N,density", ONE_SLICE + SIZES[2:4])
+def test_the_smallest_matrices_and_operands_of_one_sign(M, K, N, density, what):
+    """As test_edges_of_the_tiles. Operands of one sign: a bias in the rounding of the matrix cores' sums would add up."""
+    ro, ci, va, B, rng = matrix(M, K, N, density, 3 * M + N)
+    if what == "one sign":
+        va, B = np.abs(va), np.abs(B)
+    elif what == "unordered":
+        for r in range(5, M, 301):
+            order = rng.permutation(ro[r + 1] - ro[r])
+            ci[ro[r]:ro[r + 1]], va[ro[r]:ro[r + 1]] = ci[ro[r]:ro[r + 1]][order], va[ro[r]:ro[r + 1]][order]
+    got, other = run(ro, ci, va, B)
+    for rows in (slice(0, 70), slice(M // 2, M // 2 + 64), slice(M - 320, M)):
+        dense = np.zeros((rows.stop - rows.start, K))
+        for i, r in enumerate(range(rows.start, rows.stop)):
+            dense[i, ci[ro[r]:ro[r + 1]]] = va[ro[r]:ro[r + 1]]
+        want = dense @ B.astype(np.float64)
+        here, there = (np.linalg.norm(x[rows] - want) / np.linalg.norm(want) for x in (got, other))
+        assert here <= 1.02 * there and here <= 5e-8, (here, there)
+        if what == "one sign":  # (rounded once at the end, to nearest: no mean error to speak of)
+            assert abs(((got[rows] - want) / want).mean()) <= 5e-9

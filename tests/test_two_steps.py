@@ -187,3 +187,15 @@ def test_the_rule_holds_beside_powers_of_two():
     assert runs(17343, 3729, 128, 0.132) and runs(16075, 7628, 128, 0.305) and runs(4822, 6818, 96, 0.241) and runs(4676, 7785, 128, 0.212)
     assert not runs(2096, 7374, 128, 0.44) and not runs(7808, 7995, 96, 0.087) and not runs(23879, 3669, 64, 0.113) and not runs(17071, 7498, 32, 0.251)
     assert not runs(12772, 3715, 96, 0.135, even=False) and runs(28641, 1244, 64, 0.254, even=False)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K,D,density,second,even", CASES)
+def test_operands_of_one_sign(M, K, D, density, second, even):
+    (ro, ci, Q, Km, V), rng = operands(M, K, D, density, M - D)
+    args = ro, ci, np.abs(Q), np.abs(Km), np.abs(V)
+    got, other = run(args, 0.125, second, even)
+    rows = np.concatenate((np.arange(70), np.arange(M - 70, M)))
+    want = exact(args, 0.125, rows)
+    here, there = (np.linalg.norm(x[rows] - want) / np.linalg.norm(want) for x in (got, other))
+    assert here <= 1.02 * there, (here, there)
