@@ -559,7 +559,7 @@ static WorkspaceArg behind_scores(const WorkspaceArg& ws, int nnz)
 }
 static bool fused_two_steps(const DeviceInfo& dev, int M, int K, int D, int nnz, const WorkspaceArg& ws, FusedCall& c)
 {
-    if (!ws.mem || ws.bytes < scores_bytes(nnz)) return false;
+    if (!ws.mem || ws.bytes < scores_bytes(nnz) || !rule_on(kRuleTwoSteps)) return false;
     c.tiles = sddmm_tiles_plan(dev, M, K, D, nnz);
     if (c.tiles.ranges == 0) return false;
     c.second = spmm_decide(dev, M, K, D, nnz, behind_scores(ws, nnz));
@@ -644,7 +644,7 @@ int dlspm_set_tuning(const dlspm_tuning* t)
         t->tile_major < -1 || t->tile_major > 3 || t->tile_width < 0 || t->plan_order < 0 || t->plan_order > 2 ||
         t->xcd_contiguous < 0 || t->xcd_contiguous > 1 || t->stream_results < -1 || t->stream_results > 1 ||
         (t->cut_piece_pct != 0 && (t->cut_piece_pct < 10 || t->cut_piece_pct > 1000)) ||
-        (t->cut_longest_pct != 0 && (t->cut_longest_pct < 10 || t->cut_longest_pct > 1000)) || t->rules_off < 0 || t->rules_off > 8191 ||
+        (t->cut_longest_pct != 0 && (t->cut_longest_pct < 10 || t->cut_longest_pct > 1000)) || t->rules_off < 0 || t->rules_off > kRules ||
         (t->compute_units != 0 && (t->compute_units < 8 || t->compute_units > 1024 || t->compute_units % 8 != 0)))
         return DLSPM_E_INVALID_ARG;
     t_tuning.split_w = t->split_w;

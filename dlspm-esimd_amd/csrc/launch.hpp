@@ -102,7 +102,7 @@ struct Tuning {
 constexpr int kRuleEightWavesFewRows = 1, kRuleSixteenWavesTallLongRows = 2, kRuleMoreWavesFewLongRows = 4, kRuleGroupRows = 8,
               kRuleRowAlignedSplit = 16, kRulePlanUngroups = 32, kRuleExactWidthKernels = 64, kRuleCutRowsByColumns = 128,
               kRuleFinerColumnTiles = 256, kRuleRowPiecesFewRows = 512, kRuleMaskByRange = 1024, kRuleResidentSlices = 2048,
-              kRuleDenseGroups = 4096;
+              kRuleDenseGroups = 4096, kRuleSddmmTiles = 8192, kRuleSpmmTiles = 16384, kRuleTwoSteps = 32768, kRules = 65535;
 
 const Tuning& tuning();
 inline bool rule_on(int rule) { return (tuning().rules_off & rule) == 0; }

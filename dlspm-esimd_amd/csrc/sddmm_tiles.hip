@@ -519,7 +519,7 @@ TilePlan sddmm_tiles_choose(const DeviceInfo& dev, int M, int K, int D, int nnz)
 {
     const TilePlan best = sddmm_tiles_plan(dev, M, K, D, nnz);
     const double gathered = 32.0 * (double)ceil_div(D, 32) * (D % 4 == 0 ? 1.0 : D <= 24 ? 1.04 : 1.2);
-    return best.us < 0.9 * (2.0 + (double)nnz * (2.2 + 0.122 * gathered) * 1e-6) ? best : TilePlan{0, 0.0};
+    return rule_on(kRuleSddmmTiles) && best.us < 0.9 * (2.0 + (double)nnz * (2.2 + 0.122 * gathered) * 1e-6) ? best : TilePlan{0, 0.0};
 }
 
 void sddmm_tile_shape(int* rows, int* columns)

@@ -485,7 +485,7 @@ double spmm_tiles_us(const DeviceInfo& dev, int M, int K, int N, int nnz)
 bool spmm_tiles_choose(const DeviceInfo& dev, int M, int K, int N, int nnz, double other_us)
 {
     const Tuning& t = tuning();
-    if (!rule_on(kRuleDenseGroups) || N < 4 || M <= 0 || K <= 0 || nnz <= 0 || nnz >= (1 << 29) || K > kMostColumns || !dense_fits_buffer(K, N)) return false;
+    if (!rule_on(kRuleDenseGroups) || !rule_on(kRuleSpmmTiles) || N < 4 || M <= 0 || K <= 0 || nnz <= 0 || nnz >= (1 << 29) || K > kMostColumns || !dense_fits_buffer(K, N)) return false;
     // (a schedule that was asked for by name)
     if (t.split_w > 0 || t.flat >= 0 || t.slices >= 0 || t.tile_major >= 0 || t.tile_width > 0 || t.plan_order > 0 || t.xcd_contiguous) return false;
     return spmm_tiles_us(dev, M, K, N, nnz) < 0.9 * other_us;

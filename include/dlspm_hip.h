@@ -450,8 +450,11 @@ typedef struct dlspm_tuning {
                                                    /* whose range check zeroes the lanes past D, where rhs fits (else: by selects); */
                                                    /* the fused op's first stage likewise at D = 260 ... 380                      */
 #define DLSPM_RULE_RESIDENT_SLICES           2048  /* SpMM on dense enough matrices: slices of B in LDS, whatever memory the call has  */
-#define DLSPM_RULE_DENSE_GROUPS              4096  /* fused op, D = 36 ... 128, large calls: sixteen rows whose columns form one run on the  */
-                                                   /* matrix cores; SDDMM (D = 17 ... 128) and SpMM with memory: dense tiles  */
+#define DLSPM_RULE_DENSE_GROUPS              4096  /* everything on the matrix cores: the three below, and the fused op at D = 36 ... 128, */
+                                                   /* large calls: sixteen rows whose columns form one run                    */
+#define DLSPM_RULE_SDDMM_TILES               8192  /* SDDMM (D = 17 ... 128) on masks dense enough: dense tiles               */
+#define DLSPM_RULE_SPMM_TILES               16384  /* SpMM with memory and the even-rows hint: dense tiles                    */
+#define DLSPM_RULE_TWO_STEPS                32768  /* fused op with memory, D = 17 ... 128: SDDMM on dense tiles, then SpMM    */
 void dlspm_tuning_default(dlspm_tuning* t);   /* fills *t with "follow the rules" */
 int dlspm_set_tuning(const dlspm_tuning* t);  /* DLSPM_OK or DLSPM_E_INVALID_ARG (a field out of range) */
 int dlspm_get_tuning(dlspm_tuning* t);        /* what the calling thread's launches currently use */

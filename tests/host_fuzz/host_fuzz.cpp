@@ -67,7 +67,7 @@ int main()
             tune.compute_units = units[rng() % 6];
             tune.cut_piece_pct = pcts[rng() % 6];
             tune.cut_longest_pct = pcts[rng() % 6];
-            tune.rules_off = (int)(rng() % 8192);
+            tune.rules_off = (int)(rng() % 65536);
             if (dlspm_set_tuning(&tune) != DLSPM_OK) return 1;
         }
         const int op = (int)(rng() % 3);

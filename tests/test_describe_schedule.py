@@ -84,3 +84,23 @@ def test_what_is_described_is_what_runs(M, K, N, density, way):
     dl.set_tuning(rules_off=dl.RULES["resident_slices"])
     there = dl.spmm(*args, **kwargs)
     assert (named == "resident") == (not torch.equal(here, there))
+
+
+def test_what_runs_on_the_matrix_cores_has_a_switch_each():
+    M, K, nnz, size = 16384, 8192, 16384 * 2457, 1 << 40
+    memory = size | dl.HINT_ROWS_EVEN
+
+    def run(off):
+        dl.set_tuning(rules_off=sum(dl.RULES[name] for name in off))
+        sddmm = dl.describe_schedule(dl.OP_SDDMM, M, K, 128, nnz)
+        spmm = dl.describe_schedule(dl.OP_SPMM, M, K, 128, nnz, workspace_bytes=memory)
+        fused = dl.describe_schedule(dl.OP_FUSED, M, K, 128, nnz, workspace_bytes=memory)
+        groups = dl.describe_schedule(dl.OP_FUSED, M, M, 128, M * 128)
+        dl.set_tuning()
+        return "tile_columns" in sddmm, spmm["schedule"], fused.get("second"), groups["schedule"]
+
+    assert run([]) == (True, "dense_tiles", "dense_tiles", "dense_groups")
+    assert run(["sddmm_tiles"]) == (False, "dense_tiles", "dense_tiles", "dense_groups")
+    assert run(["spmm_tiles"]) == (True, "resident", "resident", "dense_groups")
+    assert run(["two_steps"]) == (True, "dense_tiles", None, "dense_groups")
+    assert run(["dense_groups"]) == (False, "resident", None, "row_blocks")
