@@ -1,8 +1,9 @@
 // Products of 32-bit floats on the bf16 matrix cores, for masks and matrices dense enough to be computed as dense tiles.
 //
 // A float is the sum of three bf16 (8 + 8 + 8 significand bits, each rounded to nearest: nothing is left), and a product of two
-// floats is six of the nine products of the parts; the three left out are below 2^-26 of it. The matrix cores add up bf16 products
-// in 32 bits and do 16 times the multiplications per clock that they do in fp32: six for one is still 2.7 times the fp32 rate.
+// floats is six of the nine products of the parts; the three left out come to 2^-24 of it at most, as a rule to 2^-27. The matrix cores
+// add up bf16 products in 32 bits and do 16 times the multiplications per clock that they do in fp32: six for one is still 2.7 times
+// the fp32 rate.
 // Errors against 64 bits, operands of normal distribution, the sums' order as in the kernels: dot products of 32 / 64 / 128
 // 3.8e-8 / 4.3e-8 / 5.2e-8, eight chains of fp32 fma 6.2e-8 / 7.2e-8 / 8.8e-8 (2.5e-8: rounded once).
 // What the parts cannot hold: an infinity, a NaN or a value that rounds to infinity in bf16 makes the result NaN or infinite, and the
@@ -56,15 +57,6 @@ __device__ __forceinline__ Parts split_parts(const float* x, unsigned long long&
 __device__ __forceinline__ f32x16 mfma(const bf16x8& a, const bf16x8& b, const f32x16& c)
 {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-}
-// the products other than hi x hi, smallest first
-__device__ __forceinline__ f32x16 mfma_small(const Parts& a, const Parts& b, f32x16 c)
-{
-    c = mfma(a.lo, b.hi, c);
-    c = mfma(a.mid, b.mid, c);
-    c = mfma(a.hi, b.lo, c);
-    c = mfma(a.mid, b.hi, c);
-    return mfma(a.hi, b.mid, c);
 }
 
 }  // namespace dlspm

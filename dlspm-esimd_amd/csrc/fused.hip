@@ -353,7 +353,7 @@ __global__ __launch_bounds__(W * 64) void fused_kernel(int M, int D, int col_til
 }
 
 // The same with groups of sixteen rows on the matrix cores where their columns form one run (fused_dense_group): a kernel of its
-// own, because what that needs -- 20 KB of LDS and more registers -- takes a wave per SIMD from calls that have no such groups.
+// own, because what that needs -- 24 ... 28 KB of LDS and more registers -- takes a wave per SIMD from calls that have no such groups.
 // Four waves per SIMD at least: left to itself the compiler keeps the chains in accumulation registers and ends at two or three
 // (16384 rows, 128 columns per row, D = 128: 40.5 us, D = 64: 26.7 us; with four 38.6 and 21.4 us, as the kernel was then).
 template <int VEC, int G1, int DS, int MASKED, int G, int V2, int W, int R>

@@ -470,11 +470,11 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(2,
 // Tiles for these sizes: where their estimated time is below 0.9 of `other_us`, that of the schedule which needs no memory. The estimate
 // (us): the split of B, and rounds of one workgroup per compute unit x (5 + slices x (2.95, from a density of 0.3 on 7 more per unit of
 // density, where rows have more than 64 pairs in a slice)). Measured / estimated, and the resident schedule: 16384 x 8192, N = 128 at 0.2 /
-// 0.3 / 0.5 204 / 206 / 291 (206 / 206 / 295) and 266 / 327 / 496; 8192 x 8192 at 0.3, N = 128 190 (206, on half of the units) and 187, N = 256
-// 194 (211) and 323; 32768 x 8192 at 0.3, N = 64 400 (399) and 340; 2000 x 4608 at 0.3, N = 3136 440 (488) and 703. Uneven rows (lognormal,
+// 0.3 / 0.5 204 / 206 / 291 (203 / 203 / 293) and 266 / 327 / 496; 8192 x 8192 at 0.3, N = 128 190 (203, on half of the units) and 187, N = 256
+// 194 (206) and 323; 32768 x 8192 at 0.3, N = 64 400 (395) and 340; 2000 x 4608 at 0.3, N = 3136 440 (494) and 703. Uneven rows (lognormal,
 // sigma 0.6) gain less, since a row of many pairs makes its wave come back to four rows and the others wait: 32768 x 8192 at 0.3 660 -> 545,
 // 12288 x 4096 at 0.3, N = 200 241 -> 240. The row blocks are dealt to the XCDs with all their column tiles: 85 of them in three make 33
-// workgroups for the 32 units of some, two rounds (5408 x 1340 at 0.25, N = 311: 79, resident 60).
+// workgroups for the 32 units of some, two rounds (5408 x 1340 at 0.25, N = 311: 79, estimated 82, resident 60).
 double spmm_tiles_us(const DeviceInfo& dev, int M, int K, int N, int nnz)
 {
     const double density = (double)nnz / ((double)M * K), slice_us = 2.95 + 7.0 * std::max(0.0, density - 0.3);

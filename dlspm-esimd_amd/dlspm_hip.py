@@ -539,7 +539,8 @@ def _sddmm(row_offsets, col_indices, lhs, rhs, out=None, workspace=None, plan=No
 
 
 def _fused(row_offsets, col_indices, Q, Kmat, V, scale=1.0, out=None, workspace=None, plan=None, banded=False):
-    """O = (S .* (Q Kmat^T) * scale) V on the current stream (fused_sddmm_spmm_f32); the scores are never stored.
+    """O = (S .* (Q Kmat^T) * scale) V on the current stream (fused_sddmm_spmm_f32). The scores are not stored, except on
+    dense masks with a plan from prepare(), where two steps pass them through memory of the call's own (4 bytes per nonzero).
     `workspace`: optional GPU tensor of at least workspace_bytes(OP_FUSED, ...) bytes, or ROWS_EVEN.
     `plan`: optional row plan of the mask (row_plan()), passed as the workspace with DLSPM_HINT_ROW_PLAN."""
     import torch

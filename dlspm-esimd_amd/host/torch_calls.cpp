@@ -268,8 +268,8 @@ PyMethodDef kMethods[] = {
      "those of spmm()."},
     {"fused", (PyCFunction)(void*)call_fused, METH_FASTCALL | METH_KEYWORDS,
      "fused($module, row_offsets, col_indices, Q, Kmat, V, scale=1.0, out=None, workspace=None, plan=None, banded=False)\n--\n\n"
-     "O = (S .* (Q Kmat^T) * scale) V on the current stream (fused_sddmm_spmm_f32); the scores are never stored; the\n"
-     "options are those of spmm()."},
+     "O = (S .* (Q Kmat^T) * scale) V on the current stream (fused_sddmm_spmm_f32); the scores are not stored, except\n"
+     "on dense masks with a plan from prepare(), through memory of the call's own; the options are those of spmm()."},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_dlspm_torch", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};
 

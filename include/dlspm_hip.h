@@ -38,10 +38,11 @@
  *         exceed one L2 (the column ranges of the sparse matrix one after the other, so that the part of the operands in
  *         use fits the cache; partial rows per range in the workspace, added in range order; SDDMM keeps only the range
  *         boundaries there).
- *       DLSPM_HINT_ROWS_EVEN, with workspace NULL: the caller knows that no row is much longer than the mean (longest
+ *       DLSPM_HINT_ROWS_EVEN: the caller knows that no row is much longer than the mean (longest
  *         row at most one and a half times nnz / M). Tall matrices of long rows then run one whole row per wave, which
  *         is the faster split for even rows and the slower one for uneven rows. A hint about speed only: a wrong one
- *         costs time, never correctness (a row's products are added in a different, equally fixed order).
+ *         costs time, never correctness (a row's products are added in a different, equally fixed order). Memory that comes
+ *         with it is used, and written, by the dense tiles and the two steps below only.
  *       Matrices dense enough that each row of B serves many rows of a workgroup (from a density of about 0.05 on under the
  *         even-rows hint, about 0.15 otherwise) are multiplied from slices of B in LDS where that is estimated to be faster;
  *         memory or a plan that comes with such a call is not used. Large ones under the even-rows hint are multiplied as dense
@@ -140,7 +141,8 @@ int sddmm_csr_f32(int M, int K, int D, int nnz,
                   void* workspace, size_t workspace_bytes, void* stream);
 
 /*
- * O[M x D] = (S .* (Q * Kmat^T) * scale) * V, with the sampled scores kept on chip.
+ * O[M x D] = (S .* (Q * Kmat^T) * scale) * V, with the sampled scores kept on chip (on dense masks with memory for them: 4 bytes per
+ * nonzero, written by one step and read by the next; see `workspace` above).
  * Replaces `FusedEsimd(a_row_offsets, a_column_indices, c, b, d, e, item)` of
  * FUSED/fused-esimd_cb.cpp:100-189 (launch :318-331; c->Q, b->Kmat, d->V, e->O) and computes what
  * Sddmm followed by Spmm compute in FUSED/fused.cpp:47-89. scale = 1.0f gives exactly the
@@ -220,7 +222,8 @@ int dlspm_csr_check(int M, int K, int nnz, const int* row_offsets, const int* co
  *       spmm_csr_f32(M, K, N, nnz, ..., ws, cp.bytes | cp.hints, stream);    // as often as the structure is used
  * The finer-grained queries below (dlspm_csr_row_stats, dlspm_workspace_advice, dlspm_row_plan_advice,
  * dlspm_describe_*) remain for callers that know their matrices and for tuning reports; the two advices answer for row
- * blocks, also where a call would be multiplied from slices of B in LDS.
+ * blocks, also where a call would be multiplied from slices of B in LDS or run on dense tiles: they may name memory or a plan that
+ * such a call does not look at (and refuses all the same with DLSPM_E_WORKSPACE where it is smaller than they say).
  * No counterpart in the reference, whose launch sizing needs no knowledge of the matrix (SPMM/spmmesimd2.hpp:30-60) and
  * takes the rows as they come.
  */
