@@ -244,21 +244,25 @@ inline PreparedCall prepare_call(const Options& opt, int op, int M, int K, int w
                                  passing == DLSPM_PASS_ROWS_EVEN ? DLSPM_HINT_ROWS_EVEN : 0};
         }
     }
-    int slices = 0;
-    (void)dlspm_describe_slices(op, M, K, width, nnz, &slices, nullptr);
-    std::printf("rows: longest %d, mean %.1f, empty %d; columns: widest row %d, eighths span %.2f x K -> %s%s%s\n", mi.max_row_len,
+    int schedule[4] = {};
+    (void)dlspm_describe_schedule(op, M, K, width, nnz, cp.bytes | cp.hints, schedule);
+    std::printf("rows: longest %d, mean %.1f, empty %d; columns: widest row %d, eighths span %.2f x K -> %s%s%s%s\n", mi.max_row_len,
                 (double)nnz / M, mi.empty_rows, mi.max_col_span, mi.eighths_cover_permille * 1e-3,
                 opt.workspace == Options::kAlways           ? "workspace passed (--workspace)"
                 : cp.build == DLSPM_BUILD_CUT_PLAN          ? "a row above one and a half shares, cut plan (long rows handed out in pieces)"
                 : cp.build == DLSPM_BUILD_ROW_PLAN          ? "uneven, row plan (one row per workgroup, handed out by length)"
                 : (cp.hints & DLSPM_HINT_BANDED)            ? "banded, DLSPM_HINT_BANDED passed"
-                : cp.bytes && slices > 0                    ? "dense operands beyond one L2, workspace passed (column-sliced schedule)"
-                : cp.bytes                                  ? "uneven, workspace passed (flat schedule)"
                 : (cp.hints & DLSPM_HINT_ROWS_EVEN)         ? "even, DLSPM_HINT_ROWS_EVEN passed"
+                : cp.bytes && schedule[0] == DLSPM_SCHEDULE_TWO_STEPS ? "workspace passed"
+                : cp.bytes && schedule[0] == DLSPM_SCHEDULE_SLICED    ? "dense operands beyond one L2, workspace passed (column-sliced schedule)"
+                : cp.bytes                                  ? "uneven, workspace passed (flat schedule)"
                 : (cp.hints & DLSPM_HINT_ROWS_SKEWED)       ? "long rows next to each other, fewer rows per workgroup"
                                                             : "nothing passed",
                 (cp.hints & DLSPM_HINT_BANDED) && (cp.hints & DLSPM_HINT_ROWS_EVEN) ? " with DLSPM_HINT_ROWS_EVEN" : "",
-                (cp.hints & DLSPM_HINT_ROWS_SKEWED) ? " with DLSPM_HINT_ROWS_SKEWED" : "");
+                (cp.hints & DLSPM_HINT_ROWS_SKEWED) ? " with DLSPM_HINT_ROWS_SKEWED" : "",
+                schedule[0] == DLSPM_SCHEDULE_DENSE_TILES  ? " (dense tiles)"
+                : schedule[0] == DLSPM_SCHEDULE_TWO_STEPS ? " (two steps: scores of dense tiles, then their products)"
+                                                          : "");
     pc.memory = DevBuf<char>(cp.bytes);
     pc.hints = cp.hints;
     pc.build = cp.build;

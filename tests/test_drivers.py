@@ -406,6 +406,17 @@ def test_drivers_pass_the_workspace_only_for_uneven_rows():
 
 
 @pytest.mark.gpu
+def test_drivers_say_that_dense_tiles_and_two_steps_run():
+    """Memory beside the even-rows hint is for dense tiles (SpMM) and for the two steps of the fused op, which also take it
+    without the hint: not a sign of uneven rows, and no flat schedule."""
+    for app, says, *shape in (("spmm_run", "even, DLSPM_HINT_ROWS_EVEN passed (dense tiles)", 16384, 4096, 128, 0.3),
+                              ("fused_run", "even, DLSPM_HINT_ROWS_EVEN passed (two steps", 8192, 2048, 128, 0.3),
+                              ("fused_run", "workspace passed (two steps", 8192, 2048, 128, 0.3, "--sigma", 0.6)):
+        rc, out = run(app, "--shape", *shape, "--iters", 3)
+        assert rc == 0 and "PASS" in out and "-> " + says in out and "workspace:" in out, out
+
+
+@pytest.mark.gpu
 def test_spmm_driver_builds_a_row_plan_for_small_uneven_matrices():
     """The headline configuration (2048 x 512, lognormal rows, one row per workgroup): the driver builds the row plan
     once and launches spmm_csr_f32 with it; with --no-plan, or on even rows, it does not; all self-check."""
