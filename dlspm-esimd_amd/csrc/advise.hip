@@ -175,13 +175,14 @@ using namespace dlspm;
 
 extern "C" {
 
-int dlspm_analyze(int M, int K, int nnz, const int* row_offsets, const int* col_indices, void* stream, dlspm_matrix_info* info)
+int dlspm_analyze_details(int M, int K, int nnz, const int* row_offsets, const int* col_indices, void* stream, dlspm_matrix_details* details)
 {
-    if (!info || M < 0 || K < 0 || nnz < 0) return DLSPM_E_INVALID_ARG;
+    if (!details || M < 0 || K < 0 || nnz < 0) return DLSPM_E_INVALID_ARG;
     if ((long long)nnz > (long long)M * K) return DLSPM_E_INVALID_ARG;
     if (M > 0 && !row_offsets) return DLSPM_E_INVALID_ARG;
     if (nnz > 0 && !col_indices) return DLSPM_E_INVALID_ARG;
-    *info = dlspm_matrix_info{};
+    *details = dlspm_matrix_details{};
+    dlspm_matrix_info* const info = &details->shape;
     info->M = M;
     info->K = K;
     info->nnz = nnz;
@@ -231,10 +232,19 @@ int dlspm_analyze(int M, int K, int nnz, const int* row_offsets, const int* col_
         total += h[3 + 2 * kEighths + x];
     }
     info->eighths_cover_permille = K > 0 ? (int)std::min<long long>(cover * 1000 / K, 1000ll * kEighths) : 0;
-    info->unordered_rows = h[kUnordered];
-    info->heaviest_64_rows = h[kHeaviest];
     info->eighths_nnz_permille = total > 0 ? (int)std::min<long long>(heaviest * 1000 * kEighths / total, 1000ll * kEighths) : 0;
+    details->unordered_rows = h[kUnordered];
+    details->heaviest_64_rows = h[kHeaviest];
     return DLSPM_OK;
+}
+
+int dlspm_analyze(int M, int K, int nnz, const int* row_offsets, const int* col_indices, void* stream, dlspm_matrix_info* info)
+{
+    if (!info) return DLSPM_E_INVALID_ARG;
+    dlspm_matrix_details details;
+    const int status = dlspm_analyze_details(M, K, nnz, row_offsets, col_indices, stream, &details);
+    if (status != DLSPM_E_INVALID_ARG) *info = details.shape;
+    return status;
 }
 
 // A band: every XCD, handed a contiguous eighth of the rows, gathers from about its own eighth of the K-side operand
@@ -252,6 +262,13 @@ constexpr int kClusteredEighthPermille = 1600;  // (1000: every eighth of the ro
 
 int dlspm_advise(int op, int N_or_D, const dlspm_matrix_info* info, dlspm_call_plan* plan)
 {
+    const dlspm_matrix_details details{info ? *info : dlspm_matrix_info{}, 0, 0};
+    return dlspm_advise_details(op, N_or_D, info ? &details : nullptr, plan);
+}
+
+int dlspm_advise_details(int op, int N_or_D, const dlspm_matrix_details* details, dlspm_call_plan* plan)
+{
+    const dlspm_matrix_info* const info = details ? &details->shape : nullptr;
     if (!info || !plan || N_or_D < 0) return DLSPM_E_INVALID_ARG;
     if (op != DLSPM_OP_SPMM && op != DLSPM_OP_SDDMM && op != DLSPM_OP_FUSED) return DLSPM_E_INVALID_ARG;
     *plan = dlspm_call_plan{DLSPM_BUILD_NOTHING, 0, 0};
@@ -270,14 +287,14 @@ int dlspm_advise(int op, int N_or_D, const dlspm_matrix_info* info, dlspm_call_p
     // (fused, all rows shuffled, the schedules below / two steps: 16384 x 4096 at 0.2, D = 64 224 / 320 us, 12288 x 2048 at 0.3, D = 128 240 / 518,
     // 32768 x 8192 at 0.3, D = 32 900 / 1570): not more than one in sixteen, except in place of column slices, which want them to ascend
     // too (8192 x 8192, D = 128 at 0.2 / 0.3 955 / 657 and 1423 / 958, 16384 x 8192 at 0.2 1888 / 1520).
-    const bool ascend = 16ll * info->unordered_rows <= M;
+    const bool ascend = 16ll * details->unordered_rows <= M;
     int slices = 0;
     (void)dlspm_describe_slices(op, M, K, N_or_D, nnz, &slices, nullptr);
     // Workgroups that own 64 rows and more end when the heaviest does. Heaviest 64 rows / mean, and the time of the row plan or slices / of two
     // steps: all nonzeros in full rows at the top (5.0) 16384 x 8192 at 0.2, D = 128 838 / 1217, (3.3) 12288 x 2048 at 0.3 236 / 305, 32768 x 8192
     // at 0.3, D = 32 860 / 1299; a triangle (2.0) 860 / 667, 239 / 216, and at D = 32 862 / 918; full rows anywhere (1.6) 985 / 678,
     // 237 / 198, at D = 32 856 / 862; lognormal rows, sigma 1 (1.5) 885 / 550, 215 / 150.
-    const double heavy = info->heaviest_64_rows > 0 ? (double)info->heaviest_64_rows * M / (64.0 * nnz) : info->eighths_nnz_permille * 1e-3;
+    const double heavy = details->heaviest_64_rows > 0 ? (double)details->heaviest_64_rows * M / (64.0 * nnz) : info->eighths_nnz_permille * 1e-3;
     // 2. the fused op on dense masks: memory for the scores between its two steps (never less than what the call would refuse)
     if (op == DLSPM_OP_FUSED && (ascend || slices > 0) && (even || heavy <= (N_or_D <= 32 ? 1.5 : 2.5))) {
         const size_t bytes = fused_two_steps_bytes(dev, M, K, N_or_D, nnz, even);

@@ -72,6 +72,8 @@ EXPORTS = (
     "dlspm_row_plan_bytes_for",
     "dlspm_analyze",
     "dlspm_advise",
+    "dlspm_analyze_details",
+    "dlspm_advise_details",
     "dlspm_row_plan_build_cut",
     "dlspm_tuning_default",
     "dlspm_set_tuning",
@@ -98,7 +100,7 @@ RULES = {"eight_waves_few_rows": 1, "sixteen_waves_tall_long_rows": 2, "more_wav
 
 
 class MatrixInfo(ctypes.Structure):
-    """dlspm_matrix_info of include/dlspm_hip.h."""
+    """dlspm_matrix_details of include/dlspm_hip.h: a dlspm_matrix_info, and two figures behind it."""
     _shape = ("M", "K", "nnz", "max_row_len", "empty_rows", "max_col_span", "eighths_cover_permille", "eighths_nnz_permille")
     _fields_ = [(n, ctypes.c_int) for n in (*_shape, "unordered_rows", "heaviest_64_rows")]
 
@@ -168,6 +170,10 @@ def lib() -> ctypes.CDLL:
         L.dlspm_analyze.restype = ci
         L.dlspm_advise.argtypes = [ci, ci, ctypes.POINTER(MatrixInfo), ctypes.POINTER(CallPlan)]
         L.dlspm_advise.restype = ci
+        L.dlspm_analyze_details.argtypes = L.dlspm_analyze.argtypes
+        L.dlspm_analyze_details.restype = ci
+        L.dlspm_advise_details.argtypes = L.dlspm_advise.argtypes
+        L.dlspm_advise_details.restype = ci
         L.spmm_csr_f32_static.argtypes = [ci, ci, ci, ci, vp, vp, vp, vp, vp, vp]
         L.spmm_csr_f32_static.restype = ci
         L.dlspm_static_scratch_bytes.restype = sz
@@ -307,29 +313,29 @@ def cut_plan(row_offsets, op, width, out=None) -> CutPlan:
 
 
 def analyze(row_offsets, col_indices, K) -> MatrixInfo:
-    """dlspm_analyze: one synchronising pass over the CSR structure on the GPU."""
+    """dlspm_analyze_details: one synchronising pass over the CSR structure on the GPU."""
     import torch
 
     M, nnz = row_offsets.numel() - 1, col_indices.numel()
     info = MatrixInfo()
-    st = lib().dlspm_analyze(M, K, nnz, _ptr(row_offsets, torch.int32, "row_offsets", M + 1),
-                             _ptr(col_indices, torch.int32, "col_indices"), _stream(), ctypes.byref(info))
+    st = lib().dlspm_analyze_details(M, K, nnz, _ptr(row_offsets, torch.int32, "row_offsets", M + 1),
+                                     _ptr(col_indices, torch.int32, "col_indices"), _stream(), ctypes.byref(info))
     if st != OK:
-        raise DlspmError(st, "dlspm_analyze")
+        raise DlspmError(st, "dlspm_analyze_details")
     return info
 
 
 def advise(op, width, info: MatrixInfo) -> CallPlan:
-    """dlspm_advise (host only): what to allocate, build and hint for op at this dense width."""
+    """dlspm_advise_details (host only): what to allocate, build and hint for op at this dense width."""
     cp = CallPlan()
-    st = lib().dlspm_advise(op, width, ctypes.byref(info), ctypes.byref(cp))
+    st = lib().dlspm_advise_details(op, width, ctypes.byref(info), ctypes.byref(cp))
     if st != OK:
-        raise DlspmError(st, "dlspm_advise")
+        raise DlspmError(st, "dlspm_advise_details")
     return cp
 
 
 class Prepared:
-    """What dlspm_advise said for one matrix, op and width, allocated and built (prepare()): pass as plan=... . A size without
+    """What advise() said for one matrix, op and width, allocated and built (prepare()): pass as plan=... . A size without
     memory is that of memory which each call takes from PyTorch's allocator (B's parts for dense tiles, the scores between two steps)."""
 
     def __init__(self, memory, size_and_hints, call_plan):
@@ -345,7 +351,7 @@ class Prepared:
 
 
 def prepare(row_offsets, col_indices, K, op, width, info=None) -> Prepared:
-    """The lead path of a caller: dlspm_analyze (unless `info` is given) -> dlspm_advise -> allocate -> build."""
+    """The lead path of a caller: analyze() (unless `info` is given) -> advise() -> allocate -> build."""
     import torch
 
     info = info if info is not None else analyze(row_offsets, col_indices, K)

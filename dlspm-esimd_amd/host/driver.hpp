@@ -207,17 +207,17 @@ struct Options {
     int iters = 20;  // the reference keeps the minimum of 20 launches (SPMM/spmm-esimd-fromfile2.cpp:194-243)
     bool cold = false;
     int graph = 0;  // --graph n: also time a HIP graph of n launches, replayed five times (no event between the launches)
-    // what to pass as `workspace`: by default what dlspm_advise says after one look at the matrix (dlspm_analyze);
+    // what to pass as `workspace`: by default what dlspm_advise_details says after one look at the matrix (dlspm_analyze_details);
     // --workspace: always the schedule memory of dlspm_workspace_bytes, --no-workspace: always NULL
     enum Workspace { kAuto, kAlways, kNever } workspace = kAuto;
-    bool plan = true;  // build a row plan or a cut plan where dlspm_advise says so (--no-plan: never)
+    bool plan = true;  // build a row plan or a cut plan where dlspm_advise_details says so (--no-plan: never)
     std::string csv, dump;
     std::string dump_each;  // --dump-each DIR: every case dumps into its own sub-directory DIR/case_000, DIR/case_001, ...
     double tol = 1e-4;  // relative Frobenius error allowed between the kernel and the check kernel
 };
 
-// What this run passes as (workspace, workspace_bytes): one look at the matrix (dlspm_analyze, once per matrix structure)
-// and the library's answer for the op and the width (dlspm_advise) -- nothing, a hint, schedule memory, a row plan or a
+// What this run passes as (workspace, workspace_bytes): one look at the matrix (dlspm_analyze_details, once per matrix structure)
+// and the library's answer for the op and the width (dlspm_advise_details) -- nothing, a hint, schedule memory, a row plan or a
 // cut plan -- allocated and, for the plans, built on the device here, with the time that took.
 struct PreparedCall {
     DevBuf<char> memory{0};
@@ -231,13 +231,15 @@ inline PreparedCall prepare_call(const Options& opt, int op, int M, int K, int w
 {
     PreparedCall pc;
     if (opt.workspace == Options::kNever || M <= 0 || nnz <= 0) return pc;
-    dlspm_matrix_info mi;
-    if (dlspm_analyze(M, K, nnz, row_offsets_dev, col_indices_dev, nullptr, &mi) != DLSPM_OK) throw std::runtime_error("dlspm_analyze failed");
+    dlspm_matrix_details details;
+    if (dlspm_analyze_details(M, K, nnz, row_offsets_dev, col_indices_dev, nullptr, &details) != DLSPM_OK)
+        throw std::runtime_error("dlspm_analyze_details failed");
+    const dlspm_matrix_info& mi = details.shape;
     dlspm_call_plan cp{DLSPM_BUILD_NOTHING, 0, 0};
     if (opt.workspace == Options::kAlways) {
         cp.bytes = dlspm_workspace_bytes(op, M, K, width, nnz);
     } else {
-        if (dlspm_advise(op, width, &mi, &cp) != DLSPM_OK) throw std::runtime_error("dlspm_advise failed");
+        if (dlspm_advise_details(op, width, &details, &cp) != DLSPM_OK) throw std::runtime_error("dlspm_advise_details failed");
         if (!opt.plan && cp.build != DLSPM_BUILD_NOTHING) {  // --no-plan: what the advice says without plans
             const int passing = dlspm_workspace_advice(op, M, K, width, nnz, mi.max_row_len);
             cp = dlspm_call_plan{DLSPM_BUILD_NOTHING, passing == DLSPM_PASS_WORKSPACE ? dlspm_workspace_bytes(op, M, K, width, nnz) : 0,

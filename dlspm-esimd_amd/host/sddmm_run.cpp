@@ -40,7 +40,7 @@ static bool run_case(const CaseSpec& s, const Options& opt)
     DLSPM_HIP_CHECK(hipMemset(out_d.p, 0xFF, std::max(nnz, 1) * sizeof(float)));
 
     // SDDMM needs memory only for the slice boundaries of the column-sliced schedule or for a plan; otherwise the
-    // argument only carries what dlspm_advise found out about the rows and columns
+    // argument only carries what dlspm_advise_details found out about the rows and columns
     const PreparedCall pc = prepare_call(opt, DLSPM_OP_SDDMM, M, K, D, nnz, ro_d.p, ci_d.p);
     const Timing t = time_launches(opt, [&](hipStream_t stream) {
         return sddmm_csr_f32(M, K, D, nnz, ro_d.p, ci_d.p, lhs_d.p, rhs_d.p, out_d.p, pc.arg(), pc.size(), stream);

@@ -42,8 +42,8 @@ static bool run_case(const CaseSpec& s, const Options& opt)
     if (dlspm_csr_check(M, K, nnz, ro_d.p, ci_d.p, nullptr) != DLSPM_OK) throw std::invalid_argument("malformed CSR structure");
     DLSPM_HIP_CHECK(hipMemset(C_d.p, 0xFF, (size_t)M * N * sizeof(float)));  // NaN pattern: every element must be written
 
-    // the caller owns the workspace, as it owns every other buffer. Once per matrix: one look at it (dlspm_analyze) and
-    // the library's answer for this op and width (dlspm_advise) -- nothing, a hint, schedule memory, or a plan built here
+    // the caller owns the workspace, as it owns every other buffer. Once per matrix: one look at it (dlspm_analyze_details) and
+    // the library's answer for this op and width (dlspm_advise_details) -- nothing, a hint, schedule memory, or a plan built here
     const PreparedCall pc = prepare_call(opt, DLSPM_OP_SPMM, M, K, N, nnz, ro_d.p, ci_d.p);
     const Timing t = time_launches(opt, [&](hipStream_t stream) {
         return spmm_csr_f32(M, K, N, nnz, ro_d.p, ci_d.p, va_d.p, B_d.p, C_d.p, pc.arg(), pc.size(), stream);

@@ -195,15 +195,16 @@ int dlspm_csr_check(int M, int K, int nnz, const int* row_offsets, const int* co
 
 /*
  * One look at the matrix, one answer. The compute calls see sizes only; how a matrix should be launched also depends on
- * how uneven its rows are and on whether neighbouring rows gather neighbouring dense rows. These two calls hold every
+ * how uneven its rows are and on whether neighbouring rows gather neighbouring dense rows. These calls hold every
  * such rule in one place (the thresholds live in the library's code, once):
  *   dlspm_analyze   one pass over the CSR structure on the device (synchronises `stream`; once per matrix structure, like
  *                   dlspm_csr_check): the longest row, the rows without nonzeros, the widest row (largest - smallest
  *                   column + 1), and, with the rows cut into eight contiguous eighths (the share of one XCD under
  *                   DLSPM_HINT_BANDED): the columns that the eighths span, summed, in thousandths of K (1000: a band that
  *                   moves down the columns with the row; 8000: every eighth reaches all columns), and the nonzeros of
- *                   the heaviest eighth in thousandths of the mean eighth; the rows whose columns do not ascend strictly,
- *                   and the nonzeros of the heaviest 64 rows, which one workgroup of dense tiles owns.
+ *                   the heaviest eighth in thousandths of the mean eighth. dlspm_analyze_details: in the same pass also the
+ *                   rows whose columns do not ascend strictly, and the nonzeros of the heaviest 64 rows, which one
+ *                   workgroup of dense tiles owns.
  *   dlspm_advise    host only: for op (DLSPM_OP_*) at dense width N_or_D, what to allocate (`bytes` of device memory, 0:
  *                   pass NULL), what to build into it (`build`: nothing, dlspm_row_plan_build or
  *                   dlspm_row_plan_build_cut; nothing with bytes > 0: plain schedule memory, no initialisation), and
@@ -211,11 +212,12 @@ int dlspm_csr_check(int M, int K, int nnz, const int* row_offsets, const int* co
  *                   in masks of 16 to 64 rows per compute unit get DLSPM_HINT_ROWS_SKEWED with their plan, and so do,
  *                   without a plan, tall matrices of short rows whose long rows lie next to each other and matrices of
  *                   uneven rows that SpMM multiplies from slices of B in LDS: memory that a call would not look at is
- *                   not asked for. Memory for dense tiles, and for the fused op's two steps in place of row blocks, is
- *                   asked for only where the columns of fifteen rows in sixteen ascend, that for two steps where no 64
- *                   rows hold much more than their share either.
- * Use:  dlspm_matrix_info mi; dlspm_call_plan cp;
- *       dlspm_analyze(M, K, nnz, row_offsets, col_indices, stream, &mi);   dlspm_advise(DLSPM_OP_SPMM, N, &mi, &cp);
+ *                   not asked for. dlspm_advise_details asks for memory for dense tiles, and for the fused op's two steps in
+ *                   place of row blocks, only where the columns of fifteen rows in sixteen ascend, and for two steps only
+ *                   where no 64 rows hold much more than their share either; dlspm_advise takes the one for granted and
+ *                   judges the other by the eighths.
+ * Use:  dlspm_matrix_details md; dlspm_call_plan cp;
+ *       dlspm_analyze_details(M, K, nnz, row_offsets, col_indices, stream, &md);   dlspm_advise_details(DLSPM_OP_SPMM, N, &md, &cp);
  *       void* ws = NULL; if (cp.bytes) hipMalloc(&ws, cp.bytes);
  *       if (cp.build == DLSPM_BUILD_ROW_PLAN) dlspm_row_plan_build(M, row_offsets, ws, cp.bytes, stream);
  *       if (cp.build == DLSPM_BUILD_CUT_PLAN) dlspm_row_plan_build_cut(M, row_offsets, ws, cp.bytes, stream);
@@ -234,9 +236,12 @@ typedef struct dlspm_matrix_info {
     int max_col_span;            /* widest row: largest - smallest column index + 1                           */
     int eighths_cover_permille;  /* sum over the eight eighths of the rows of the columns each spans, x 1000 / K */
     int eighths_nnz_permille;    /* nonzeros of the heaviest eighth x 1000 / those of the mean eighth         */
+} dlspm_matrix_info;
+typedef struct dlspm_matrix_details {
+    dlspm_matrix_info shape;
     int unordered_rows;          /* rows whose column indices do not ascend strictly                          */
     int heaviest_64_rows;        /* nonzeros of the heaviest 64 rows (row 64 i ... 64 i + 63); 0: not known   */
-} dlspm_matrix_info;
+} dlspm_matrix_details;
 #define DLSPM_BUILD_NOTHING   0
 #define DLSPM_BUILD_ROW_PLAN  1
 #define DLSPM_BUILD_CUT_PLAN  2
@@ -248,6 +253,9 @@ typedef struct dlspm_call_plan {
 int dlspm_analyze(int M, int K, int nnz, const int* row_offsets, const int* col_indices, void* stream,
                   dlspm_matrix_info* info);
 int dlspm_advise(int op, int N_or_D, const dlspm_matrix_info* info, dlspm_call_plan* plan);
+int dlspm_analyze_details(int M, int K, int nnz, const int* row_offsets, const int* col_indices, void* stream,
+                          dlspm_matrix_details* details);
+int dlspm_advise_details(int op, int N_or_D, const dlspm_matrix_details* details, dlspm_call_plan* plan);
 
 /*
  * Longest row and number of rows without nonzeros of a CSR structure that lives on the device (either result

@@ -36,8 +36,10 @@ int main()
         dlspm_matrix_info mi = {M, K, nnz, longest, (int)(nnz % 7), K / 3 + 1, (int)((unsigned)nnz % 8001u), (int)((unsigned)M % 8001u)};
         dlspm_call_plan cp;
         volatile int ad = dlspm_advise(op, W, &mi, &cp);
+        const dlspm_matrix_details md = {mi, (int)((unsigned)K % 9973u), longest / 2};
+        (void)dlspm_advise_details(op, W, &md, &cp);
         (void)b; (void)a; (void)p; (void)pb; (void)cb; (void)ad;
-        if (!no_device) { calls += 31; return; }
+        if (!no_device) { calls += 32; return; }
         // the compute entry points without a device and with pointers that must not be touched: a status, nothing else
         float* bad = reinterpret_cast<float*>(16);
         int* badi = reinterpret_cast<int*>(16);
@@ -50,8 +52,10 @@ int main()
         volatile int e7 = sddmm_csr_f32(M, K, W, nnz, badi, badi, bad, bad, bad, bad, (size_t)longest | DLSPM_HINT_CUT_PLAN, nullptr);
         dlspm_matrix_info got;
         volatile int e8 = dlspm_analyze(M, K, nnz, badi, badi, nullptr, &got);
+        dlspm_matrix_details seen;
+        (void)dlspm_analyze_details(M, K, nnz, badi, badi, nullptr, &seen);
         (void)e1; (void)e2; (void)e3; (void)e4; (void)e5; (void)e6; (void)e7; (void)e8;
-        calls += 39;
+        calls += 41;
     };
     for (int op = 0; op < 4; ++op)
         for (int i = 0; i < ne; ++i)

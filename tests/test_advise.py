@@ -283,6 +283,27 @@ def test_no_memory_is_asked_for_that_the_call_does_not_look_at(dl):
     assert min(seen.values()) > 20, seen
 
 
+def test_the_two_figures_of_dense_tiles_are_in_a_record_of_their_own(dl):
+    """dlspm_analyze fills the eight ints of a dlspm_matrix_info and nothing behind them, which belongs to a caller that was
+    compiled before there were two more figures; dlspm_advise reads as many."""
+    L, eight = dl.lib(), 8 * ctypes.sizeof(ctypes.c_int)
+    assert ctypes.sizeof(dl.MatrixInfo) == eight + 2 * ctypes.sizeof(ctypes.c_int)
+    mi = dl.MatrixInfo(*[-7] * 10)
+    assert L.dlspm_analyze(0, 4, 0, None, None, None, ctypes.byref(mi)) == dl.OK
+    assert (mi.M, mi.K, mi.nnz, mi.unordered_rows, mi.heaviest_64_rows) == (0, 4, 0, -7, -7)
+    assert L.dlspm_analyze_details(0, 4, 0, None, None, None, ctypes.byref(mi)) == dl.OK and (mi.unordered_rows, mi.heaviest_64_rows) == (0, 0)
+    assert L.dlspm_analyze_details(4, 4, 2, None, None, None, ctypes.byref(mi)) == dl.E_INVALID_ARG
+    assert L.dlspm_analyze_details(4, 4, 0, None, None, None, None) == dl.E_INVALID_ARG
+    M, K, nnz = 12288, 2048, int(12288 * 2048 * 0.3)
+    shuffled, bytes_of = dl.MatrixInfo(M, K, nnz, 700, 0, K, 8000, 1000, M, 0), {}
+    for name in ("dlspm_advise", "dlspm_advise_details"):
+        cp = dl.CallPlan()
+        assert getattr(L, name)(dl.OP_FUSED, 128, ctypes.byref(shuffled), ctypes.byref(cp)) == dl.OK
+        bytes_of[name] = cp.bytes
+        assert getattr(L, name)(dl.OP_FUSED, 128, None, ctypes.byref(cp)) == dl.E_INVALID_ARG
+    assert bytes_of["dlspm_advise"] >= 4 * nnz > bytes_of["dlspm_advise_details"]
+
+
 @pytest.mark.gpu
 def test_analyze_counts_rows_out_of_order_and_the_heaviest_64(dl):
     import torch
@@ -303,8 +324,12 @@ def test_analyze_counts_rows_out_of_order_and_the_heaviest_64(dl):
                 ci[a + 64] = ci[a + 3]
         for r in range(M):
             want += int((np.diff(ci[ro[r]:ro[r + 1]]) <= 0).any())
-        got = dl.analyze(dev(torch, ro), dev(torch, ci), K)
+        d_ro, d_ci = dev(torch, ro), dev(torch, ci)
+        got = dl.analyze(d_ro, d_ci, K)
         assert (got.unordered_rows, got.heaviest_64_rows) == (want, heaviest), (kind, M, K)
+        plain = dl.MatrixInfo(*[-7] * 10)
+        assert dl.lib().dlspm_analyze(M, K, len(ci), d_ro.data_ptr(), d_ci.data_ptr(), None, ctypes.byref(plain)) == dl.OK
+        assert plain.as_dict() == got.as_dict() and (plain.unordered_rows, plain.heaviest_64_rows) == (-7, -7)
 
 
 def test_tiles_are_for_rows_that_ascend_and_share_the_work(dl):
