@@ -148,9 +148,8 @@ __device__ __forceinline__ void resident_part_chunk(const char* tiles, const int
 
 // What is left of a wave's four rows, sixteen lanes each, whose columns do not ascend: from memory, in CSR order, in 64 bits. Sixteen
 // pairs of a row at a time and eight of their rows of B on their way together (16384 x 8192 at density 0.3, N = 128, all rows shuffled: 2962
-// -> 1149 us; one nonzero after the other before). Behind a branch that is not expected to be taken, out of the way of the kernel's end, and
-// in a kernel that is told of its four waves per SIMD, so that the compiler does not order the loop over the slices for five: 1.00 of
-// the time without any such rows (always walked through, 1.01; behind the branch alone, 1.03 ... 1.04).
+// -> 1149 us; one nonzero after the other before). With selects: what is behind a branch here makes the compiler order the loop over the
+// slices anew.
 template <int... L>
 __device__ __forceinline__ void gather_rest(int p, int end, int l, int N, const int* __restrict__ col_indices, const float* __restrict__ values,
                                             const float* __restrict__ B, RowSum& sum, std::integer_sequence<int, L...>)
@@ -184,7 +183,7 @@ __device__ __forceinline__ void gather_rest(int p, int end, int l, int N, const 
 // QC: chunks of 64 pairs of a row that are loaded ahead (a slice's share of a row is to fit them: what exceeds it is loaded
 // when it is needed, with nothing to hide the latency behind). CHAINS: see ChunkSum.
 template <int RR, int QC, int CHAINS>
-__global__ __launch_bounds__(kResidentThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) void spmm_resident_kernel(
+__global__ __launch_bounds__(kResidentThreads) void spmm_resident_kernel(
     int M, int K, int N, int nnz, int slice, int col_tiles, int tiles_per_xcd, int streaming, const int* __restrict__ row_offsets,
     const int* __restrict__ col_indices, const float* __restrict__ values, const float* __restrict__ B, float* __restrict__ C)
 {
@@ -378,7 +377,10 @@ __global__ __launch_bounds__(kResidentThreads) __attribute__((amdgpu_waves_per_e
 #pragma unroll
     for (int rr = 0; rr < RR; ++rr) {
         RowSum& sum = total[rr];
-        if (__builtin_expect(__ballot(p[rr] < end[rr]) != 0, 0))
+        // (Where nothing is left. A branch that is not expected to be taken keeps the gathering out of the way of the kernel's end, which
+        // the short calls notice (2048 x 2048 at 0.1, N = 392 12.5 -> 12.3 us); at two chunks ahead it also makes the compiler order the loop
+        // above for fewer registers, 2 ... 7 % slower (27241 x 5786 at 0.2, N = 128, lognormal rows 417 -> 443), and there it stays away.)
+        if (QC == 2 || __builtin_expect(__ballot(p[rr] < end[rr]) != 0, 0))
             gather_rest(p[rr], end[rr], l_end, N, col_indices, values, B + col_end, sum, std::make_integer_sequence<int, 8>{});
         if (row[rr] >= M) continue;
         const Vec<4> out{make_float4((float)sum.x, (float)sum.y, (float)sum.z, (float)sum.w)};
