@@ -10,10 +10,11 @@
 //     a prefix of them, and their results go to their slots. A row's position is carried from tile to tile; where a range does not
 //     begin with the row it is found by a binary search. Any position is a correct one: what a row has left at the end of a range,
 //     because its columns do not ascend, is computed as in sddmm.hip, and so are results that are not finite (dense_tiles.hpp).
-//   * Rows whose first 64 columns do not ascend, and rows of lhs with a nonzero value below 2^-109, are left out of the tiles. A workgroup that finds more than half of its rows to be
-//     such gathers all of them instead, otherwise its waves share them behind the tiles (us, gathering kernels / all rows shuffled /
-//     every sixteenth, at 8192 x 8192: D = 128 at 0.2 250 / 274 / 126, D = 64 at 0.2 125 / 137 / 78, D = 32 at 0.3 110 / 119 / 61; while the wave
-//     of such a row finished it alone: 1565 / 307, 654 / 158, 481 / 131; 2048 x 2048 at 0.3, D = 128, 24 / 31 / 16, was 187 / 62).
+//   * Rows whose first 64 columns do not ascend, and rows of lhs with a nonzero value below 2^-109, are left out of the tiles. A
+//     workgroup that finds more than half of its rows to be such gathers all of them instead, otherwise its waves share them behind the
+//     tiles (us, gathering kernels / all rows shuffled / every sixteenth, at 8192 x 8192: D = 128 at 0.2 250 / 274 / 126, D = 64 at 0.2
+//     125 / 137 / 78, D = 32 at 0.3 110 / 119 / 61; while the wave of such a row finished it alone: 1565 / 307, 654 / 158, 481 / 131;
+//     2048 x 2048 at 0.3, D = 128, 24 / 31 / 16, was 187 / 62).
 //   * Such a value in a row of rhs is noted for the end, where results of its column that are small enough to show what its parts lost,
 //     and results that are not finite, are gathered: a value of 1e-36 in every row of rhs takes the three from 104 / 66 / 56 to 133 / 92 /
 //     80 us (1175 / 605 / 388 while its parts were NaN and every result of the column was computed again).
@@ -26,6 +27,7 @@
 // 3.8 / 4.3 / 4.8 / 5.2e-8 at D = 32 / 64 / 96 / 128, the gathering kernels' by 6.2 / 7.2 / 8.0 / 8.8e-8; operands of one sign 3.4 / 3.8 / 3.9 /
 // 4.4e-8 and 4.1 / 4.2 / 4.3 / 4.5e-8. For the latter hi x hi has two chains of every second step above D = 32, and the last step's goes
 // behind the small products: in one chain of all steps the sums grow as they go, and so do their roundings (3.4 / 5.2 / 5.7 / 6.9e-8).
+// That is 1 % of the time in the mean of 17 sizes, up to 4 % at D = 65 ... 95.
 // What bounds it: D = 128, the products (a wave spends 6 of the 7 us of a tile in them; 3 at the rate of products of constants, 4.5 at
 // what a large bf16 product of random numbers reaches here, 1.2 ... 1.35 PFLOP/s of 2.5: the chip lowers its clocks); D = 32, the
 // turns of computing (1.5 ... 2.5 us of 4 ... 5), waiting at the barrier and sampling, which two workgroups overlap only in part.
