@@ -80,6 +80,12 @@ def schedules(dl, torch, op, M, K, N, nnz, ro_d, ci_d, every):
             out.append(("row_plan", None, dl.row_plan(ro_d)))
             if dl.row_plan_bytes_for(op, M, N) > 0:
                 out.append(("cut_plan", None, dl.cut_plan(ro_d, op, N)))
+        # memory for dense tiles and for two steps, as for even and for uneven rows, whatever the rows are
+        for longest in (-(-nnz // max(M, 1)), K):
+            cp = dl.advise(op, N, dl.MatrixInfo(M, K, nnz, longest, 0, K, 8000, 1000))
+            run = dl.describe_schedule(op, M, K, N, nnz, workspace_bytes=cp.bytes | cp.hints)["schedule"] if cp.bytes else None
+            if run in ("dense_tiles", "two_steps"):
+                out.append((run + ("_even" if cp.hints & dl.HINT_ROWS_EVEN else ""), None, dl.Prepared(None, cp.bytes | cp.hints, cp)))
         return out
     if M == 0:
         return [("null", None, None)]

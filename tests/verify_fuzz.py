@@ -7,7 +7,7 @@ switched off, the cut rule's percentages, the number of compute units the rules 
     python tests/verify_fuzz.py [--cases 1000] [--seed 1] [--report out.txt]
 
 Each case runs all three ops on the GPU through the C ABI under every schedule that applies (NULL, the even-rows hint,
-workspace memory, a row plan, a cut plan) and compares with the oracle: CSR arrays bit-identical after the call, values within 1e-4
+workspace memory, a row plan, a cut plan, memory for dense tiles and two steps) and compares with the oracle: CSR arrays bit-identical after the call, values within 1e-4
 relative Frobenius error. No tuning value may change a result beyond the summation order, and none may make a launch
 fail. The case is printed before it runs. Exit status 1 if any case fails.
 """
@@ -25,10 +25,19 @@ from verify_dlmc import Tally, check_pattern  # noqa: E402  (also puts the bindi
 SPLITS = [None, (4, 1), (4, 2), (4, 4), (4, 8), (4, 16), (8, 1), (8, 2), (8, 4), (16, 1)]
 
 
-def random_tuning(rng):
-    """Keyword arguments for dl.set_tuning: each knob left to the library's rule with probability 1/2."""
+def random_tuning(rng, by_size):
+    """Keyword arguments for dl.set_tuning: each knob left to the library's rule with probability 1/2. by_size: none that names a
+    schedule, which keeps a call from those that sizes choose (slices of B in LDS, dense tiles, two steps)."""
     t = {}
     pick = lambda values: values[int(rng.integers(0, len(values)))]
+    if by_size:
+        if rng.random() < 0.5:
+            t["stream_results"] = pick([0, 1])
+        if rng.random() < 0.3:
+            t["rules_off"] = 1 << int(rng.integers(0, 16))
+        if rng.random() < 0.2:
+            t["compute_units"] = pick([32, 64, 128, 304])
+        return t
     if rng.random() < 0.5:
         s = pick(SPLITS)
         if s is not None:
@@ -95,7 +104,8 @@ def main():
             kind = "uniform"
         while kind != "full" and M * K * density > 600000:
             density /= 4
-        # one case in ten is large and dense enough for slices of B in LDS, one a sliding window that goes to the matrix cores
+        # one case in ten is large and dense enough for slices of B in LDS and for dense tiles, one a sliding window that goes to the
+        # matrix cores
         large = rng.random()
         if large < 0.1:
             M, K, kind, density = int(rng.integers(1500, 6000)), int(rng.integers(200, 1500)), "uniform", float(rng.choice([0.15, 0.3, 0.6]))
@@ -106,7 +116,7 @@ def main():
             ro, ci = sliding_window(rng, M, int(rng.integers(40, 310)))
         else:
             ro, ci = random_csr(rng, M, K, kind, 1.0 if kind == "full" else density)
-        tuning = random_tuning(rng)
+        tuning = random_tuning(rng, large < 0.2 and rng.random() < 0.8)
         what = f"case {case}: M={M} K={K} N={N} {kind} density={density:g} nnz={ci.size} tuning={tuning}"
         print(what, flush=True)
         dl.set_tuning(**tuning)
